@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define PIC_ABI_VERSION 12
+#define PIC_ABI_VERSION 13
 #define PIC_MAX_SPECIES 16
 
 /* Scalar run description: StaticParameters + DynamicParameters fields the hot
@@ -91,11 +91,23 @@ int pic_constant_boundary(const PicDesc* desc, float* field, int axis, void* str
  * VALID correlation of in; out ghosts <- in ghosts.  in != out. */
 int pic_filter_digital(const PicDesc* desc, const float* in, float* out, double alpha, void* stream);
 int pic_filter_bilinear(const PicDesc* desc, const float* in, float* out, void* stream);
+/* Up to three components at once (NULL: skipped), each call one launch:
+ * zeros in every cell; fold_tiled_vector_ghost_cells followed by
+ * update_tiled_vector_ghost_cells with the same codes, in place
+ * (Esirkepov.py:357-359, J_from_rhov.py:224-232); the bilinear (1) or digital
+ * (0) filter of in into out with out's guard cells refreshed and, if walls is
+ * nonzero, tangential E zero on the conducting walls (first_order_yee.py:76-92);
+ * those walls alone, in place.  Guard cells of in must be refreshed. */
+int pic_zero_fields(const PicDesc* desc, float* const f[3], void* stream);
+int pic_finish_current(const PicDesc* desc, float* const f[3], int bc_type, void* stream);
+int pic_filter_refresh(const PicDesc* desc, const float* const in[3], float* const out[3], int bilinear,
+                       double alpha, int bc_type, int walls, void* stream);
+int pic_conducting_walls(const PicDesc* desc, float* const E[3], void* stream);
 
 /* ---- Yee solver (solvers/first_order_yee.py) --------------------------- */
 /* B_out interior = B_in - (dt/2) curl E with E neighbours read as refreshed
  * ghosts (first_order_yee.py:96-142); then B_out ghosts refreshed.  The
- * do_filter branch (:145-159) is pic_filter_digital + pic_halo_refresh. */
+ * do_filter branch (:145-159) is pic_filter_refresh. */
 int pic_yee_update_b(const PicDesc* desc, const float* const E[3], const float* const B_in[3],
                      float* const B_out[3], void* stream);
 /* E_out interior = E_in + dt (C^2 curl B - J/eps) (first_order_yee.py:12-74);
@@ -352,6 +364,11 @@ int pic_zero_boundary_f64(const PicDesc* desc, double* field, int axis, void* st
 int pic_constant_boundary_f64(const PicDesc* desc, double* field, int axis, void* stream);
 int pic_filter_digital_f64(const PicDesc* desc, const double* in, double* out, double alpha, void* stream);
 int pic_filter_bilinear_f64(const PicDesc* desc, const double* in, double* out, void* stream);
+int pic_zero_fields_f64(const PicDesc* desc, double* const f[3], void* stream);
+int pic_finish_current_f64(const PicDesc* desc, double* const f[3], int bc_type, void* stream);
+int pic_filter_refresh_f64(const PicDesc* desc, const double* const in[3], double* const out[3], int bilinear,
+                           double alpha, int bc_type, int walls, void* stream);
+int pic_conducting_walls_f64(const PicDesc* desc, double* const E[3], void* stream);
 int pic_yee_update_b_f64(const PicDesc* desc, const double* const E[3], const double* const B_in[3],
                          double* const B_out[3], void* stream);
 int pic_yee_update_e_f64(const PicDesc* desc, const double* const E_in[3], const double* const B[3],

@@ -17,7 +17,7 @@ LIB_PATH = os.path.join(HERE, "libpypic3d_hip.so")
 MAX_SPECIES = 16
 PUSHERS = {"boris": 0, "higuera_cary": 1}
 FUSED_VARIANTS = 6
-ABI_VERSION = 12
+ABI_VERSION = 13
 
 c_int = ctypes.c_int
 c_i32 = ctypes.c_int32
@@ -69,6 +69,14 @@ SIGNATURES = {
     "pic_constant_boundary": (c_int, [DP, c_vp, c_int, c_vp]),
     "pic_filter_digital": (c_int, [DP, c_vp, c_vp, c_dbl, c_vp]),
     "pic_filter_bilinear": (c_int, [DP, c_vp, c_vp, c_vp]),
+    "pic_zero_fields": (c_int, [DP, P3, c_vp]),
+    "pic_finish_current": (c_int, [DP, P3, c_int, c_vp]),
+    "pic_filter_refresh": (c_int, [DP, P3, P3, c_int, c_dbl, c_int, c_int, c_vp]),
+    "pic_conducting_walls": (c_int, [DP, P3, c_vp]),
+    "pic_zero_fields_f64": (c_int, [DP, P3, c_vp]),
+    "pic_finish_current_f64": (c_int, [DP, P3, c_int, c_vp]),
+    "pic_filter_refresh_f64": (c_int, [DP, P3, P3, c_int, c_dbl, c_int, c_int, c_vp]),
+    "pic_conducting_walls_f64": (c_int, [DP, P3, c_vp]),
     "pic_yee_update_b": (c_int, [DP, P3, P3, P3, c_vp]),
     "pic_yee_update_e": (c_int, [DP, P3, P3, P3, P3, c_vp]),
     "pic_push": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, P3, c_vp]),
@@ -202,3 +210,8 @@ def ptr(t):
 
 def p3(ts):
     return P3(*[t.data_ptr() for t in ts])
+
+
+def p1(t):
+    """A single component for the entry points that take up to three."""
+    return P3(t.data_ptr(), None, None)

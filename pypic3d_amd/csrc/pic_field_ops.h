@@ -19,12 +19,7 @@ __host__ __device__ inline void other_dims(const PicDesc& d, int axis, int& da, 
     db = d.dims[axis == 2 ? 1 : 2];
 }
 
-// Number of element ids of each operation on one axis.
-__host__ __device__ inline int64_t refresh_elems(const PicDesc& d, int axis) {
-    int da, db;
-    other_dims(d, axis, da, db);
-    return (int64_t)2 * d.g * da * db;
-}
+// Number of element ids of the fold on one axis.
 __host__ __device__ inline int64_t fold_elems(const PicDesc& d, int axis) {
     int da, db;
     other_dims(d, axis, da, db);
@@ -33,27 +28,6 @@ __host__ __device__ inline int64_t fold_elems(const PicDesc& d, int axis) {
 
 __device__ inline void atomic_add_t(float* p, float v) { unsafeAtomicAdd(p, v); }
 __device__ inline void atomic_add_t(double* p, double v) { unsafeAtomicAdd(p, v); }
-
-// ghost_cells.py:142-196: ghost element t (< refresh_elems) of one axis.
-template <class T>
-__device__ inline void refresh_elem(const PicDesc& d, T* f, int axis, int mode, int64_t t) {
-    int g = d.g, n = d.n[axis];
-    int da, db;
-    other_dims(d, axis, da, db);
-    int b = (int)(t % db);
-    int64_t r = t / db;
-    int a = (int)(r % da);
-    int l = (int)(r / da);
-    int dst = l < g ? l : n + l;          // upper ghosts n+g .. n+2g-1
-    T v = (T)0;
-    if (mode == MODE_REDUCED_COPY) {
-        v = f[slab_to_index(d, axis, g, a, b)];
-    } else if (mode == MODE_PERIODIC) {
-        int src = l < g ? n + l : l;      // lower l <- n+l ; upper (l-g) <- g+(l-g)
-        v = f[slab_to_index(d, axis, src, a, b)];
-    }
-    f[slab_to_index(d, axis, dst, a, b)] = v;
-}
 
 // ghost_cells.py:218-289: fold element t (< fold_elems) of a non-reduced axis.
 // bc: 0 periodic self-exchange, 1 conducting reflection, other: dropped.
@@ -104,6 +78,182 @@ __device__ inline void fold_reduced_elem(const PicDesc& d, T* f, int axis, int b
     else if (bc == 1) f[c] += -s;
 }
 
+// ---- images: the ghost cells that belong to an interior cell --------------
+// On every axis each ghost index belongs to exactly one interior index: its
+// periodic partner, the cell at the same depth inside a non-periodic wall, or
+// index g of a reduced axis.  The product over the axes assigns every ghost
+// cell of the array to one interior cell.  A refreshed field holds the interior
+// value at all images across periodic axes and 0 where a non-periodic axis is
+// crossed (the x -> y -> z sequence of ghost_cells.py:142-215 composed), and
+// the fold adds the images into the interior cell (:218-289), so the thread of
+// an interior cell can do both in place without a second launch.
+
+__device__ inline int image_count(const PicDesc& d, int axis) { return d.n[axis] == 1 ? 2 * d.g : 2; }
+
+// Image q of interior index i along an axis; -1 if there is none.
+__device__ inline int image_index(const PicDesc& d, int axis, int mode, int i, int q) {
+    const int g = d.g, n = d.n[axis];
+    if (n == 1) return q < g ? q : q + 1;
+    if (q == 0) return i < 2 * g ? (mode == MODE_PERIODIC ? i + n : i - g) : -1;
+    return i >= n ? (mode == MODE_PERIODIC ? i - n : i + g) : -1;
+}
+
+// Whether interior index i has images on an axis.
+__device__ inline bool has_images(const PicDesc& d, int axis, int i) {
+    return d.n[axis] == 1 || i < 2 * d.g || i >= d.n[axis];
+}
+
+// The image of an interior index on an axis of at least two guard bands, which
+// has at most one; -1 if it has none.
+__device__ inline int single_image(const PicDesc& d, int axis, int mode, int i) {
+    const int g = d.g, n = d.n[axis];
+    if (i < 2 * g) return mode == MODE_PERIODIC ? i + n : i - g;
+    if (i >= n) return mode == MODE_PERIODIC ? i - n : i + g;
+    return -1;
+}
+
+// Every axis with at most one image per cell (uniform over a launch).
+__device__ inline bool single_images(const PicDesc& d) {
+    return d.n[0] >= 2 * d.g && d.n[1] >= 2 * d.g && d.n[2] >= 2 * d.g;
+}
+
+// Stores v[] at interior cell (i, j, k) of kC components and at all its images
+// (v across periodic axes, 0 across others): the refresh that would follow.
+template <int kC, class T>
+__device__ inline void store_refreshed(const PicDesc& d, const int mode[3], T* const out[kC], int i, int j, int k,
+                                       const T v[kC]) {
+    const auto put = [&](int ii, int jj, int kk, bool zero) {
+        const int64_t t = fidx(d, ii, jj, kk);
+#pragma unroll
+        for (int m = 0; m < kC; ++m) out[m][t] = zero ? (T)0 : v[m];
+    };
+    put(i, j, k, false);
+    if (single_images(d)) {
+        const int ii = single_image(d, 0, mode[0], i), jj = single_image(d, 1, mode[1], j);
+        const int kk = single_image(d, 2, mode[2], k);
+        const bool zi = mode[0] == MODE_ZERO, zj = mode[1] == MODE_ZERO, zk = mode[2] == MODE_ZERO;
+        if (kk >= 0) put(i, j, kk, zk);
+        if (jj >= 0) {
+            put(i, jj, k, zj);
+            if (kk >= 0) put(i, jj, kk, zj || zk);
+        }
+        if (ii >= 0) {
+            put(ii, j, k, zi);
+            if (kk >= 0) put(ii, j, kk, zi || zk);
+            if (jj >= 0) {
+                put(ii, jj, k, zi || zj);
+                if (kk >= 0) put(ii, jj, kk, zi || zj || zk);
+            }
+        }
+        return;
+    }
+    if (!(has_images(d, 0, i) || has_images(d, 1, j) || has_images(d, 2, k))) return;
+    const int n0 = image_count(d, 0), n1 = image_count(d, 1), n2 = image_count(d, 2);
+    for (int a = -1; a < n0; ++a) {
+        const int ii = a < 0 ? i : image_index(d, 0, mode[0], i, a);
+        if (ii < 0) continue;
+        for (int b = -1; b < n1; ++b) {
+            const int jj = b < 0 ? j : image_index(d, 1, mode[1], j, b);
+            if (jj < 0) continue;
+            for (int e = -1; e < n2; ++e) {
+                const int kk = e < 0 ? k : image_index(d, 2, mode[2], k, e);
+                if (kk < 0 || (a < 0 && b < 0 && e < 0)) continue;
+                put(ii, jj, kk, (a >= 0 && mode[0] == MODE_ZERO) || (b >= 0 && mode[1] == MODE_ZERO) ||
+                                    (e >= 0 && mode[2] == MODE_ZERO));
+            }
+        }
+    }
+}
+
+// Interior value of the fold of f at (i, j, k): the cell plus its images, each
+// axis' images with the sign of its code (0 periodic: +, 1 conducting /
+// reflecting: -, other: dropped), x summed first as the sequential fold does.
+template <class T>
+__device__ inline T folded_at(const PicDesc& d, const int mode[3], const int sign[3], const T* f, int i, int j,
+                              int k) {
+    if (single_images(d)) {
+        // the up to eight cells as independent loads
+        const int at[3][2] = {{i, sign[0] ? single_image(d, 0, mode[0], i) : -1},
+                              {j, sign[1] ? single_image(d, 1, mode[1], j) : -1},
+                              {k, sign[2] ? single_image(d, 2, mode[2], k) : -1}};
+        T v[2][2][2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+                    v[e][b][a] = (a && at[0][1] < 0) || (b && at[1][1] < 0) || (e && at[2][1] < 0)
+                                     ? (T)0
+                                     : f[fidx(d, at[0][a], at[1][b], at[2][e])];
+        T plane[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const T l0 = v[e][0][0] + (sign[0] < 0 ? -v[e][0][1] : v[e][0][1]);
+            const T l1 = v[e][1][0] + (sign[0] < 0 ? -v[e][1][1] : v[e][1][1]);
+            plane[e] = l0 + (sign[1] < 0 ? -l1 : l1);
+        }
+        return plane[0] + (sign[2] < 0 ? -plane[1] : plane[1]);
+    }
+    T total = (T)0;
+    const int n0 = sign[0] ? image_count(d, 0) : 0, n1 = sign[1] ? image_count(d, 1) : 0;
+    const int n2 = sign[2] ? image_count(d, 2) : 0;
+    for (int e = -1; e < n2; ++e) {
+        const int kk = e < 0 ? k : image_index(d, 2, mode[2], k, e);
+        if (kk < 0) continue;
+        T plane = (T)0;
+        for (int b = -1; b < n1; ++b) {
+            const int jj = b < 0 ? j : image_index(d, 1, mode[1], j, b);
+            if (jj < 0) continue;
+            T line = (T)0;
+            for (int a = -1; a < n0; ++a) {
+                const int ii = a < 0 ? i : image_index(d, 0, mode[0], i, a);
+                if (ii < 0) continue;
+                const T v = f[fidx(d, ii, jj, kk)];
+                line += a >= 0 && sign[0] < 0 ? -v : v;
+            }
+            plane += b >= 0 && sign[1] < 0 ? -line : line;
+        }
+        total += e >= 0 && sign[2] < 0 ? -plane : plane;
+    }
+    return total;
+}
+
+// Fold and refresh of f at interior cell (i, j, k), in place; nothing to do
+// (and nothing read) where the cell has no images.
+template <class T>
+__device__ inline void finish_point(const PicDesc& d, const int mode[3], const int sign[3], T* f, int i, int j, int k) {
+    if (!(has_images(d, 0, i) || has_images(d, 1, j) || has_images(d, 2, k))) return;
+    const T v[1] = {folded_at(d, mode, sign, f, i, j, k)};
+    T* const out[1] = {f};
+    store_refreshed<1>(d, mode, out, i, j, k, v);
+}
+
+// Interior indices of an axis with images, and the s-th of them; the others
+// are 2g .. n-1.
+__host__ __device__ inline int shell_count(const PicDesc& d, int axis) {
+    return d.n[axis] < 2 * d.g ? d.n[axis] : 2 * d.g;
+}
+__device__ inline int shell_index(const PicDesc& d, int axis, int s) {
+    return s < d.g || d.n[axis] < 2 * d.g ? d.g + s : d.n[axis] + s - d.g;
+}
+
+// Sign of each axis' images in a fold with the particle (bc_type 1) or field codes.
+__host__ __device__ inline int fold_sign(const PicDesc& d, int axis, int bc_type) {
+    const int bc = bc_type == 0 ? d.bc[axis] : d.pbc[axis];
+    return bc == 0 ? 1 : (bc == 1 ? -1 : 0);
+}
+
+// Whether component c of E is tangential to a conducting wall at (i, j, k)
+// (first_order_yee.py:80-92: zero on the planes g and n+g-1).
+__device__ inline bool on_wall(const PicDesc& d, int c, int i, int j, int k) {
+    const int at[3] = {i, j, k};
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        if (a != c && d.bc[a] == 1 && (at[a] == d.g || at[a] == d.n[a] + d.g - 1)) return true;
+    return false;
+}
+
 // Value of a refreshed copy of f at (i,j,k) where exactly one coordinate may
 // sit one cell outside the interior along `axis`.
 template <class T>
@@ -138,7 +288,8 @@ __host__ __device__ inline YeeConstT<T> yee_const(const PicDesc& d) {
 }
 
 // first_order_yee.py:96-142 at interior array point (i, j, k):
-// B_out = B_in - (dt/2) curl E with forward differences.
+// B_out = B_in - (dt/2) curl E with forward differences, guard cells refreshed
+// (out may be B: only the point itself is read from it).
 template <class T>
 __device__ inline void yee_b_point(const PicDesc& d, const YeeConstT<T>& y, const T* const E[3], const T* const B[3],
                                    T* const out[3], int i, int j, int k) {
@@ -153,13 +304,13 @@ __device__ inline void yee_b_point(const PicDesc& d, const YeeConstT<T>& y, cons
     T curl_x = (ez_yp - ez) * y.id[1] - (ey_zp - ey) * y.id[2];
     T curl_y = (ex_zp - ex) * y.id[2] - (ez_xp - ez) * y.id[0];
     T curl_z = (ey_xp - ey) * y.id[0] - (ex_yp - ex) * y.id[1];
-    out[0][c] = B[0][c] - y.hdt * curl_x;
-    out[1][c] = B[1][c] - y.hdt * curl_y;
-    out[2][c] = B[2][c] - y.hdt * curl_z;
+    const T v[3] = {B[0][c] - y.hdt * curl_x, B[1][c] - y.hdt * curl_y, B[2][c] - y.hdt * curl_z};
+    store_refreshed<3>(d, y.mode, out, i, j, k, v);
 }
 
 // first_order_yee.py:12-72 at interior array point (i, j, k):
-// E_out = E_in + dt (C^2 curl B - J/eps) with backward differences.
+// E_out = E_in + dt (C^2 curl B - J/eps) with backward differences, guard
+// cells refreshed.
 template <class T>
 __device__ inline void yee_e_point(const PicDesc& d, const YeeConstT<T>& y, const T* const E[3], const T* const B[3],
                                    const T* const J[3], T* const out[3], int i, int j, int k) {
@@ -174,9 +325,10 @@ __device__ inline void yee_e_point(const PicDesc& d, const YeeConstT<T>& y, cons
     T curl_x = (bz - bz_ym) * y.id[1] - (by - by_zm) * y.id[2];
     T curl_y = (bx - bx_zm) * y.id[2] - (bz - bz_xm) * y.id[0];
     T curl_z = (by - by_xm) * y.id[0] - (bx - bx_ym) * y.id[1];
-    out[0][c] = E[0][c] + (y.c2 * curl_x - J[0][c] * y.inv_eps) * y.dt;
-    out[1][c] = E[1][c] + (y.c2 * curl_y - J[1][c] * y.inv_eps) * y.dt;
-    out[2][c] = E[2][c] + (y.c2 * curl_z - J[2][c] * y.inv_eps) * y.dt;
+    const T v[3] = {E[0][c] + (y.c2 * curl_x - J[0][c] * y.inv_eps) * y.dt,
+                    E[1][c] + (y.c2 * curl_y - J[1][c] * y.inv_eps) * y.dt,
+                    E[2][c] + (y.c2 * curl_z - J[2][c] * y.inv_eps) * y.dt};
+    store_refreshed<3>(d, y.mode, out, i, j, k, v);
 }
 
 // PML coordinate stretch of the six curl derivatives (PML.py:251-359): for a
@@ -225,9 +377,9 @@ __device__ inline void yee_b_point_pml(const PicDesc& d, const YeeConst& y, cons
                    (refreshed_at(E[1], d, y.mode, i + 1, j, k, 0) - ey) * y.id[0],
                    (refreshed_at(E[0], d, y.mode, i, j + 1, k, 1) - ex) * y.id[1]};
     pml_stretch6(d, pml, i, j, k, dv);
-    out[0][c] = B[0][c] - y.hdt * (dv[0] - dv[1]);
-    out[1][c] = B[1][c] - y.hdt * (dv[2] - dv[3]);
-    out[2][c] = B[2][c] - y.hdt * (dv[4] - dv[5]);
+    const float v[3] = {B[0][c] - y.hdt * (dv[0] - dv[1]), B[1][c] - y.hdt * (dv[2] - dv[3]),
+                        B[2][c] - y.hdt * (dv[4] - dv[5])};
+    store_refreshed<3>(d, y.mode, out, i, j, k, v);
 }
 
 // yee_e_point with the PML stretch of the B derivatives (first_order_yee.py:49-72).
@@ -243,9 +395,10 @@ __device__ inline void yee_e_point_pml(const PicDesc& d, const YeeConst& y, cons
                    (by - refreshed_at(B[1], d, y.mode, i - 1, j, k, 0)) * y.id[0],
                    (bx - refreshed_at(B[0], d, y.mode, i, j - 1, k, 1)) * y.id[1]};
     pml_stretch6(d, pml, i, j, k, dv);
-    out[0][c] = E[0][c] + (y.c2 * (dv[0] - dv[1]) - J[0][c] * y.inv_eps) * y.dt;
-    out[1][c] = E[1][c] + (y.c2 * (dv[2] - dv[3]) - J[1][c] * y.inv_eps) * y.dt;
-    out[2][c] = E[2][c] + (y.c2 * (dv[4] - dv[5]) - J[2][c] * y.inv_eps) * y.dt;
+    const float v[3] = {E[0][c] + (y.c2 * (dv[0] - dv[1]) - J[0][c] * y.inv_eps) * y.dt,
+                        E[1][c] + (y.c2 * (dv[2] - dv[3]) - J[1][c] * y.inv_eps) * y.dt,
+                        E[2][c] + (y.c2 * (dv[4] - dv[5]) - J[2][c] * y.inv_eps) * y.dt};
+    store_refreshed<3>(d, y.mode, out, i, j, k, v);
 }
 
 }  // namespace pic

@@ -17,17 +17,13 @@ def deposit_esirkepov_into(desc, sp, pp, J3, stream, fill=True):
     """Zero (optionally), deposit, fold and refresh into the 3-D tensors J3."""
     f64 = is_f64(J3[0])
     if fill:
-        for c in J3:
-            N.fill(c, 0.0, stream)
+        N.call(N.op("pic_zero_fields", f64), desc, N.p3(J3), stream)
     N.call(N.op("pic_deposit_esirkepov", f64), desc, sp, pp, N.p3(J3), stream)
     finish_current(desc, J3, stream)
 
 
 def finish_current(desc, J3, stream):
-    f64 = is_f64(J3[0])
-    for c in J3:
-        N.call(N.op("pic_halo_fold", f64), desc, N.ptr(c), 1, stream)
-        N.call(N.op("pic_halo_refresh", f64), desc, N.ptr(c), 1, stream)
+    N.call(N.op("pic_finish_current", is_f64(J3[0])), desc, N.p3(J3), 1, stream)
 
 
 def Esirkepov_current(particles, species_config, J, static_parameters, dynamic_parameters):

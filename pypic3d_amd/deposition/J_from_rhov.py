@@ -16,8 +16,7 @@ def deposit_direct_into(desc, sp, pp, J3, current_filter, stream, scratch=None, 
     """tile/starts: tile-ordered deposit for particles sorted by pic_tile_keys
     (FP32 only); float64 J runs the FP64 path."""
     f64 = is_f64(J3[0])
-    for c in J3:
-        N.fill(c, 0.0, stream)
+    N.call(N.op("pic_zero_fields", f64), desc, N.p3(J3), stream)
     if tile and not f64:
         N.call("pic_deposit_direct_tiled", desc, sp, pp, N.p3(J3), int(tile), N.ptr(starts), stream)
     else:
@@ -27,20 +26,16 @@ def deposit_direct_into(desc, sp, pp, J3, current_filter, stream, scratch=None, 
 
 def finish_direct_current(desc, J3, current_filter, stream, scratch=None):
     """Fold + refresh of the raw direct deposit, then the optional filter
-    (J_from_rhov.py:224-258)."""
+    (J_from_rhov.py:224-258).  The filter writes the other set of arrays, which
+    J3 then holds (scratch, if given, holds the raw deposit's)."""
     f64 = is_f64(J3[0])
-    for c in J3:
-        N.call(N.op("pic_halo_fold", f64), desc, N.ptr(c), 1, stream)
-        N.call(N.op("pic_halo_refresh", f64), desc, N.ptr(c), 1, stream)
+    N.call(N.op("pic_finish_current", f64), desc, N.p3(J3), 1, stream)
     if current_filter in ("bilinear", "digital"):
-        tmp = scratch if scratch is not None else [c.clone() for c in J3]
-        for c, t in zip(J3, tmp):
-            if current_filter == "bilinear":
-                N.call(N.op("pic_filter_bilinear", f64), desc, N.ptr(c), N.ptr(t), stream)
-            else:
-                N.call(N.op("pic_filter_digital", f64), desc, N.ptr(c), N.ptr(t), float(desc.alpha), stream)
-            N.call(N.op("pic_halo_refresh", f64), desc, N.ptr(t), 1, stream)
-            c.copy_(t)
+        tmp = scratch if scratch is not None else [c.new_empty(c.shape) for c in J3]
+        N.call(N.op("pic_filter_refresh", f64), desc, N.p3(J3), N.p3(tmp), int(current_filter == "bilinear"),
+               float(desc.alpha), 1, 0, stream)
+        for c in range(3):
+            J3[c], tmp[c] = tmp[c], J3[c]
 
 
 def J_from_rhov(particles, species_config, J, static_parameters, dynamic_parameters):

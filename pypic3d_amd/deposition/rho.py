@@ -14,18 +14,18 @@ def deposit_rho_into(desc, sp, pp, rho3, current_filter, stream, scratch=None, t
     """tile/starts: tile-ordered deposit for particles sorted by pic_tile_keys
     (FP32 only); float64 rho runs the FP64 path."""
     f64 = is_f64(rho3)
-    N.fill(rho3, 0.0, stream)
+    filtered = current_filter == "digital"
+    raw = rho3      # the filter reads the raw deposit from an array of its own
+    if filtered:
+        raw = scratch if scratch is not None else rho3.new_empty(rho3.shape)
+    N.call(N.op("pic_zero_fields", f64), desc, N.p1(raw), stream)
     if tile and not f64:
-        N.call("pic_deposit_rho_tiled", desc, sp, pp, N.ptr(rho3), int(tile), N.ptr(starts), stream)
+        N.call("pic_deposit_rho_tiled", desc, sp, pp, N.ptr(raw), int(tile), N.ptr(starts), stream)
     else:
-        N.call(N.op("pic_deposit_rho", f64), desc, sp, pp, N.ptr(rho3), stream)
-    N.call(N.op("pic_halo_fold", f64), desc, N.ptr(rho3), 1, stream)
-    N.call(N.op("pic_halo_refresh", f64), desc, N.ptr(rho3), 1, stream)
-    if current_filter == "digital":
-        tmp = scratch if scratch is not None else rho3.clone()
-        N.call(N.op("pic_filter_digital", f64), desc, N.ptr(rho3), N.ptr(tmp), float(desc.alpha), stream)
-        N.call(N.op("pic_halo_refresh", f64), desc, N.ptr(tmp), 1, stream)
-        rho3.copy_(tmp)
+        N.call(N.op("pic_deposit_rho", f64), desc, sp, pp, N.ptr(raw), stream)
+    N.call(N.op("pic_finish_current", f64), desc, N.p1(raw), 1, stream)
+    if filtered:
+        N.call(N.op("pic_filter_refresh", f64), desc, N.p1(raw), N.p1(rho3), 0, float(desc.alpha), 1, 0, stream)
 
 
 def compute_rho(particles, species_config, rho, static_parameters, dynamic_parameters):

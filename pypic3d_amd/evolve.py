@@ -86,8 +86,7 @@ def time_loop_electrodynamic(particles, species_config, fields, static_parameter
         xs, xv = new_soa(S, P, dev)
         us, uv = new_soa(S, P, dev)
         act_out = act.new_empty(act.shape)
-        for c in J3:
-            N.call("pic_fill_f32", N.ptr(c), c.numel(), 0.0, stream)
+        N.call("pic_zero_fields", desc, N.p3(J3), stream)
         out = pic_particles([xs[0], xs[1], xs[2]], [us[0], us[1], us[2]], act_out)
         N.call("pic_fused_push_esirkepov", desc, sp, pic_particles(xp, up, act), N.p3(E3), N.p3(B3), Ee, Be,
                out, N.p3(J3), stream)

@@ -148,8 +148,7 @@ class ElectrodynamicRunner:
             src, dst = self._cur, 1 - self._cur
         E, Et = self.E[self.ecur], self.E[1 - self.ecur]
         if self.esirkepov:
-            for c in self.J:
-                N.call("pic_fill_f32", N.ptr(c), c.numel(), 0.0, s)
+            N.call("pic_zero_fields", d, N.p3(self.J), s)
             ev = self._mark("particles")
             if self.tile and self._pending:
                 N.call("pic_fused_push_esirkepov_tiled_gather", d, self.sp, self._pp(src), N.ptr(self.perm), N.p3(E),
@@ -168,8 +167,7 @@ class ElectrodynamicRunner:
             ev = self._mark("current_fold")
             finish_current(d, self.J, s)
         elif self.tile and self.direct_fused:
-            for c in self.J:
-                N.call("pic_fill_f32", N.ptr(c), c.numel(), 0.0, s)
+            N.call("pic_zero_fields", d, N.p3(self.J), s)
             ev = self._mark("particles")
             if self._pending:
                 N.call("pic_fused_push_direct_tiled_gather", d, self.sp, self._pp(src), N.ptr(self.perm), N.p3(E),

@@ -104,17 +104,17 @@ def yee_b(desc, E3, B3, out3, do_filter, stream, scratch=None, pml=None):
     f64 = is_f64(E3[0])
     if f64 and pml is not None:
         raise ValueError("the PML runs in FP32 (float32 fields)")
+    filtered = do_filter and desc.alpha != 1.0
+    raw = out3      # the filter reads the update from arrays of its own
+    if filtered:
+        raw = scratch if scratch is not None else [c.new_empty(c.shape) for c in out3]
     if pml is None:
-        N.call(N.op("pic_yee_update_b", f64), desc, N.p3(E3), N.p3(B3), N.p3(out3), stream)
+        N.call(N.op("pic_yee_update_b", f64), desc, N.p3(E3), N.p3(B3), N.p3(raw), stream)
     else:
-        N.call("pic_yee_update_b_pml", desc, N.p3(E3), N.p3(B3), N.p3(out3),
+        N.call("pic_yee_update_b_pml", desc, N.p3(E3), N.p3(B3), N.p3(raw),
                ctypes.byref(pml_struct(*pml, desc=desc)), stream)
-    if do_filter and desc.alpha != 1.0:
-        tmp = scratch if scratch is not None else [c.clone() for c in out3]
-        for c, t in zip(out3, tmp):
-            N.call(N.op("pic_filter_digital", f64), desc, N.ptr(c), N.ptr(t), float(desc.alpha), stream)
-            N.call(N.op("pic_halo_refresh", f64), desc, N.ptr(t), 0, stream)
-            c.copy_(t)
+    if filtered:
+        N.call(N.op("pic_filter_refresh", f64), desc, N.p3(raw), N.p3(out3), 0, float(desc.alpha), 0, 0, stream)
     return out3
 
 
@@ -124,28 +124,21 @@ def yee_e(desc, E3, B3, J3, out3, stream, scratch=None, pml=None):
     f64 = is_f64(E3[0])
     if f64 and pml is not None:
         raise ValueError("the PML runs in FP32 (float32 fields)")
+    filtered = desc.alpha != 1.0
+    walls = any(desc.bc[axis] == 1 for axis in range(3))
+    raw = out3
+    if filtered:
+        raw = scratch if scratch is not None else [c.new_empty(c.shape) for c in out3]
     if pml is None:
-        N.call(N.op("pic_yee_update_e", f64), desc, N.p3(E3), N.p3(B3), N.p3(J3), N.p3(out3), stream)
+        N.call(N.op("pic_yee_update_e", f64), desc, N.p3(E3), N.p3(B3), N.p3(J3), N.p3(raw), stream)
     else:
-        N.call("pic_yee_update_e_pml", desc, N.p3(E3), N.p3(B3), N.p3(J3), N.p3(out3),
+        N.call("pic_yee_update_e_pml", desc, N.p3(E3), N.p3(B3), N.p3(J3), N.p3(raw),
                ctypes.byref(pml_struct(*pml, desc=desc)), stream)
-    if desc.alpha != 1.0:
-        tmp = scratch if scratch is not None else [c.clone() for c in out3]
-        for c, t in zip(out3, tmp):
-            N.call(N.op("pic_filter_digital", f64), desc, N.ptr(c), N.ptr(t), float(desc.alpha), stream)
-            c.copy_(t)
-    walls = {0: (1, 2), 1: (0, 2), 2: (0, 1)}
-    changed = desc.alpha != 1.0
-    for axis in range(3):
-        if desc.bc[axis] == 1:
-            changed = True
-            for comp in walls[axis]:
-                N.call(N.op("pic_zero_boundary", f64), desc, N.ptr(out3[comp]), axis, stream)
-    # the update kernels refresh the guard cells themselves; only a filter or the
-    # conducting walls change the interior after that
-    if changed:
-        for c in out3:
-            N.call(N.op("pic_halo_refresh", f64), desc, N.ptr(c), 0, stream)
+    # the kernels refresh the guard cells themselves
+    if filtered:
+        N.call(N.op("pic_filter_refresh", f64), desc, N.p3(raw), N.p3(out3), 0, float(desc.alpha), 0, int(walls), stream)
+    elif walls:
+        N.call(N.op("pic_conducting_walls", f64), desc, N.p3(out3), stream)
     return out3
 
 
