@@ -251,6 +251,27 @@ int pic_fused_push_direct_tiled_gather(const PicDesc* desc, const PicSpecies* sp
                                        float* const J[3], int32_t tile, const int32_t* starts, int32_t min_blocks,
                                        int32_t* workspace, void* stream);
 
+/* The same deposits, and the fused Esirkepov phase, of 3-D particles in any
+ * slot order through cell bins (pic_binned.hip): kind 0 rho, 1 J_from_rhov,
+ * 2 Esirkepov (deposit or fused phase), 3 push.  The workspace query returns -1
+ * where the grid is not covered (an axis of one cell, or more cells than the
+ * bins hold) and, for the push, for small sets.  pic_push_binned samples the
+ * slot order on the device and pushes sorted sets in slot order. */
+int64_t pic_binned_workspace_bytes(const PicDesc* desc, const PicSpecies* sp, int32_t kind);
+int pic_deposit_rho_binned(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in, float* rho,
+                           void* workspace, int64_t workspace_bytes, void* stream);
+int pic_deposit_direct_binned(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in, float* const J[3],
+                              void* workspace, int64_t workspace_bytes, void* stream);
+int pic_deposit_esirkepov_binned(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                 float* const J[3], void* workspace, int64_t workspace_bytes, void* stream);
+int pic_push_binned(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in, const float* const E[3],
+                    const float* const B[3], const float* const E_ext[3], const float* const B_ext[3],
+                    float* const u_out[3], void* workspace, int64_t workspace_bytes, void* stream);
+int pic_fused_push_esirkepov_binned(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                    const float* const E[3], const float* const B[3], const float* const E_ext[3],
+                                    const float* const B_ext[3], PicParticles* out, float* const J[3],
+                                    void* workspace, int64_t workspace_bytes, void* stream);
+
 /* ---- cell sort (particle_initialization.py:89-102, 140-160) ------------- */
 /* key = s*(N+1) + (ix*Ny+iy)*Nz+iz with ix = clip(floor((x+W/2)/dx),0,Nx-1);
  * inactive slots get key s*(N+1) + N. */

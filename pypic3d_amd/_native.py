@@ -87,6 +87,12 @@ SIGNATURES = {
     "pic_deposit_rho": (c_int, [DP, SP, PP, c_vp, c_vp]),
     "pic_deposit_direct_tiled": (c_int, [DP, SP, PP, P3, c_i32, c_vp, c_vp]),
     "pic_deposit_rho_tiled": (c_int, [DP, SP, PP, c_vp, c_i32, c_vp, c_vp]),
+    "pic_binned_workspace_bytes": (c_i64, [DP, SP, c_i32]),
+    "pic_deposit_rho_binned": (c_int, [DP, SP, PP, c_vp, c_vp, c_i64, c_vp]),
+    "pic_deposit_direct_binned": (c_int, [DP, SP, PP, P3, c_vp, c_i64, c_vp]),
+    "pic_deposit_esirkepov_binned": (c_int, [DP, SP, PP, P3, c_vp, c_i64, c_vp]),
+    "pic_push_binned": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, P3, c_vp, c_i64, c_vp]),
+    "pic_fused_push_esirkepov_binned": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_vp, c_i64, c_vp]),
     "pic_fused_push_esirkepov": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_vp]),
     "pic_fused_push_esirkepov_tiled": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_i32, c_vp, c_i32, c_i32,
                                                c_vp, c_vp]),

@@ -245,6 +245,27 @@ def soa_view(store):
     return store.permute(1, 2, 0).unsqueeze(0).unsqueeze(0).unsqueeze(0)
 
 
+# Fewer slots than this deposit faster with plain atomics than through the four
+# launches of the binned deposits.
+BINNED_SLOTS = 1 << 15
+RHO, DIRECT, ESIRKEPOV, PUSH = 0, 1, 2, 3
+
+
+def binned_workspace(desc, sp, kind, device):
+    """Scratch of a binned deposit (pic_binned.hip) on particles in any slot
+    order, or None where the slot-ordered kernel is used instead: few slots, a
+    grid the bins do not cover, or no memory for the records."""
+    if sp.count * sp.slots < BINNED_SLOTS:
+        return None
+    nbytes = int(N.lib().pic_binned_workspace_bytes(desc, sp, kind))
+    if nbytes <= 0:
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device=device)
+    except torch.OutOfMemoryError:
+        return None
+
+
 def tiled_particles_from_arrays(x, u, active, device="cuda", dtype=torch.float32):
     """Build TiledParticles on the GPU from (S, P, 3) arrays (NumPy or torch);
     dtype float32, or float64 for the FP64 path."""

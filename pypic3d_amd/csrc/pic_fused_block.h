@@ -137,6 +137,208 @@ __device__ inline float gather_cic(const float* __restrict__ f, const float* __r
     return ax.w0 * (ay.w0 * c00 + ay.w1 * c01) + ax.w1 * (ay.w0 * c10 + ay.w1 * c11);
 }
 
+// Gather stencil of one axis and node line with kN = 2 (first order: points a,
+// a+1) or 3 (second order: a-1 .. a+1) points, wrapped into the ghosted line; a
+// reduced axis is point g with weight one.  Compile-time point counts keep the
+// stencil in registers.
+template <int kShape>
+struct PointAxis {
+    static constexpr int kN = kShape == 1 ? 2 : 3;
+    int p[kN];
+    float w[kN];
+};
+
+template <int kShape>
+__device__ inline void point_axis(float x, double org, double sp, int L, int g, bool active, PointAxis<kShape>& s) {
+    if (!active) {
+#pragma unroll
+        for (int q = 0; q < s.kN; ++q) {
+            s.p[q] = g;
+            s.w[q] = q == 0 ? 1.0f : 0.0f;
+        }
+        return;
+    }
+    const float isp32 = (float)(1.0 / sp);
+    const int a = anchor_fast(x, (float)org, isp32, org, sp, kShape);
+    const double dl = (double)x - node_coord(a, sp, org);
+    if constexpr (kShape == 1) {
+        const float r = (float)dl * isp32;
+        s.p[0] = pmod(a, L);
+        s.p[1] = pmod(a + 1, L);
+        s.w[0] = 1.0f - r;
+        s.w[1] = r;
+    } else {
+        double w[3];
+        shape3(dl * (1.0 / sp), 2, w);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            s.p[q] = pmod(a - 1 + q, L);
+            s.w[q] = (float)w[q];
+        }
+    }
+}
+
+// Weighted sum of kN values in the order of gather_cic (the roundings of the
+// first-order kernels then agree).
+template <int kN>
+__device__ inline float weighted(const float (&v)[kN], const float (&w)[kN]) {
+    if constexpr (kN == 2) return v[0] * w[0] + v[1] * w[1];
+    else return v[0] * w[0] + v[1] * w[1] + v[2] * w[2];
+}
+
+// kN consecutive floats at p (4-byte aligned): one load instruction.
+template <int kN>
+__device__ inline void load_run(const float* p, float (&v)[kN]) {
+    __builtin_memcpy(v, p, sizeof(v));
+}
+
+// Value of one component at the particle.  kRun: the z points are consecutive
+// (every lane of the wave), so a stencil row is one load instead of kN; a
+// random-order gather is bound by its load instructions (one line per lane
+// each).  Offsets are 32-bit where the component spans under 4 GiB.
+template <int kShape, bool kRun, class Idx>
+__device__ inline float gather_point(const float* __restrict__ f, const float* __restrict__ fe, Idx sx, Idx sy,
+                                     const PointAxis<kShape>& ax, const PointAxis<kShape>& ay,
+                                     const PointAxis<kShape>& az) {
+    constexpr int kN = PointAxis<kShape>::kN;
+    float sx_[kN];
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+        float sy_[kN];
+#pragma unroll
+        for (int j = 0; j < kN; ++j) {
+            const Idx row = (Idx)ax.p[i] * sx + (Idx)ay.p[j] * sy;
+            float v[kN];
+            if constexpr (kRun) {
+                load_run<kN>(f + (row + (Idx)az.p[0]), v);
+            } else {
+#pragma unroll
+                for (int k = 0; k < kN; ++k) v[k] = f[row + (Idx)az.p[k]];
+            }
+            if (fe) {
+                float e[kN];
+                if constexpr (kRun) {
+                    load_run<kN>(fe + (row + (Idx)az.p[0]), e);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < kN; ++k) e[k] = fe[row + (Idx)az.p[k]];
+                }
+#pragma unroll
+                for (int k = 0; k < kN; ++k) v[k] += e[k];
+            }
+            sy_[j] = weighted<kN>(v, az.w);
+        }
+        sx_[i] = weighted<kN>(ay.w, sy_);
+    }
+    return weighted<kN>(ax.w, sx_);
+}
+
+template <int kShape, bool kRun, class Idx>
+__device__ inline void gather_six(const PicDesc& d, const FieldPtrs& fp, const PointAxis<kShape> (&c)[3],
+                                  const PointAxis<kShape> (&v)[3], float E[3], float B[3]) {
+    const Idx sy = (Idx)d.dims[2], sx = (Idx)d.dims[1] * sy;
+    E[0] = gather_point<kShape, kRun, Idx>(fp.E[0], fp.Ee[0], sx, sy, v[0], c[1], c[2]);
+    E[1] = gather_point<kShape, kRun, Idx>(fp.E[1], fp.Ee[1], sx, sy, c[0], v[1], c[2]);
+    E[2] = gather_point<kShape, kRun, Idx>(fp.E[2], fp.Ee[2], sx, sy, c[0], c[1], v[2]);
+    B[0] = gather_point<kShape, kRun, Idx>(fp.B[0], fp.Be[0], sx, sy, c[0], v[1], v[2]);
+    B[1] = gather_point<kShape, kRun, Idx>(fp.B[1], fp.Be[1], sx, sy, v[0], c[1], v[2]);
+    B[2] = gather_point<kShape, kRun, Idx>(fp.B[2], fp.Be[2], sx, sy, v[0], v[1], c[2]);
+}
+
+// The six staggered components (particle_push.py:63-68) at x, any
+// dimensionality.
+template <int kShape, class Idx>
+__device__ inline void gather_points(const PicDesc& d, const FieldPtrs& fp, const float x[3], float E[3], float B[3]) {
+    PointAxis<kShape> c[3], v[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const bool act = d.n[a] > 1;
+        point_axis<kShape>(x[a], d.org_c[a], d.sp_c[a], d.dims[a], d.g, act, c[a]);
+        point_axis<kShape>(x[a], d.org_v[a], d.sp_v[a], d.dims[a], d.g, act, v[a]);
+    }
+    constexpr int kLast = PointAxis<kShape>::kN - 1;
+    const bool run = c[2].p[kLast] - c[2].p[0] == kLast && v[2].p[kLast] - v[2].p[0] == kLast;
+    if (__all(run)) gather_six<kShape, true, Idx>(d, fp, c, v, E, B);
+    else gather_six<kShape, false, Idx>(d, fp, c, v, E, B);
+}
+
+// Second-order Esirkepov of a 3-D particle whose anchor moves by at most one
+// cell per axis: the 5-slot new-anchor frame of Esirkepov.py:158-189 with
+// compile-time slots.  Without a crossing in the wave only slots 1..3 are
+// alive.
+struct TscAxis {
+    int base;
+    float S0[5], D[5], C[4];
+};
+
+__device__ inline bool tsc_axis(double xo, double xn, double org, double sp, double dd, TscAxis& e, bool& moved) {
+    const int ao = anchor_of(xo, org, sp, 2), an = anchor_of(xn, org, sp, 2);
+    const int shift = an - ao;
+    double wo[3], wn[3];
+    shape3((xo - node_coord(ao, sp, org)) / dd, 2, wo);
+    shape3((xn - node_coord(an, sp, org)) / dd, 2, wn);
+    const double S1[5] = {0.0, wn[0], wn[1], wn[2], 0.0};
+    const double S0[5] = {shift > 0 ? wo[0] : 0.0, shift > 0 ? wo[1] : (shift < 0 ? 0.0 : wo[0]),
+                          shift > 0 ? wo[2] : (shift < 0 ? wo[0] : wo[1]),
+                          shift > 0 ? 0.0 : (shift < 0 ? wo[1] : wo[2]), shift < 0 ? wo[2] : 0.0};
+    const int last = shift < 0 ? 4 : 3;          // the running sum is zero from the last live slot on
+    double run = 0.0;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) {
+        const double D = S1[q] - S0[q];
+        run += D;
+        e.S0[q] = (float)S0[q];
+        e.D[q] = (float)D;
+        if (q < 4) e.C[q] = q < last ? (float)run : 0.0f;
+    }
+    e.base = an - 2;
+    moved = moved || shift != 0;
+    return shift >= -1 && shift <= 1;
+}
+
+template <int kLo, int kHi, int kC, class Sink>
+__device__ inline void tsc_component(const PicDesc& d, float pre, const TscAxis& A, const TscAxis& P, const TscAxis& Q,
+                                     const Sink& sink) {
+#pragma unroll
+    for (int j = kLo; j <= kHi; ++j) {
+#pragma unroll
+        for (int k = kLo; k <= kHi; ++k) {
+            const float y = P.S0[j] * Q.S0[k] + 0.5f * (P.S0[j] * Q.D[k] + P.D[j] * Q.S0[k]) +
+                            (1.0f / 3.0f) * P.D[j] * Q.D[k];
+#pragma unroll
+            for (int i = kLo; i < kHi; ++i) {
+                const int ic = A.base + i, i1 = P.base + j, i2 = Q.base + k;
+                sink.add(d, kC, kC == 0 ? ic : i1, kC == 0 ? i1 : (kC == 1 ? ic : i2), kC == 2 ? ic : i2,
+                         pre * A.C[i] * y);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);     // bound the live terms to one row
+    }
+}
+
+template <class Sink>
+__device__ inline void esirkepov_second_order(const PicDesc& d, const SpeciesK& k, const double xo[3],
+                                              const double xn[3], const float v[3], const Sink& sink) {
+    TscAxis ax[3];
+    bool ok = true, moved = false;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) ok = tsc_axis(xo[a], xn[a], d.org_c[a], d.sp_c[a], d.d[a], ax[a], moved) && ok;
+    if (!ok) {
+        float* const J[3] = {sink.J[0], sink.J[1], sink.J[2]};
+        esirkepov_particle(d, k.qw, xo, xn, v, J);
+        return;
+    }
+    if (moved) {
+        tsc_component<0, 4, 0>(d, k.pre[0], ax[0], ax[1], ax[2], sink);
+        tsc_component<0, 4, 1>(d, k.pre[1], ax[1], ax[0], ax[2], sink);
+        tsc_component<0, 4, 2>(d, k.pre[2], ax[2], ax[0], ax[1], sink);
+    } else {
+        tsc_component<1, 3, 0>(d, k.pre[0], ax[0], ax[1], ax[2], sink);
+        tsc_component<1, 3, 1>(d, k.pre[1], ax[1], ax[0], ax[2], sink);
+        tsc_component<1, 3, 2>(d, k.pre[2], ax[2], ax[0], ax[1], sink);
+    }
+}
+
 // Deposit targets.  GlobalSink adds straight into the J arrays (JAX scatter
 // "drop" index semantics, Esirkepov.py:232-240).  BoxSink accumulates into an
 // LDS box of B^3 nodes per component whose origin is `o` (array indices) and

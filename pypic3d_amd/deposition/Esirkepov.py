@@ -10,7 +10,7 @@ particles and J run the FP64 path.
 from __future__ import annotations
 
 from .. import _native as N
-from .._tensors import as_field3, check_fields, is_f64, like_input, make_desc, make_species, particle_planes, pic_particles
+from .._tensors import ESIRKEPOV, as_field3, binned_workspace, check_fields, is_f64, like_input, make_desc, make_species, particle_planes, pic_particles
 
 
 def deposit_esirkepov_into(desc, sp, pp, J3, stream, fill=True):
@@ -18,7 +18,11 @@ def deposit_esirkepov_into(desc, sp, pp, J3, stream, fill=True):
     f64 = is_f64(J3[0])
     if fill:
         N.call(N.op("pic_zero_fields", f64), desc, N.p3(J3), stream)
-    N.call(N.op("pic_deposit_esirkepov", f64), desc, sp, pp, N.p3(J3), stream)
+    ws = None if f64 else binned_workspace(desc, sp, ESIRKEPOV, J3[0].device)
+    if ws is not None:
+        N.call("pic_deposit_esirkepov_binned", desc, sp, pp, N.p3(J3), N.ptr(ws), ws.numel(), stream)
+    else:
+        N.call(N.op("pic_deposit_esirkepov", f64), desc, sp, pp, N.p3(J3), stream)
     finish_current(desc, J3, stream)
 
 

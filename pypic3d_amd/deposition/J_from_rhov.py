@@ -9,7 +9,7 @@ codes, and the optional bilinear / digital filter (+ refresh).
 from __future__ import annotations
 
 from .. import _native as N
-from .._tensors import as_field3, check_fields, is_f64, like_input, make_desc, make_species, particle_planes, pic_particles
+from .._tensors import DIRECT, as_field3, binned_workspace, check_fields, is_f64, like_input, make_desc, make_species, particle_planes, pic_particles
 
 
 def deposit_direct_into(desc, sp, pp, J3, current_filter, stream, scratch=None, tile=None, starts=None):
@@ -20,7 +20,11 @@ def deposit_direct_into(desc, sp, pp, J3, current_filter, stream, scratch=None, 
     if tile and not f64:
         N.call("pic_deposit_direct_tiled", desc, sp, pp, N.p3(J3), int(tile), N.ptr(starts), stream)
     else:
-        N.call(N.op("pic_deposit_direct", f64), desc, sp, pp, N.p3(J3), stream)
+        ws = None if f64 else binned_workspace(desc, sp, DIRECT, J3[0].device)
+        if ws is not None:
+            N.call("pic_deposit_direct_binned", desc, sp, pp, N.p3(J3), N.ptr(ws), ws.numel(), stream)
+        else:
+            N.call(N.op("pic_deposit_direct", f64), desc, sp, pp, N.p3(J3), stream)
     finish_direct_current(desc, J3, current_filter, stream, scratch)
 
 

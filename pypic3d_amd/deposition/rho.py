@@ -7,7 +7,7 @@ particle codes, digital filter (+ refresh) when current_filter == "digital".
 from __future__ import annotations
 
 from .. import _native as N
-from .._tensors import as_field3, check_fields, is_f64, like_input, make_desc, make_species, particle_planes, pic_particles
+from .._tensors import RHO, as_field3, binned_workspace, check_fields, is_f64, like_input, make_desc, make_species, particle_planes, pic_particles
 
 
 def deposit_rho_into(desc, sp, pp, rho3, current_filter, stream, scratch=None, tile=None, starts=None):
@@ -22,7 +22,11 @@ def deposit_rho_into(desc, sp, pp, rho3, current_filter, stream, scratch=None, t
     if tile and not f64:
         N.call("pic_deposit_rho_tiled", desc, sp, pp, N.ptr(raw), int(tile), N.ptr(starts), stream)
     else:
-        N.call(N.op("pic_deposit_rho", f64), desc, sp, pp, N.ptr(raw), stream)
+        ws = None if f64 else binned_workspace(desc, sp, RHO, raw.device)
+        if ws is not None:
+            N.call("pic_deposit_rho_binned", desc, sp, pp, N.ptr(raw), N.ptr(ws), ws.numel(), stream)
+        else:
+            N.call(N.op("pic_deposit_rho", f64), desc, sp, pp, N.ptr(raw), stream)
     N.call(N.op("pic_finish_current", f64), desc, N.p1(raw), 1, stream)
     if filtered:
         N.call(N.op("pic_filter_refresh", f64), desc, N.p1(raw), N.p1(rho3), 0, float(desc.alpha), 1, 0, stream)

@@ -16,12 +16,12 @@ from __future__ import annotations
 import torch
 
 from . import _native as N
-from ._tensors import (as_field3, check_fields, is_f64, like_input, make_desc, make_species, new_soa, particle_planes,
-                       pic_particles)
+from ._tensors import (ESIRKEPOV, as_field3, binned_workspace, check_fields, is_f64, like_input, make_desc,
+                       make_species, new_soa, particle_planes, pic_particles)
 from .deposition.Esirkepov import deposit_esirkepov_into, finish_current
 from .deposition.J_from_rhov import deposit_direct_into
 from .particles.particle_class import TiledParticles
-from .pusher.particle_push import check_pusher
+from .pusher.particle_push import check_pusher, push_into
 from .solvers.electrostatic_yee import electrostatic_fields_into
 from .solvers.first_order_yee import _check_pml, _pml_args, yee_b, yee_e
 from .utils import is_all_zero
@@ -88,15 +88,19 @@ def time_loop_electrodynamic(particles, species_config, fields, static_parameter
         act_out = act.new_empty(act.shape)
         N.call("pic_zero_fields", desc, N.p3(J3), stream)
         out = pic_particles([xs[0], xs[1], xs[2]], [us[0], us[1], us[2]], act_out)
-        N.call("pic_fused_push_esirkepov", desc, sp, pic_particles(xp, up, act), N.p3(E3), N.p3(B3), Ee, Be,
-               out, N.p3(J3), stream)
+        ws = binned_workspace(desc, sp, ESIRKEPOV, dev)
+        if ws is not None:
+            N.call("pic_fused_push_esirkepov_binned", desc, sp, pic_particles(xp, up, act), N.p3(E3), N.p3(B3), Ee,
+                   Be, out, N.p3(J3), N.ptr(ws), ws.numel(), stream)
+        else:
+            N.call("pic_fused_push_esirkepov", desc, sp, pic_particles(xp, up, act), N.p3(E3), N.p3(B3), Ee, Be,
+                   out, N.p3(J3), stream)
         finish_current(desc, J3, stream)
         new_particles = TiledParticles(x=xv, u=uv, active=act_out.view(1, 1, 1, S, P))
     else:
         us, uv = new_soa(S, P, dev, dtype)
-        N.call(N.op("pic_push", f64), desc, sp, pic_particles(xp, up, act), N.p3(E3), N.p3(B3), Ee, Be,
-               N.p3([us[0], us[1], us[2]]), stream)
         u_planes = [us[0], us[1], us[2]]
+        push_into(desc, sp, xp, up, act, E3, B3, Ee, Be, u_planes, stream)
         act_h = act.clone()
         xh, _ = _advance(desc, sp, xp, u_planes, act_h, 0.5, stream)
         N.call(N.op("pic_particle_boundaries", f64), desc, sp, pic_particles(xh, u_planes, act_h), stream)
@@ -145,9 +149,8 @@ def time_loop_electrostatic(particles, species_config, fields, static_parameters
     Ee, Be = _external(desc, external_fields, torch.float32)
     dev = xp[0].device
     us, uv = new_soa(S, P, dev)
-    N.call("pic_push", desc, sp, pic_particles(xp, up, act), N.p3(E3), N.p3(B3), Ee, Be,
-           N.p3([us[0], us[1], us[2]]), stream)
     u_planes = [us[0], us[1], us[2]]
+    push_into(desc, sp, xp, up, act, E3, B3, Ee, Be, u_planes, stream)
     act_o = act.clone()
     xf, xv = _advance(desc, sp, xp, u_planes, act_o, 1.0, stream)
     N.call("pic_particle_boundaries", desc, sp, pic_particles(xf, u_planes, act_o), stream)
