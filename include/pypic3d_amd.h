@@ -207,6 +207,14 @@ int pic_fused_push_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, co
                                    const float* const B_ext[3], PicParticles* out, float* const J[3], int32_t tile,
                                    const int32_t* starts, int32_t rounds, int32_t min_blocks, int32_t* workspace,
                                    void* stream);
+/* pic_fused_push_esirkepov_tiled on a grid whose lines are not FP32-exact: the
+ * same launch with FP64 anchors.  workspace is used on every grid (the rare
+ * list).  On an exact grid it is that entry point. */
+int pic_fused_push_esirkepov_tiled_general(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                           const float* const E[3], const float* const B[3],
+                                           const float* const E_ext[3], const float* const B_ext[3],
+                                           PicParticles* out, float* const J[3], int32_t tile,
+                                           const int32_t* starts, int32_t rounds, int32_t* workspace, void* stream);
 /* pic_fused_push_esirkepov_tiled on particles re-binned without their
  * gather (pic_tile_rebin with out == NULL): slot i of the sorted order reads
  * in's slot gather[i] (perm of that re-bin; starts index the sorted order)

@@ -96,6 +96,8 @@ SIGNATURES = {
     "pic_fused_push_esirkepov": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_vp]),
     "pic_fused_push_esirkepov_tiled": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_i32, c_vp, c_i32, c_i32,
                                                c_vp, c_vp]),
+    "pic_fused_push_esirkepov_tiled_general": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_i32, c_vp, c_i32,
+                                                       c_vp, c_vp]),
     "pic_fused_push_esirkepov_tiled_gather": (c_int, [DP, SP, PP, c_vp, P3, P3, c_vp, c_vp, PP, P3, c_i32, c_vp,
                                                       c_i32, c_i32, c_vp, c_vp]),
     "pic_fused_push_direct_tiled_gather": (c_int, [DP, SP, PP, c_vp, P3, P3, c_vp, c_vp, PP, P3, c_i32, c_vp,

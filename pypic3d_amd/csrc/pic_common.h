@@ -203,16 +203,19 @@ __device__ inline void row_scan_step(int r, int& seg, float (&v)[kN]) {
 // lanes (other lanes hold partial sums, which the caller discards).  Equal
 // keys in lanes that are not consecutive form separate runs.  Every lane of
 // the wave must execute it.
-template <int kN>
+// kRow: 16, or 4 for aligned groups of four lanes in half the steps.
+template <int kRow = 16, int kN>
 __device__ inline bool row_run_sums(int key, float (&v)[kN]) {
-    const int r = (int)(threadIdx.x & 15u);
+    const int r = (int)(threadIdx.x & (kRow - 1u));
     const int kprev = dpp_row_shr<1>(key), knext = dpp_row_shl1(key);
     int seg = ((r == 0) | (kprev != key)) ? 1 : 0;    // run head
     row_scan_step<1>(r, seg, v);
     row_scan_step<2>(r, seg, v);
-    row_scan_step<4>(r, seg, v);
-    row_scan_step<8>(r, seg, v);
-    return (r == 15) | (knext != key);
+    if constexpr (kRow == 16) {
+        row_scan_step<4>(r, seg, v);
+        row_scan_step<8>(r, seg, v);
+    }
+    return (r == kRow - 1) | (knext != key);
 }
 
 // kP consecutive floats from 16-byte (kP = 4) or 8-byte (kP = 2) aligned memory

@@ -54,6 +54,94 @@ __device__ inline void loads_together(const float (&x)[3], const float (&u)[3]) 
     asm volatile("" ::"v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(u[0]), "v"(u[1]), "v"(u[2]));
 }
 
+// Grid constants of the tile kernels.  Anchors are found relative to the first
+// node of the tile's field box: an FP32 estimate that is never too small
+// (isp_up or bias) and at most one too large, corrected by one comparison with
+// the node.  On an exact grid node and offset are FP32 (see ExactGrid); on any
+// other they are evaluated in FP64 as the reference does, and a position within
+// edge of a face, where its division could round either way, is left to the
+// rare list.
+struct TileGrid {
+    float sp[3], isp[3], isp_up[3], half[3], inv_d[3];
+    float bias[3], edge[3];
+    float lim[3];       // a new offset from the cell's middle below lim stays in the cell (ExactGrid::band_*)
+    double sp64[3], org64[3], half64[3];
+    // the rest of cross_axis' arguments, and the time step: scalar kernel arguments, where
+    // a division or conversion in the kernel would hold a vector register across its loops
+    double inv_d64[3];
+    float org32[3], dt32;
+};
+
+// False where a grid's vertex line is not the centre line shifted by half a
+// spacing up to rounding (no grid of the solver; the slot-ordered kernel takes
+// any lines).
+bool make_tile_grid(const PicDesc& d, TileGrid& t) {
+    for (int a = 0; a < 3; ++a) {
+        const double org = d.org_c[a], sp = d.sp_c[a];
+        if (!(sp > 0.0) || d.dims[a] > (1 << 20) || !(d.d[a] > 0.0)) return false;
+        const double off = d.org_v[a] - org - 0.5 * sp;
+        if (std::fabs(off) > 1.0e-7 * sp || std::fabs(d.sp_v[a] - sp) * d.dims[a] > 1.0e-7 * sp) return false;
+        if (std::fabs(org) > 4.0e6 * sp) return false;
+        t.sp[a] = (float)sp;
+        t.isp[a] = (float)(1.0 / sp);
+        t.isp_up[a] = t.isp[a] * (1.0f + 0x1p-21f);
+        t.half[a] = 0.5f * t.sp[a];
+        t.inv_d[a] = (float)(1.0 / d.d[a]);
+        // FP32 errors of (x - node) * isp: half an ulp of the node and of x, the rounding of the rest
+        t.bias[a] = 0x1p-22f * ((float)(std::fabs(org) / sp) + d.dims[a] + 32.0f);
+        t.edge[a] = (float)((0.5 - 0x1p-20) * sp);
+        t.lim[a] = (float)((0.5 - 0x1p-19) * sp);
+        t.sp64[a] = sp;
+        t.org64[a] = org;
+        t.half64[a] = 0.5 * sp;
+        t.inv_d64[a] = 1.0 / d.d[a];
+        t.org32[a] = (float)org;
+    }
+    t.dt32 = (float)d.dt;
+    return true;
+}
+
+// Node coordinate of the reference (a*sp + org, both roundings) for an index
+// held as a float.
+__device__ inline double node_at(float a, double sp, double org) {
+#pragma clang fp contract(off)
+    return (double)a * sp + org;
+}
+
+// Cell of x relative to the field box (first node nb, index fo), offset dc from
+// its node, offset q from its middle (the vertex node), whether x is in its
+// upper half, and offset dv from the vertex node below x.  False: too near a
+// face for the FP64 evaluation to be certain.
+template <bool kExact>
+__device__ inline bool tile_anchor(const TileGrid& tg, int a, float x, float nb, float fo, float& f, float& dc,
+                                   float& q, bool& up, float& dv) {
+    if constexpr (kExact) {
+        f = floorf((x - nb) * tg.isp_up[a]);
+        float nd = fmaf(f, tg.sp[a], nb);
+        const float b = x < nd ? 1.0f : 0.0f;
+        f -= b;
+        nd = fmaf(-b, tg.sp[a], nd);
+        const float mid = nd + tg.half[a];
+        dc = x - nd;
+        q = x - mid;
+        up = x >= mid;
+        dv = x - (up ? mid : mid - tg.sp[a]);
+        return true;
+    } else {
+        f = floorf(fmaf(x - nb, tg.isp[a], tg.bias[a]));
+        double dd = (double)x - node_at(f + fo, tg.sp64[a], tg.org64[a]);
+        const bool below = dd < 0.0;
+        f -= below ? 1.0f : 0.0f;
+        dd += below ? tg.sp64[a] : 0.0;
+        const double q64 = dd - tg.half64[a];
+        dc = (float)dd;
+        q = (float)q64;
+        up = q64 >= 0.0;
+        dv = (float)(up ? q64 : q64 + tg.sp64[a]);
+        return fabsf(q) < tg.edge[a];
+    }
+}
+
 // Host check for ExactGrid (see its comment); false when any axis fails.
 bool make_exact_grid(const PicDesc& d, ExactGrid& eg) {
     for (int a = 0; a < 3; ++a) {

@@ -2,6 +2,7 @@
 // and its design notes live in pic_fused_block.h).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 
 #include "pic_exact_grid.h"
 #include "pic_fused_block.h"
@@ -91,49 +92,6 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void fused_tiled_kernel(PicDe
     }
 }
 
-// Grouped variant of the tile-ordered launch.  Thread t of a chunk owns kP
-// consecutive sorted slots [base + kP t, base + kP t + kP), loaded and stored
-// as one kP-wide vector per plane when the group lies inside the block's
-// range and the planes are aligned.  Sorted slots of one cell are contiguous,
-// so a thread's particles mostly share a cell: their twelve regular-case
-// values are summed in registers and added into the LDS box when the cell
-// changes and once at the end of the group, which replaces the wave
-// segmented scan.  Face crossings go through the block's queue as in
-// fused_block.
-// Per-block LDS queue of face-crossing particles (slot offset from the chunk
-// base and the pushed velocity); a full queue sends further particles to the
-// rare list.
-constexpr int kCrossCap = 512;
-struct CrossQueue {
-    int q_idx[kCrossCap];
-    float q_f[6][kCrossCap];
-    int q_n;
-};
-
-// Add the twelve regular-case values of a particle anchored at cell
-// (a0, a1, a2) (RegularLayout<3> order) into the box, or into J when the
-// 2x2x2 node block around the cell leaves the box.
-template <int kB>
-__device__ inline void flush_cell(const PicDesc& d, const BoxSink& sink, int a0, int a1, int a2, const float acc[12]) {
-    const int bi = a0 - sink.o[0], bj = a1 - sink.o[1], bk = a2 - sink.o[2];
-    if ((unsigned)bi < (unsigned)(kB - 1) && (unsigned)bj < (unsigned)(kB - 1) && (unsigned)bk < (unsigned)(kB - 1)) {
-        float* p = sink.box + (bi * kB + bj) * kB + bk;
-#pragma unroll
-        for (int m = 0; m < 12; ++m) {
-            int dx, dy, dz;
-            RegularLayout<3>::delta(m, dx, dy, dz);
-            atomicAdd(p + (m >> 2) * kB * kB * kB + (dx * kB + dy) * kB + dz, acc[m]);
-        }
-    } else {
-#pragma unroll
-        for (int m = 0; m < 12; ++m) {
-            int dx, dy, dz;
-            RegularLayout<3>::delta(m, dx, dy, dz);
-            deposit_at(sink.J[m >> 2], d, a0 + dx, a1 + dy, a2 + dz, acc[m]);
-        }
-    }
-}
-
 // Periodic wrap of wrap_periodic_position (grid_and_stencil.py:14-35) with
 // the one-period cases done without fmod (fmod(s, W) = s - W exactly for
 // W <= s < 2W, and = s for -W < s < 0); anything else takes the general form.
@@ -217,75 +175,34 @@ __device__ inline void tile_particle_general(const PicDesc& d, const SpeciesK& k
     out.active[i] = act ? 1 : 0;
 }
 
-// Tile-ordered launch on an exact grid.  Block b owns the sorted slot range
-// [starts[b], starts[b+1]) of one (species, tile) pair.  Thread t of a chunk
-// owns kP consecutive slots; sorted slots of one cell are contiguous, so a
-// thread's particles mostly share a cell and their twelve regular-case values
-// are summed in registers and added into the LDS current box when the cell
-// changes; at the end of the group the lanes of each 16-lane row first sum
-// their values over equal cells (row_run_sums), so one lane per cell and row
-// adds into the box.  Fields are
-// gathered from the LDS field box.  Particles that cross a face go to the
-// block's crossing queue (3-slot deposit into the box after the chunk).
-// Anything else -- a particle outside the tile's field box or the exact
-// anchor range, a step of a cell or more on some axis, a crossing that finds
-// the queue full -- is appended to the rare list (rare[0] = count, slots from
-// rare[1]) without being stored; fused_tile_rare_kernel then runs it whole.
-// Keeping those paths out of this kernel keeps its register count low.
-
+// A block-uniform value computed by vector instructions, moved to a scalar register.
+__device__ inline float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
 
 __device__ inline void rare_push(int32_t* rare, int64_t i) {
     const int p = atomicAdd(rare, 1);
     rare[1 + p] = (int32_t)i;
 }
 
-// 3-slot crossing frame of one axis (the values cross_axis computes in FP64)
-// from the quantities the fast loop queues: the anchor step st = a_new -
-// a_old in {-1, 0, +1}, ro = (x_old - node_old)/d and f = (x_new -
-// node_new)/d, or the step itself v dt/d when st = 0 (no cancellation then).
-// rel is the old anchor relative to the box origin; b becomes the frame's
-// first node relative to it.
-__device__ inline void cross_frame(int rel, int st, float ro, float f, CrossAxis& e) {
-    if (st == 0) {                    // frame (a, a+1, -): S0 = (1-ro, ro), D = (-dl, dl)
-        e.b = rel;
-        e.S0[0] = 1.0f - ro;
-        e.S0[1] = ro;
-        e.S0[2] = 0.0f;
-        e.D[0] = -f;
-        e.D[1] = f;
-        e.D[2] = 0.0f;
-        e.C0 = -f;
-        e.C1 = 0.0f;
-    } else if (st > 0) {              // frame (a, a+1, a+2): S0 = (1-ro, ro, 0), S1 = (0, 1-rn, rn)
-        e.b = rel;
-        e.S0[0] = 1.0f - ro;
-        e.S0[1] = ro;
-        e.S0[2] = 0.0f;
-        e.D[0] = ro - 1.0f;
-        e.D[2] = f;
-        e.D[1] = -(e.D[0] + f);
-        e.C0 = e.D[0];
-        e.C1 = -f;
-    } else {                          // frame (a-1, a, a+1): S0 = (0, 1-ro, ro), S1 = (1-rn, rn, 0)
-        e.b = rel - 1;
-        e.S0[0] = 0.0f;
-        e.S0[1] = 1.0f - ro;
-        e.S0[2] = ro;
-        e.D[0] = 1.0f - f;
-        e.D[2] = -ro;
-        e.D[1] = -(e.D[0] - ro);
-        e.C0 = e.D[0];
-        e.C1 = ro;
-    }
+// LDS accumulators of the current boxes.  ds_add_f64 takes 0.24-0.36 cycles per
+// lane on this card and ds_add_f32 3.0, so the 4-cell tiles sum in FP64; the
+// 8-cell tiles keep FP32, whose box leaves room for two blocks per CU.
+template <int kT>
+using BoxSum = std::conditional_t<kT == 4, double, float>;
+
+template <class T>
+__device__ inline void box_add(T* p, float v) {
+    unsafeAtomicAdd(p, (T)v);
 }
 
 // Face-crossing deposit (the 54 terms of crossing_deposit) straight into the
 // LDS box when the particle's 3x3x3 frame lies inside it: one base address,
 // the term offsets are compile-time constants, no per-term bounds checks.
 // pre[c] = -(q w / (d_p d_q dt)) as in SpeciesK.
-template <int kC, int kB>
+template <int kC, int kB, class T>
 __device__ inline void crossing_component_box(const float pre, const CrossAxis& A, const CrossAxis& P,
-                                              const CrossAxis& Q, float* p) {
+                                              const CrossAxis& Q, T* p) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
         const float ci = i == 0 ? A.C0 : A.C1;
@@ -300,96 +217,131 @@ __device__ inline void crossing_component_box(const float pre, const CrossAxis& 
                 const int dx = kC == 0 ? i : j;
                 const int dy = kC == 0 ? j : (kC == 1 ? i : k);
                 const int dz = kC == 2 ? i : k;
-                atomicAdd(p + kC * kB * kB * kB + (dx * kB + dy) * kB + dz, w * y);
+                box_add(p + kC * kB * kB * kB + (dx * kB + dy) * kB + dz, w * y);
             }
+            __builtin_amdgcn_sched_barrier(0);   // bound the live terms to one row of three
         }
-        __builtin_amdgcn_sched_barrier(0);   // bound the live terms to one row of nine
     }
 }
 
-// Frames given relative to the box origin; the caller has checked that
-// every frame base lies in [0, kB - 3].
-template <int kB>
-__device__ inline void crossing_deposit_box(const SpeciesK& k, const CrossAxis& cx, const CrossAxis& cy,
-                                            const CrossAxis& cz, float* box) {
-    float* p = box + (cx.b * kB + cy.b) * kB + cz.b;
-    crossing_component_box<0, kB>(k.pre[0], cx, cy, cz, p);
-    crossing_component_box<1, kB>(k.pre[1], cy, cx, cz, p);
-    crossing_component_box<2, kB>(k.pre[2], cz, cx, cy, p);
+// Adds the moments of a cell's regular particles into the four nodes of each
+// component: per component M = sum p (1, A_p, A_q, A_p A_q + d_p d_q / 12) with
+// p the current of the particle and A_p, A_q its upper weights along the other
+// axes, so node (1,1) is M3, (1,0) M1 - M3, (0,1) M2 - M3, (0,0) the rest.
+template <int kB, class T>
+__device__ inline void flush_moments(T* p, const float m[12]) {
+    constexpr int kB3 = kB * kB * kB, s[3] = {kB * kB, kB, 1};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        const int sp = s[c == 0 ? 1 : 0], sq = s[c == 2 ? 1 : 2];
+        const float v10 = m[4 * c + 1] - m[4 * c + 3], v01 = m[4 * c + 2] - m[4 * c + 3];
+        box_add(p + c * kB3, (m[4 * c] - m[4 * c + 1]) - v01);
+        box_add(p + c * kB3 + sq, v01);
+        box_add(p + c * kB3 + sp, v10);
+        box_add(p + c * kB3 + sp + sq, m[4 * c + 3]);
+        __builtin_amdgcn_sched_barrier(0);   // bound the live FP64 values to one component
+    }
 }
 
-template <int kT, int kP, int kMinBlocks, int kG, bool kGather>
-__global__ __launch_bounds__(kThreads, kMinBlocks) void fused_tile_exact_kernel(
-    PicDesc d, PicSpecies sp, PicParticles in, FieldPtrs fp, PicParticles out, float* Jx, float* Jy, float* Jz,
-    const int32_t* __restrict__ starts, TileGeom tg, ExactGrid eg, int32_t* __restrict__ rare, int vec_ok, SpeciesTable st,
-    const int32_t* __restrict__ gather) {
-    constexpr int kB = kT + 4;
+// Particles of a chunk that do not stay in their cell: slot offset from the
+// chunk base and pushed velocity; the queue's pass reloads the old position.
+// A full queue sends further particles to the rare list.
+constexpr int kCrossCap = 512;
+struct CrossQueue {
+    int slot[kCrossCap];
+    float v[3][kCrossCap];
+    int n;
+};
+
+// Tile-ordered launch: gather + push + Esirkepov + position update +
+// boundaries.  Block b owns the sorted slot range [starts[b], starts[b+1]) of
+// one (species, tile) pair: the particles that were in that T^3-cell tile at the
+// last sort.  Fields are gathered from an LDS box of the (T+4)^3 nodes around
+// the tile, J is summed in an LDS box of the same nodes and added into the
+// arrays once per block.  Thread t of a chunk owns four
+// consecutive slots, loaded and stored with one 16-byte access per plane;
+// sorted slots of one cell are contiguous, so a thread's particles mostly share
+// a cell and their twelve moments (flush_moments) are summed in registers, added
+// into the box when the cell changes and, after a sum over equal cells of
+// neighbouring lanes, at the end of the group.
+//
+// A particle that leaves its cell, or ends within 2^-19 spacings of a face, is
+// queued with its velocity and deposited in the 3-slot frame after the chunk,
+// by lanes that all do so (in the particle's own iteration that code would run
+// for one lane of most waves).  One whose anchors leave the field box, whose
+// frame leaves the current box, that moves its anchor by two or finds the queue
+// full is put on the rare list (rare[0] = count, slots from rare[1]) and run
+// whole by fused_tile_rare_kernel, which overwrites what is stored here.
+//
+// Bound by VALU instructions (about 600 per 64 particles; the LDS and memory
+// traffic overlap them).  Summing cell moments in registers, FP64 box adds in
+// place of ds_add_f32 and a queue of (slot, velocity) took 128^3 with 2 x 16
+// particles per cell from 1963 to 1548 us (43 G particles/s, 2.2 TB/s) and
+// 256^3 with 32 from 12.1 to 9.7 ms; FP64 anchors in the same kernel take a
+// 64^3 step with 8 and 4 per cell from 1132 to 396 us.  kExact: FP32 anchors of
+// an exact grid, else FP64 ones (TileGrid).  kAll: no species has a frozen axis.
+template <int kT, bool kGather, bool kExact, bool kAll>
+__global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_exact_kernel(
+    PicDesc d, PicParticles in, FieldPtrs fp, PicParticles out, float* Jx, float* Jy, float* Jz,
+    const int32_t* __restrict__ starts, TileGeom tg, TileGrid grid, int32_t* __restrict__ rare, int vec_ok,
+    SpeciesTable st, const int32_t* __restrict__ gather) {
+    constexpr int kP = 4;
+    constexpr int kB = kT + 4;                     // nodes per axis of both boxes
     constexpr int kB3 = kB * kB * kB;
-    constexpr int kFB = kT + 4;
-    constexpr int kFV = kFB * kFB * kFB;
-    constexpr int kChunk = kThreads * kP * kG;     // a thread owns kG * kP consecutive slots
+    constexpr int kChunk = kThreads * kP;          // a thread owns kP consecutive slots
+    // unrolled, the slots need no register shifts (128^3, 2 x 16 particles per cell: 1590 -> 1550 us,
+    // 256^3, 32: 11.0 -> 9.7 ms); with FP64 anchors the rolled loop is shorter on the clock (396, 438 us)
+    constexpr int kUnroll = kExact ? kP : 1;
+    using Sum = BoxSum<kT>;
     __shared__ CrossQueue sh;
-    __shared__ float box[3 * kB3];
-    __shared__ float fbox[6 * kFV];
+    __shared__ Sum box[3 * kB3];
+    __shared__ float fbox[6 * kB3];
     const int b = xcd_block((int)blockIdx.x, (int)gridDim.x);
     const int64_t begin = starts[b], end = starts[b + 1];
     if (begin >= end) return;
     const int t = b % (tg.tiles + 1);
     const int s = b / (tg.tiles + 1);          // blocks are grouped per species
-    int o[3] = {0, 0, 0}, fo[3] = {0, 0, 0};
+    int fo[3] = {0, 0, 0};
     // interior: every particle the fast path handles (anchors inside the field
-    // box, cells c0 - 2 .. c0 + T + 1, a step of under one cell) stays inside
-    // [-W/2, W/2) on every axis, so its particle boundaries do nothing and are
-    // skipped (a block-uniform branch)
+    // box, cells c0 - 2 .. c0 + T + 1, an anchor step of at most one) stays
+    // inside [-W/2, W/2) on every axis, so its particle boundaries do nothing
+    // and are skipped (a block-uniform branch)
     bool interior = t < tg.tiles;
     if (t < tg.tiles) {
-        const int tx = t / (tg.nt[1] * tg.nt[2]), ty = (t / tg.nt[2]) % tg.nt[1], tz = t % tg.nt[2];
-        const int c0[3] = {tx * kT, ty * kT, tz * kT};
+        const int c0[3] = {(t / (tg.nt[1] * tg.nt[2])) * kT, ((t / tg.nt[2]) % tg.nt[1]) * kT, (t % tg.nt[2]) * kT};
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            o[a] = c0[a] + d.g - 1;
             fo[a] = c0[a] + d.g - 2;
             interior = interior && c0[a] >= 3 && c0[a] + kT + 3 <= d.n[a];
         }
     }
-    for (int e = threadIdx.x; e < 3 * kB3; e += kThreads) box[e] = 0.0f;
-    fill_field_box<kFB>(d, fp, fo, fbox);
-    const BoxSink sink{{Jx, Jy, Jz}, box, {o[0], o[1], o[2]}, kB};
-    const FieldBox fb{fbox, {fo[0], fo[1], fo[2]}, kFB};
-    const SpeciesK k = st.k[s];
-    const float fdt = (float)d.dt;
-
-    for (int64_t base = begin & ~(int64_t)(kP - 1); base < end; base += kChunk) {
-        if (threadIdx.x == 0) sh.q_n = 0;
-        __syncthreads();    // also orders the box fills before the first deposits
-        float acc[12];
+    // Positions whose anchors on both node lines lie in the field box and whose
+    // nodes lie in the arrays.  The bounds are rounded up, so an FP32 position
+    // is inside exactly when its value is; off an exact grid a margin keeps the
+    // rounding of the vertex line out.
+    float nb[3], xlo[3], xhi[3];
 #pragma unroll
-        for (int m = 0; m < 12; ++m) acc[m] = 0.0f;
-        int h0 = 0, h1 = 0, h2 = 0;
-        bool have = false;
-#pragma unroll 1
-        for (int g = 0; g < kG; ++g) {
-        const int64_t s0 = base + (int64_t)kP * (kG * (int)threadIdx.x + g);
-        const bool full = vec_ok && s0 >= begin && s0 + kP <= end;
-        // The thread's kP slots are loaded at once, with one kP-wide vector load
-        // per plane when the group lies inside the range (the lanes of a wave
-        // then read contiguous memory, and all loads share one round trip).
-        // One particle per iteration (the loop stays rolled to bound register
-        // pressure): slot j's inputs are taken from the front of PX/PU/pact,
-        // which shift by one, and its outputs enter at the back, so after kP
-        // iterations PX/PU/oact hold the outputs in slot order for the vector
-        // stores.  Slots sent to the rare list are stored as zeros here and
-        // rewritten by the rare kernel.
-        float PX[3][kP], PU[3][kP];
-        uint32_t pact = 0u, oact = 0u;
+    for (int a = 0; a < 3; ++a) {
+        const double org = d.org_c[a], sp = d.sp_c[a], margin = kExact ? 0.0 : 1.0e-6 * sp;
+        nb[a] = uniform((float)(fo[a] * sp + org));
+        xlo[a] = uniform(__double2float_ru(fmax(fo[a] * sp + org + 0.5 * sp, org) + margin));
+        xhi[a] = uniform(__double2float_ru(min(fo[a] + kB - 1, d.dims[a] - 1) * sp + org - margin));
+    }
+    // A group's kP slots are loaded at once, with one kP-wide vector load per
+    // plane when the group lies inside the range (the lanes of a wave then read
+    // contiguous memory, and all loads share one round trip).  The first group is
+    // loaded before the field box is filled, so both wait for memory together.
+    float PX[3][kP], PU[3][kP];
+    uint32_t pact;
+    const auto load_group = [&](int64_t s0, bool full) {
+        pact = 0u;
         if (!kGather && full) {
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
                 load_vec<kP>(in.x[a] + s0, PX[a]);
                 load_vec<kP>(in.u[a] + s0, PU[a]);
             }
-            if constexpr (kP == 4) pact = *reinterpret_cast<const uint32_t*>(in.active + s0);
-            else pact = *reinterpret_cast<const uint16_t*>(in.active + s0);
+            pact = *reinterpret_cast<const uint32_t*>(in.active + s0);
         } else if (kGather && full) {
             // slot i's input is in.*[gather[i]]: the permutation of a re-bin,
             // applied by this launch while it reads.  The flags are loaded
@@ -428,7 +380,32 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void fused_tile_exact_kernel(
                 pact |= (inr && in.active[src] != 0 ? 1u : 0u) << (8 * j);
             }
         }
-#pragma unroll 1
+    };
+    const auto inside = [&](int64_t s0) { return vec_ok && s0 >= begin && s0 + kP <= end; };
+    const int64_t first = begin & ~(int64_t)(kP - 1);
+    load_group(first + (int64_t)kP * (int)threadIdx.x, inside(first + (int64_t)kP * (int)threadIdx.x));
+    for (int e = threadIdx.x; e < 3 * kB3; e += kThreads) box[e] = (Sum)0;
+    fill_field_box<kB>(d, fp, fo, fbox);
+    const SpeciesK& k = st.k[s];
+
+    for (int64_t base = first; base < end; base += kChunk) {
+        if (threadIdx.x == 0) sh.n = 0;
+        __syncthreads();    // also orders the box fills before the first deposits
+        float acc[12];
+#pragma unroll
+        for (int m = 0; m < 12; ++m) acc[m] = 0.0f;
+        int cell = -1;
+        const int64_t s0 = base + (int64_t)kP * (int)threadIdx.x;
+        const bool full = inside(s0);
+        if (base != first) load_group(s0, full);
+        // One particle per iteration (the loop stays rolled to bound register
+        // pressure): slot j's inputs are taken from the front of PX/PU/pact,
+        // which shift by one, and its outputs enter at the back, so after kP
+        // iterations PX/PU/oact hold the outputs in slot order for the vector
+        // stores.  Slots sent to the rare list are stored as zeros here and
+        // rewritten by the rare kernel.
+        uint32_t oact = 0u;
+#pragma unroll kUnroll
         for (int j = 0; j < kP; ++j) {
             const float xf[3] = {PX[0][0], PX[1][0], PX[2][0]};
             float v[3] = {PU[0][0], PU[1][0], PU[2][0]};
@@ -442,145 +419,122 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void fused_tile_exact_kernel(
                     PU[a][q] = PU[a][q + 1];
                 }
             }
-            const int64_t i = s0 + j;
             float ox[3] = {0.0f, 0.0f, 0.0f}, ou[3] = {0.0f, 0.0f, 0.0f};
             uint32_t oa = 0u;
             do {
             if (!act0) break;          // inactive, or outside [begin, end)
-            // ---- anchors on both node lines (grid_and_stencil.py:92-166), exact in FP32
-            int anc[3], anv[3];
-            float dc[3], dv[3], nodec[3];
+            // ---- anchors on both node lines (grid_and_stencil.py:92-166)
             bool fast = true;
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                fast = fast && xf[a] >= eg.xlo[a] && xf[a] < eg.xhi[a];
-                exact_anchors(xf[a], eg.org_c[a], eg.sp_c[a], eg.isp_c[a], eg.half_sp[a], anc[a], dc[a], nodec[a],
-                              anv[a], dv[a]);
-                fast = fast && (unsigned)(anc[a] - fo[a]) < (unsigned)(kFB - 1) &&
-                       (unsigned)(anv[a] - fo[a]) < (unsigned)(kFB - 1);
-            }
+            for (int a = 0; a < 3; ++a) fast = fast & (xf[a] >= xlo[a]) & (xf[a] < xhi[a]);
+            float f[3], dc[3], qm[3], dv[3];
+            bool up[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                fast = tile_anchor<kExact>(grid, a, xf[a], nb[a], (float)fo[a], f[a], dc[a], qm[a], up[a], dv[a]) & fast;
             if (!fast) {
-                rare_push(rare, i);
+                rare_push(rare, s0 + j);
                 break;
             }
+            const int at = (int)fmaf(f[0], (float)(kB * kB), fmaf(f[1], (float)kB, f[2]));
             // ---- gather (boris.py:302-433) from the tile's field box
-            CicAxis gc[3], gv[3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const float rc = dc[a] * eg.isp_c[a], rv = dv[a] * eg.isp_c[a];
-                gc[a].p0 = gc[a].p1 = gv[a].p0 = gv[a].p1 = 0;
-                gc[a].w0 = 1.0f - rc;
-                gc[a].w1 = rc;
-                gv[a].w0 = 1.0f - rv;
-                gv[a].w1 = rv;
-            }
             float E[3], Bf[3];
-            E[0] = gather_box(fb, 0, anv[0], anc[1], anc[2], gv[0], gc[1], gc[2]);
-            E[1] = gather_box(fb, 1, anc[0], anv[1], anc[2], gc[0], gv[1], gc[2]);
-            E[2] = gather_box(fb, 2, anc[0], anc[1], anv[2], gc[0], gc[1], gv[2]);
-            Bf[0] = gather_box(fb, 3, anc[0], anv[1], anv[2], gc[0], gv[1], gv[2]);
-            Bf[1] = gather_box(fb, 4, anv[0], anc[1], anv[2], gv[0], gc[1], gv[2]);
-            Bf[2] = gather_box(fb, 5, anv[0], anv[1], anc[2], gv[0], gv[1], gc[2]);
+            {
+                CicAxis gc[3], gv[3];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    gc[a].w0 = fmaf(-dc[a], grid.isp[a], 1.0f);
+                    gc[a].w1 = dc[a] * grid.isp[a];
+                    gv[a].w0 = fmaf(-dv[a], grid.isp[a], 1.0f);
+                    gv[a].w1 = dv[a] * grid.isp[a];
+                }
+                const int lx = up[0] ? 0 : kB * kB, ly = up[1] ? 0 : kB, lz = up[2] ? 0 : 1;   // vertex node below
+                E[0] = gather_at<kB>(fbox + at - lx, gv[0], gc[1], gc[2]);
+                E[1] = gather_at<kB>(fbox + kB3 + at - ly, gc[0], gv[1], gc[2]);
+                E[2] = gather_at<kB>(fbox + 2 * kB3 + at - lz, gc[0], gc[1], gv[2]);
+                Bf[0] = gather_at<kB>(fbox + 3 * kB3 + at - ly - lz, gc[0], gv[1], gv[2]);
+                Bf[1] = gather_at<kB>(fbox + 4 * kB3 + at - lx - lz, gv[0], gc[1], gv[2]);
+                Bf[2] = gather_at<kB>(fbox + 5 * kB3 + at - lx - ly, gv[0], gv[1], gc[2]);
+            }
             // ---- push (boris.py:14-124), masked by update_u (particle_push.py:134-142)
             float nv[3] = {v[0], v[1], v[2]};
             push_velocity(nv, E, Bf, k.h, d);
 #pragma unroll
             for (int a = 0; a < 3; ++a)
-                if ((k.uu >> a) & 1u) v[a] = nv[a];
-            // ---- new position (Esirkepov.py:125-127, FP64) and regular-case test: the
-            // new position stays in the old cell, away from its faces by more than the
-            // FP64 rounding of floor((x - origin)/spacing).  The test runs on the FP32
-            // offset (x - node) + v dt with a band twice as wide (ExactGrid::band_*),
-            // which implies the FP64 one; a particle inside the extra band width takes
-            // the crossing queue, which treats a stay in the cell like any other step
-            double xn[3];
-            bool regular = true, short_step = true;
-            float S0[3][2], D[3];
+                if (kAll || ((k.uu >> a) & 1u)) v[a] = nv[a];
+            // ---- regular case: the new position stays in the old cell, away from its
+            // faces by more than the FP64 rounding of floor((x - origin)/spacing).
+            // The FP32 offset from the cell's middle is within 2^-22 spacings of the
+            // FP64 one, the band 2^-19 wide; a particle in the band takes the queue,
+            // which treats a stay in the cell like any other step
+            bool regular = true;
+            float D[3], A[3], qn[3];
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                const bool ux = (k.ux >> a) & 1u;
-                xn[a] = ux ? step_pos((double)xf[a], (double)v[a], d.dt) : (double)xf[a];
-                const float dvt = ux ? v[a] * fdt : 0.0f;
-                const float e = dc[a] + dvt;      // a frozen axis tests its offset the same way
-                regular = regular && e >= eg.band_lo[a] && e < eg.band_hi[a] && anc[a] >= 0 && anc[a] + 1 < d.dims[a];
-                short_step = short_step && fabsf(dvt) < 0.99f * eg.sp_c[a];   // anchor moves by one node at most
-                const float r0 = dc[a] * eg.inv_d[a];
-                S0[a][0] = 1.0f - r0;
-                S0[a][1] = r0;
-                D[a] = dvt * eg.inv_d[a];
-            }
-            if (!regular) {
-                // face crossing: the new anchor by bracketing the FP64 new position
-                // between the exact nodes next to the old cell (outside the face band)
-                // and a frame inside the box, else the rare list; the crossing pass
-                // rebuilds the frame from (step, ro, f, old anchor)
-                bool ok = short_step;
-                int packed = 0;
-                float fro[3], ff[3];
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    const float hi32 = nodec[a] + eg.sp_c[a];
-                    const int st = xn[a] < (double)nodec[a] ? -1 : (xn[a] >= (double)hi32 ? 1 : 0);
-                    const float noden = st == 0 ? nodec[a] : (st < 0 ? nodec[a] - eg.sp_c[a] : hi32);
-                    ok = ok && xn[a] >= (double)noden + eg.tol[a] &&
-                         xn[a] < (double)(noden + eg.sp_c[a]) - eg.tol[a];
-                    const int rel = anc[a] - o[a];
-                    ok = ok && (unsigned)(rel + (st < 0 ? -1 : 0)) <= (unsigned)(kB - 3);
-                    fro[a] = dc[a] * eg.inv_d[a];
-                    ff[a] = st == 0 ? D[a] : (float)(xn[a] - (double)noden) * eg.inv_d[a];
-                    packed |= ((st + 1) << (10 + 2 * a)) | ((rel & 31) << (16 + 5 * a));
-                }
-                const int slot = ok ? atomicAdd(&sh.q_n, 1) : kCrossCap;
-                if (slot >= kCrossCap) {
-                    rare_push(rare, i);
-                    break;
-                }
-                sh.q_idx[slot] = packed;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    sh.q_f[a][slot] = fro[a];
-                    sh.q_f[3 + a][slot] = ff[a];
-                }
+                const float dvt = kAll || ((k.ux >> a) & 1u) ? v[a] * grid.dt32 : 0.0f;
+                qn[a] = qm[a] + dvt;
+                regular = regular & (fabsf(qn[a]) < grid.lim[a]);
+                D[a] = dvt * grid.inv_d[a];
+                A[a] = fmaf(0.5f, D[a], dc[a] * grid.inv_d[a]);      // upper weight S0 + d/2
             }
             if (regular) {
                 // difference-form Esirkepov weights of a particle that stays in its
                 // cell (Esirkepov.py:158-214): for component c over the other axes p, q,
                 // W = D_c (S0p S0q + (S0p dq + dp S0q)/2 + dp dq/3) with d = -D, +D at
                 // slots 0, 1, i.e. W = D_c (Ap Aq + dp dq/12) with A = S0 + d/2;
-                // J_c = -(q/(d_p d_q dt)) W at slot a only
-                float A[3][2];
+                // J_c = -(q/(d_p d_q dt)) W at slot a only.  The lower weight is 1 - A,
+                // so the four nodes are linear in the four moments below
+                if (at != cell) {
+                    if (cell >= 0) flush_moments<kB>(box + cell, acc);
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    A[a][1] = S0[a][1] + 0.5f * D[a];
-                    A[a][0] = S0[a][0] - 0.5f * D[a];
+                    for (int m = 0; m < 12; ++m) acc[m] = 0.0f;
+                    cell = at;
                 }
-                float val[12];
 #pragma unroll
                 for (int c = 0; c < 3; ++c) {
                     const int o1 = c == 0 ? 1 : 0, o2 = c == 2 ? 1 : 2;
-                    const float pre = k.pre[c] * (-D[c]);
-                    const float e = D[o1] * D[o2] * (1.0f / 12.0f);
-                    val[c * 4 + 0] = pre * fmaf(A[o1][0], A[o2][0], e);
-                    val[c * 4 + 1] = pre * fmaf(A[o1][0], A[o2][1], -e);
-                    val[c * 4 + 2] = pre * fmaf(A[o1][1], A[o2][0], -e);
-                    val[c * 4 + 3] = pre * fmaf(A[o1][1], A[o2][1], e);
+                    const float pc = k.pre[c] * (-D[c]);
+                    const float y = fmaf(A[o1], A[o2], D[o1] * (D[o2] * (1.0f / 12.0f)));
+                    acc[4 * c] += pc;
+                    acc[4 * c + 1] = fmaf(pc, A[o1], acc[4 * c + 1]);
+                    acc[4 * c + 2] = fmaf(pc, A[o2], acc[4 * c + 2]);
+                    acc[4 * c + 3] = fmaf(pc, y, acc[4 * c + 3]);
                 }
-                const bool same = have && anc[0] == h0 && anc[1] == h1 && anc[2] == h2;
-                if (have && !same) flush_cell<kB>(d, sink, h0, h1, h2, acc);
+            } else {
+                // queued only if the frame of the pass lies in the box and the anchor
+                // moves by at most one, so that how many particles are rare does not
+                // depend on the order in which the queue fills (within the band of a
+                // face the pass has the last word)
+                bool near = true;
 #pragma unroll
-                for (int m = 0; m < 12; ++m) acc[m] = (same ? acc[m] : 0.0f) + val[m];
-                h0 = anc[0];
-                h1 = anc[1];
-                h2 = anc[2];
-                have = true;
+                for (int a = 0; a < 3; ++a) {
+                    const float low = f[a] - (qn[a] < 0.0f ? 1.0f : 0.0f);
+                    near = near & (low >= 0.0f) & (low <= kB - 3.0f) & (fabsf(D[a]) < 0.99f);
+                }
+                const int slot = near ? atomicAdd(&sh.n, 1) : kCrossCap;
+                if (slot >= kCrossCap) {
+                    rare_push(rare, s0 + j);
+                    break;
+                }
+                sh.slot[slot] = (int)(s0 - base) + j;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) sh.v[a][slot] = v[a];
             }
             // ---- position update + particle boundaries (particle_tile_communication.py)
             bool act = true;
+            double xn[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                xn[a] = kAll || ((k.ux >> a) & 1u) ? step_pos((double)xf[a], (double)v[a], d.dt) : (double)xf[a];
             if (!interior) {
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    if (d.pbc[a] == 0) periodic_wrap(d.wind[a], xn[a]);
-                    else apply_axis_boundary(d.pbc[a], d.wind[a], xn[a], v[a], act);
+                    // the asm keeps the remainder's loop-invariant half (a dozen vector
+                    // registers) from being hoisted into every block
+                    double wind = d.wind[a];
+                    asm volatile("" : "+s"(wind));
+                    if (d.pbc[a] == 0) periodic_wrap(wind, xn[a]);
+                    else apply_axis_boundary(d.pbc[a], wind, xn[a], v[a], act);
                 }
             }
 #pragma unroll
@@ -603,8 +557,7 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void fused_tile_exact_kernel(
                 store_vec<kP>(out.x[a] + s0, PX[a]);
                 store_vec<kP>(out.u[a] + s0, PU[a]);
             }
-            if constexpr (kP == 4) *reinterpret_cast<uint32_t*>(out.active + s0) = oact;
-            else *reinterpret_cast<uint16_t*>(out.active + s0) = (uint16_t)oact;
+            *reinterpret_cast<uint32_t*>(out.active + s0) = oact;
         } else {
 #pragma unroll
             for (int j = 0; j < kP; ++j) {
@@ -618,32 +571,35 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void fused_tile_exact_kernel(
                 out.active[i] = (uint8_t)((oact >> (8 * j)) & 0xffu);
             }
         }
-        }   // slot groups
-        {
-            // the thread's last cell: equal cells of neighbouring lanes are summed
-            // first, so one lane per cell and 16-lane row adds into the box (a
-            // cell outside the box keeps a key of its own)
-            const int bi = h0 - o[0], bj = h1 - o[1], bk = h2 - o[2];
-            const bool inbox = (unsigned)bi < (unsigned)(kB - 1) && (unsigned)bj < (unsigned)(kB - 1) &&
-                               (unsigned)bk < (unsigned)(kB - 1);
-            const int key = !have ? -1 : (inbox ? (bi * kB + bj) * kB + bk : -2 - (int)(threadIdx.x & 63u));
-            if (row_run_sums(key, acc) && have) flush_cell<kB>(d, sink, h0, h1, h2, acc);
-        }
+        // the thread's last cell: equal cells of four neighbouring lanes are summed
+        // first (over sixteen the two further steps cost more than the adds saved)
+        if (row_run_sums<4>(cell, acc) && cell >= 0) flush_moments<kB>(box + cell, acc);
         __syncthreads();
-        // ---- queued face crossings (3-slot frame, Esirkepov.py:105-331)
-        const int nq = min(sh.q_n, kCrossCap);
+        // ---- queued particles (3-slot frame, Esirkepov.py:105-331)
+        const int nq = min(sh.n, kCrossCap);
         for (int q = threadIdx.x; q < nq; q += kThreads) {
-            const int e = sh.q_idx[q];
+            const int64_t i = base + sh.slot[q], src = kGather ? (int64_t)gather[i] : i;
             CrossAxis ca[3];
+            bool ok = true;
 #pragma unroll
-            for (int a = 0; a < 3; ++a)
-                cross_frame((e >> (16 + 5 * a)) & 31, ((e >> (10 + 2 * a)) & 3) - 1, sh.q_f[a][q], sh.q_f[3 + a][q],
-                            ca[a]);
-            crossing_deposit_box<kB>(k, ca[0], ca[1], ca[2], box);
+            for (int a = 0; a < 3; ++a) {
+                const double xo = (double)in.x[a][src];
+                const double xn = kAll || ((k.ux >> a) & 1u) ? step_pos(xo, (double)sh.v[a][q], d.dt) : xo;
+                ok = cross_axis(xo, xn, grid.org64[a], grid.sp64[a], grid.inv_d64[a], grid.org32[a], grid.isp[a], ca[a]) && ok;
+                ok = ok && (unsigned)(ca[a].b - fo[a]) <= (unsigned)(kB - 3);
+            }
+            if (!ok) {
+                rare_push(rare, i);
+                continue;
+            }
+            Sum* p = box + ((ca[0].b - fo[0]) * kB + ca[1].b - fo[1]) * kB + ca[2].b - fo[2];
+            crossing_component_box<0, kB>(k.pre[0], ca[0], ca[1], ca[2], p);
+            crossing_component_box<1, kB>(k.pre[1], ca[1], ca[0], ca[2], p);
+            crossing_component_box<2, kB>(k.pre[2], ca[2], ca[0], ca[1], p);
         }
         __syncthreads();
     }
-    flush_current_box<kB>(d, o, box, Jx, Jy, Jz);
+    flush_current_box<kB>(d, fo, box, Jx, Jy, Jz);
 }
 
 // The rare list of fused_tile_exact_kernel: each listed particle runs the
@@ -1174,11 +1130,51 @@ int pic_tile_exact_grid(const PicDesc* desc) {
     return desc && desc_ok(desc) && make_exact_grid(*desc, eg) ? 1 : 0;
 }
 
+// The tile kernel has one launch shape: rounds and min_blocks are those of the
+// strided kernel.
+static void launch_tile_esirkepov(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                  const FieldPtrs& fp, const PicParticles* out, float* const J[3],
+                                  const int32_t* starts, const TileGeom& tg, const TileGrid& grid, bool exact,
+                                  int32_t* workspace, const int32_t* gather, int64_t blocks,
+                                  hipStream_t st) {
+    // vector loads and stores of a thread's slot group need 16-byte aligned planes
+    int vec_ok = 1;
+    for (int a = 0; a < 3; ++a)
+        vec_ok &= ((((uintptr_t)out->x[a]) | ((uintptr_t)out->u[a]) | ((uintptr_t)in->x[a]) |
+                    ((uintptr_t)in->u[a])) & 15u) == 0;
+    vec_ok &= ((((uintptr_t)out->active) | ((uintptr_t)in->active)) & 3u) == 0;
+    vec_ok &= (((uintptr_t)gather) & 15u) == 0;
+    hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, st, workspace);
+    const SpeciesTable stab = species_table(*desc, *sp);
+    bool all = true;
+    for (int s = 0; s < sp->count; ++s) all = all && stab.k[s].ux == 7u && stab.k[s].uu == 7u;
+#define PIC_EXACT_LAUNCH(T, GA, EX, ALL)                                                                        \
+    hipLaunchKernelGGL((fused_tile_exact_kernel<T, GA, EX, ALL>), dim3((unsigned)blocks), dim3(kThreads), 0, st, \
+                       *desc, *in, fp, *out, J[0], J[1], J[2], starts, tg, grid, workspace, vec_ok, stab, gather)
+#define PIC_EXACT_ALL(T, GA, EX)                          \
+    do {                                                     \
+        if (all) PIC_EXACT_LAUNCH(T, GA, EX, true);       \
+        else PIC_EXACT_LAUNCH(T, GA, EX, false);          \
+    } while (0)
+    // a gathered launch is only made on exact grids
+#define PIC_EXACT_SHAPE(T)                                \
+    do {                                                     \
+        if (!exact) PIC_EXACT_ALL(T, false, false);       \
+        else if (gather) PIC_EXACT_ALL(T, true, true);    \
+        else PIC_EXACT_ALL(T, false, true);               \
+    } while (0)
+    if (tg.T == 8) PIC_EXACT_SHAPE(8);
+    else PIC_EXACT_SHAPE(4);
+#undef PIC_EXACT_SHAPE
+#undef PIC_EXACT_ALL
+#undef PIC_EXACT_LAUNCH
+}
+
 static int fused_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
                                  const float* const E[3], const float* const B[3], const float* const E_ext[3],
                                  const float* const B_ext[3], PicParticles* out, float* const J[3], int32_t tile,
                                  const int32_t* starts, int32_t rounds, int32_t min_blocks, int32_t* workspace,
-                                 const int32_t* gather, void* stream) {
+                                 const int32_t* gather, bool general, void* stream) {
     PIC_REQUIRE(desc_ok(desc) && particles_ok(sp, in) && particles_ok(sp, out) && E && B && J && starts);
     PIC_REQUIRE(fused_kind(*desc) == 3 && (tile == 4 || tile == 8) &&
                 (rounds == 2 || rounds == 4 || rounds == 8));
@@ -1209,46 +1205,11 @@ static int fused_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, cons
         else PIC_TILED_LAUNCH(R, T, 1);                 \
     } while (0)
     ExactGrid eg;
-    if (desc->variant != 1 && make_exact_grid(*desc, eg)) {
+    TileGrid grid;
+    const bool exact = desc->variant != 1 && make_exact_grid(*desc, eg);
+    if ((exact || general) && make_tile_grid(*desc, grid)) {
         PIC_REQUIRE(workspace);
-        // vector loads and stores of a thread's slot group need 16-byte aligned planes
-        int vec_ok = 1;
-        for (int a = 0; a < 3; ++a)
-            vec_ok &= ((((uintptr_t)out->x[a]) | ((uintptr_t)out->u[a]) | ((uintptr_t)in->x[a]) |
-                        ((uintptr_t)in->u[a])) & 15u) == 0;
-        vec_ok &= ((((uintptr_t)out->active) | ((uintptr_t)in->active)) & 3u) == 0;
-        vec_ok &= (((uintptr_t)gather) & 15u) == 0;
-        hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, st, workspace);
-        const SpeciesTable stab = species_table(*desc, *sp);
-#define PIC_EXACT_LAUNCH(T, P, MB, G)                                                                               \
-        do {                                                                                                        \
-            if (gather)                                                                                             \
-                hipLaunchKernelGGL((fused_tile_exact_kernel<T, P, MB, G, true>), dim3((unsigned)blocks),            \
-                                   dim3(kThreads), 0, st, *desc, *sp, *in, fp, *out, J[0], J[1], J[2], starts, tg,  \
-                                   eg, workspace, vec_ok, stab, gather);                                            \
-            else                                                                                                    \
-                hipLaunchKernelGGL((fused_tile_exact_kernel<T, P, MB, G, false>), dim3((unsigned)blocks),           \
-                                   dim3(kThreads), 0, st, *desc, *sp, *in, fp, *out, J[0], J[1], J[2], starts, tg,  \
-                                   eg, workspace, vec_ok, stab, gather);                                            \
-        } while (0)
-#define PIC_EXACT_MB(T, P, G)                                  \
-        do {                                                   \
-            if (min_blocks == 3) PIC_EXACT_LAUNCH(T, P, 3, G); \
-            else if (min_blocks == 4) PIC_EXACT_LAUNCH(T, P, 4, G); \
-            else PIC_EXACT_LAUNCH(T, P, 1, G);                 \
-        } while (0)
-        // rounds: slots per thread (8: two groups of four)
-        if (tile == 8) {
-            if (rounds == 2) PIC_EXACT_MB(8, 2, 1);
-            else if (rounds == 4) PIC_EXACT_MB(8, 4, 1);
-            else PIC_EXACT_MB(8, 4, 2);
-        } else {
-            if (rounds == 2) PIC_EXACT_MB(4, 2, 1);
-            else if (rounds == 4) PIC_EXACT_MB(4, 4, 1);
-            else PIC_EXACT_MB(4, 4, 2);
-        }
-#undef PIC_EXACT_MB
-#undef PIC_EXACT_LAUNCH
+        launch_tile_esirkepov(desc, sp, in, fp, out, J, starts, tg, grid, exact, workspace, gather, blocks, st);
         const int64_t rare_grid = std::min<int64_t>(std::max<int64_t>(grid_1d(n, kThreads), 1), 1024);
         hipLaunchKernelGGL(fused_tile_rare_kernel, dim3((unsigned)rare_grid), dim3(kThreads), 0, st, *desc, *sp, *in,
                            fp, *out, J[0], J[1], J[2], workspace, gather);
@@ -1271,7 +1232,16 @@ int pic_fused_push_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, co
                                    const int32_t* starts, int32_t rounds, int32_t min_blocks, int32_t* workspace,
                                    void* stream) {
     return fused_esirkepov_tiled(desc, sp, in, E, B, E_ext, B_ext, out, J, tile, starts, rounds, min_blocks,
-                                 workspace, nullptr, stream);
+                                 workspace, nullptr, false, stream);
+}
+
+int pic_fused_push_esirkepov_tiled_general(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                           const float* const E[3], const float* const B[3],
+                                           const float* const E_ext[3], const float* const B_ext[3],
+                                           PicParticles* out, float* const J[3], int32_t tile, const int32_t* starts,
+                                           int32_t rounds, int32_t* workspace, void* stream) {
+    return fused_esirkepov_tiled(desc, sp, in, E, B, E_ext, B_ext, out, J, tile, starts, rounds, 4, workspace, nullptr,
+                                 true, stream);
 }
 
 int pic_fused_push_esirkepov_tiled_gather(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
@@ -1283,7 +1253,7 @@ int pic_fused_push_esirkepov_tiled_gather(const PicDesc* desc, const PicSpecies*
     PIC_REQUIRE(desc && desc_ok(desc) && sp && desc->variant != 1 && make_exact_grid(*desc, eg));
     PIC_REQUIRE(gather || (int64_t)sp->count * sp->slots == 0);
     return fused_esirkepov_tiled(desc, sp, in, E, B, E_ext, B_ext, out, J, tile, starts, rounds, min_blocks,
-                                 workspace, gather, stream);
+                                 workspace, gather, false, stream);
 }
 
 }  // extern "C"

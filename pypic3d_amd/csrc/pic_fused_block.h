@@ -109,8 +109,20 @@ __device__ inline void cic_axis(float x, float org32, float isp32, double org, d
     float r = (float)dl * isp32;
     s.p0 = pmod(a, L);
     s.p1 = pmod(a + 1, L);
-    s.w0 = 1.0f - r;
+    s.w0 = fmaf(-(float)dl, isp32, 1.0f);
     s.w1 = r;
+}
+
+// Both products rounded in one stated way.  Left to contraction, which of two
+// products is fused differs between kernels that inline the same source; with
+// the fused operations written out every kernel gives a particle the same field.
+__device__ inline float mix(float w0, float a, float w1, float b) { return fmaf(w1, b, w0 * a); }
+
+__device__ inline float cic_value(float v000, float v001, float v010, float v011, float v100, float v101, float v110,
+                                  float v111, const CicAxis& ax, const CicAxis& ay, const CicAxis& az) {
+    const float c00 = mix(az.w0, v000, az.w1, v001), c01 = mix(az.w0, v010, az.w1, v011);
+    const float c10 = mix(az.w0, v100, az.w1, v101), c11 = mix(az.w0, v110, az.w1, v111);
+    return mix(ax.w0, mix(ay.w0, c00, ay.w1, c01), ax.w1, mix(ay.w0, c10, ay.w1, c11));
 }
 
 __device__ inline float gather_cic(const float* __restrict__ f, const float* __restrict__ fe, const PicDesc& d,
@@ -132,9 +144,7 @@ __device__ inline float gather_cic(const float* __restrict__ f, const float* __r
         v110 += fe[r11 + z0];
         v111 += fe[r11 + z1];
     }
-    float c00 = v000 * az.w0 + v001 * az.w1, c01 = v010 * az.w0 + v011 * az.w1;
-    float c10 = v100 * az.w0 + v101 * az.w1, c11 = v110 * az.w0 + v111 * az.w1;
-    return ax.w0 * (ay.w0 * c00 + ay.w1 * c01) + ax.w1 * (ay.w0 * c10 + ay.w1 * c11);
+    return cic_value(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
 }
 
 // Gather stencil of one axis and node line with kN = 2 (first order: points a,
@@ -162,11 +172,10 @@ __device__ inline void point_axis(float x, double org, double sp, int L, int g, 
     const int a = anchor_fast(x, (float)org, isp32, org, sp, kShape);
     const double dl = (double)x - node_coord(a, sp, org);
     if constexpr (kShape == 1) {
-        const float r = (float)dl * isp32;
         s.p[0] = pmod(a, L);
         s.p[1] = pmod(a + 1, L);
-        s.w[0] = 1.0f - r;
-        s.w[1] = r;
+        s.w[0] = fmaf(-(float)dl, isp32, 1.0f);
+        s.w[1] = (float)dl * isp32;
     } else {
         double w[3];
         shape3(dl * (1.0 / sp), 2, w);
@@ -182,7 +191,7 @@ __device__ inline void point_axis(float x, double org, double sp, int L, int g, 
 // first-order kernels then agree).
 template <int kN>
 __device__ inline float weighted(const float (&v)[kN], const float (&w)[kN]) {
-    if constexpr (kN == 2) return v[0] * w[0] + v[1] * w[1];
+    if constexpr (kN == 2) return mix(w[0], v[0], w[1], v[1]);
     else return v[0] * w[0] + v[1] * w[1] + v[2] * w[2];
 }
 
@@ -506,15 +515,21 @@ struct FieldBox {
     int B;
 };
 
+// Value of a component whose box of kB^3 nodes is at p, the stencil's first node.
+template <int kB>
+__device__ inline float gather_at(const float* p, const CicAxis& ax, const CicAxis& ay, const CicAxis& az) {
+    const float v000 = p[0], v001 = p[1], v010 = p[kB], v011 = p[kB + 1];
+    const float v100 = p[kB * kB], v101 = p[kB * kB + 1], v110 = p[kB * kB + kB], v111 = p[kB * kB + kB + 1];
+    return cic_value(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
+}
+
 __device__ inline float gather_box(const FieldBox& fb, int c, int a0, int a1, int a2, const CicAxis& ax,
                                    const CicAxis& ay, const CicAxis& az) {
     const int B = fb.B;
     const float* p = fb.box + c * B * B * B + ((a0 - fb.o[0]) * B + (a1 - fb.o[1])) * B + (a2 - fb.o[2]);
     const float v000 = p[0], v001 = p[1], v010 = p[B], v011 = p[B + 1];
     const float v100 = p[B * B], v101 = p[B * B + 1], v110 = p[B * B + B], v111 = p[B * B + B + 1];
-    float c00 = v000 * az.w0 + v001 * az.w1, c01 = v010 * az.w0 + v011 * az.w1;
-    float c10 = v100 * az.w0 + v101 * az.w1, c11 = v110 * az.w0 + v111 * az.w1;
-    return ax.w0 * (ay.w0 * c00 + ay.w1 * c01) + ax.w1 * (ay.w0 * c10 + ay.w1 * c11);
+    return cic_value(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
 }
 
 // Per-block LDS: the face-crossing queue and the species constants.
@@ -997,18 +1012,23 @@ __device__ inline void fill_field_box(const PicDesc& d, const FieldPtrs& fp, con
         const int k = pmod(fo[2] + r % kFB, d.dims[2]);
         off[q] = (int)fidx(d, i, j, k);
     }
+    // all loads of the arrays before any external field: one round trip, not one per component
+    float v[6][kQ];
 #pragma unroll
     for (int c = 0; c < 6; ++c) {
         const float* F = c < 3 ? fp.E[c] : fp.B[c - 3];
+#pragma unroll
+        for (int q = 0; q < kQ; ++q) v[c][q] = F[off[q]];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) {
         const float* Fe = c < 3 ? fp.Ee[c] : fp.Be[c - 3];
 #pragma unroll
         for (int q = 0; q < kQ; ++q) {
             const int r = (int)threadIdx.x + q * kThreads;
-            if (kFV % kThreads == 0 || r < kFV) {
-                float v = F[off[q]];
-                if (Fe) v += Fe[off[q]];
-                fbox[c * kFV + r] = v;
-            }
+            if (Fe) v[c][q] += Fe[off[q]];
+            if (kFV % kThreads == 0 || r < kFV) fbox[c * kFV + r] = v[c][q];
         }
     }
 }
@@ -1017,8 +1037,8 @@ __device__ inline void fill_field_box(const PicDesc& d, const FieldPtrs& fp, con
 // per component from array index o) into J, dropping indices past the array
 // end and wrapping negative ones once (deposit_at); node offsets computed
 // once per thread.
-template <int kB, int kC = 3>
-__device__ inline void flush_current_box(const PicDesc& d, const int o[3], const float* box, float* Jx, float* Jy,
+template <int kB, int kC = 3, class T>
+__device__ inline void flush_current_box(const PicDesc& d, const int o[3], const T* box, float* Jx, float* Jy,
                                          float* Jz) {
     constexpr int kB3 = kB * kB * kB;
     constexpr int kQ = (kB3 + kThreads - 1) / kThreads;
@@ -1038,7 +1058,7 @@ __device__ inline void flush_current_box(const PicDesc& d, const int o[3], const
         for (int q = 0; q < kQ; ++q) {
             const int r = (int)threadIdx.x + q * kThreads;
             if (off[q] < 0) continue;
-            const float v = box[c * kB3 + r];
+            const float v = (float)box[c * kB3 + r];
             if (v != 0.0f) atomic_add_f32(J[c] + off[q], v);
         }
     }

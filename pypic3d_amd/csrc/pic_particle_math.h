@@ -129,10 +129,18 @@ __device__ inline void gather_EB(const PicDesc& d, const FieldPtrs& fp, const do
 // pushers (boris.py:14-124)
 // ------------------------------------------------------------------------
 
+// The fused operations of the pushers are written out: which product of a sum
+// the compiler fuses by itself differs between kernels that inline the same
+// source, and particles pushed by two kernels have to agree bit for bit.
 __device__ inline void cross(const float a[3], const float b[3], float o[3]) {
-    o[0] = a[1] * b[2] - a[2] * b[1];
-    o[1] = a[2] * b[0] - a[0] * b[2];
-    o[2] = a[0] * b[1] - a[1] * b[0];
+    o[0] = fmaf(a[1], b[2], -(a[2] * b[1]));
+    o[1] = fmaf(a[2], b[0], -(a[0] * b[2]));
+    o[2] = fmaf(a[0], b[1], -(a[1] * b[0]));
+}
+
+// c + a . a
+__device__ inline float plus_square(float c, const float a[3]) {
+    return fmaf(a[2], a[2], fmaf(a[1], a[1], fmaf(a[0], a[0], c)));
 }
 
 // Boris rotation with hardware reciprocal / reciprocal-square-root (1 ulp),
@@ -144,26 +152,25 @@ __device__ inline void boris_push(float v[3], const float E[3], const float B[3]
     float um[3], t[3], up[3], s[3], c1[3];
     const float invC2 = __builtin_amdgcn_rcpf(C * C);
     if (relativistic) {
-        float v2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-        float gamma = __builtin_amdgcn_rsqf(1.0f - v2 * invC2);
-        for (int a = 0; a < 3; ++a) um[a] = v[a] * gamma + h * E[a];
-        float igm = __builtin_amdgcn_rsqf(1.0f + (um[0] * um[0] + um[1] * um[1] + um[2] * um[2]) * invC2);
+        float gamma = __builtin_amdgcn_rsqf(fmaf(-plus_square(0.0f, v), invC2, 1.0f));
+        for (int a = 0; a < 3; ++a) um[a] = fmaf(h, E[a], v[a] * gamma);
+        float igm = __builtin_amdgcn_rsqf(fmaf(plus_square(0.0f, um), invC2, 1.0f));
         for (int a = 0; a < 3; ++a) t[a] = h * B[a] * igm;
     } else {
         for (int a = 0; a < 3; ++a) {
-            um[a] = v[a] + h * E[a];
+            um[a] = fmaf(h, E[a], v[a]);
             t[a] = h * B[a];
         }
     }
     cross(um, t, c1);
     for (int a = 0; a < 3; ++a) up[a] = um[a] + c1[a];
-    float f = 2.0f * __builtin_amdgcn_rcpf(1.0f + t[0] * t[0] + t[1] * t[1] + t[2] * t[2]);
+    float f = 2.0f * __builtin_amdgcn_rcpf(plus_square(1.0f, t));
     for (int a = 0; a < 3; ++a) s[a] = t[a] * f;
     cross(up, s, c1);
     float nu[3];
-    for (int a = 0; a < 3; ++a) nu[a] = um[a] + c1[a] + h * E[a];
+    for (int a = 0; a < 3; ++a) nu[a] = fmaf(h, E[a], um[a] + c1[a]);
     if (relativistic) {
-        float ing = __builtin_amdgcn_rsqf(1.0f + (nu[0] * nu[0] + nu[1] * nu[1] + nu[2] * nu[2]) * invC2);
+        float ing = __builtin_amdgcn_rsqf(fmaf(plus_square(0.0f, nu), invC2, 1.0f));
         for (int a = 0; a < 3; ++a) v[a] = nu[a] * ing;
     } else {
         for (int a = 0; a < 3; ++a) v[a] = nu[a];

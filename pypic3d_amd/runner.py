@@ -94,7 +94,7 @@ class ElectrodynamicRunner:
         self.direct_min_blocks = 1
         self.sort_lookahead = None      # tile re-sort keys at x + t u; None: t = sort_every * dt / 2
         self.tile_ws, self.direct_fused = None, False
-        self.defer_permute = False
+        self.defer_permute = self.tile_general = False
         if tile is not None:
             self.set_tile(tile)
 
@@ -155,6 +155,10 @@ class ElectrodynamicRunner:
                        N.p3(self.B), self.Ee, self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts),
                        self.rounds, self.min_blocks, N.ptr(self.tile_ws), s)
                 self._pending = False
+            elif self.tile and self.tile_general and d.variant != 1:
+                N.call("pic_fused_push_esirkepov_tiled_general", d, self.sp, self._pp(src), N.p3(E), N.p3(self.B),
+                       self.Ee, self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts), self.rounds,
+                       N.ptr(self.tile_ws), s)
             elif self.tile:
                 N.call("pic_fused_push_esirkepov_tiled", d, self.sp, self._pp(src), N.p3(E), N.p3(self.B), self.Ee,
                        self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts), self.rounds,
@@ -271,6 +275,8 @@ class ElectrodynamicRunner:
         # the particles through perm (both branches' fused kernels on exact grids)
         self.defer_permute = self.direct_fused or (self.esirkepov and d.variant != 1
                                                    and bool(N.lib().pic_tile_exact_grid(d)))
+        # other grids take the same kernel with FP64 anchors, which reads its slots directly
+        self.tile_general = self.esirkepov and not bool(N.lib().pic_tile_exact_grid(d))
         tiles = int(N.lib().pic_tile_count(d, self.tile))
         self.starts = torch.empty(self.S * (tiles + 1) + 1, dtype=torch.int32, device=self.device)
         # the tiled kernel's list of particles for its general route (1 + slots int32)
