@@ -238,15 +238,23 @@ int pic_fused_push_esirkepov_tiled_gather(const PicDesc* desc, const PicSpecies*
  * pic_deposit_direct, pic_advance_positions, pic_particle_boundaries up to
  * FP32 rounding (an ulp in a velocity where the compiler fuses the push's
  * multiply-adds differently) and summation order in J.  tile 4 or 8;
- * min_blocks 1 (each thread's four slots loaded and stored with 16-byte
- * accesses) or 4 (tile 4: two slots per thread with 8-byte accesses, which
- * fits 128 VGPRs for 4 resident blocks per CU, about 15 % faster at 256^3 x
- * 32 ppc; tile 8: slots stored one by one); workspace as for
+ * min_blocks 1 or 4 (both take the kernel's one launch shape, four slots per
+ * thread with 16-byte accesses); workspace as for
  * pic_fused_push_esirkepov_tiled. */
 int pic_fused_push_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
                                 const float* const E[3], const float* const B[3], const float* const E_ext[3],
                                 const float* const B_ext[3], PicParticles* out, float* const J[3], int32_t tile,
                                 const int32_t* starts, int32_t min_blocks, int32_t* workspace, void* stream);
+/* pic_fused_push_direct_tiled on any 3-D first-order grid: FP64 anchors where
+ * the lines are not FP32-exact or cell size and node spacing differ.  Needs a
+ * grid pic_tile_general_grid accepts (3-D, first order, vertex line half a
+ * spacing above the centre line); -1 otherwise. */
+int pic_tile_general_grid(const PicDesc* desc);
+int pic_fused_push_direct_tiled_general(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                        const float* const E[3], const float* const B[3],
+                                        const float* const E_ext[3], const float* const B_ext[3],
+                                        PicParticles* out, float* const J[3], int32_t tile, const int32_t* starts,
+                                        int32_t* workspace, void* stream);
 /* pic_fused_push_direct_tiled reading slot i of the sorted order from in's
  * slot gather[i] (the perm of a pic_tile_rebin called with out == NULL), as
  * pic_fused_push_esirkepov_tiled_gather does for the Esirkepov branch:

@@ -386,23 +386,13 @@ __device__ inline bool line_points(float x, double org, double sp, int o, int e,
     }
 }
 
-template <int kN>
+template <int kN, CicRounding kR>
 __device__ inline float box_value(const float* p, int plane, int row, const float (&wx)[kN], const float (&wy)[kN],
                                   const float (&wz)[kN]) {
-    float sx[kN];
+    return stencil_sum<kN, kR>(wx, wy, wz, [&](int i, int j, float (&v)[kN]) {
 #pragma unroll
-    for (int i = 0; i < kN; ++i) {
-        float sy[kN];
-#pragma unroll
-        for (int j = 0; j < kN; ++j) {
-            float v[kN];
-#pragma unroll
-            for (int k = 0; k < kN; ++k) v[k] = p[i * plane + j * row + k];
-            sy[j] = weighted<kN>(v, wz);
-        }
-        sx[i] = weighted<kN>(wy, sy);
-    }
-    return weighted<kN>(wx, sx);
+        for (int k = 0; k < kN; ++k) v[k] = p[i * plane + j * row + k];
+    });
 }
 
 // One block per work item: E + E_ext and B + B_ext of the tile's box in LDS
@@ -449,9 +439,11 @@ __global__ __launch_bounds__(kWide) void bin_tile_push_kernel(PicDesc d, BinGeom
                 const auto pick = [&](int axis, bool vertex) { return vertex ? pv[axis] : pc[axis]; };
                 const int e0 = pick(0, m == 0), e1 = pick(1, m == 1), e2 = pick(2, m == 2);
                 const int b0 = pick(0, m != 0), b1 = pick(1, m != 1), b2 = pick(2, m != 2);
-                E[m] = box_value<kN>(box + m * g.box + (e0 * g.e[1] + e1) * g.e[2] + e2, plane, g.e[2],
-                                     m == 0 ? wv[0] : wc[0], m == 1 ? wv[1] : wc[1], m == 2 ? wv[2] : wc[2]);
-                B[m] = box_value<kN>(box + (3 + m) * g.box + (b0 * g.e[1] + b1) * g.e[2] + b2, plane, g.e[2],
+                const float* pe = box + m * g.box + (e0 * g.e[1] + e1) * g.e[2] + e2;
+                E[m] = m == 1 ? box_value<kN, kSecond>(pe, plane, g.e[2], wc[0], wv[1], wc[2])
+                              : box_value<kN, kPlain>(pe, plane, g.e[2], m == 0 ? wv[0] : wc[0], wc[1],
+                                                      m == 2 ? wv[2] : wc[2]);
+                B[m] = box_value<kN, kMagnetic>(box + (3 + m) * g.box + (b0 * g.e[1] + b1) * g.e[2] + b2, plane, g.e[2],
                                      m != 0 ? wv[0] : wc[0], m != 1 ? wv[1] : wc[1], m != 2 ? wv[2] : wc[2]);
             }
         } else {

@@ -46,14 +46,6 @@ __device__ inline void exact_anchors(float x, float org, float sp, float isp, fl
     dv = upper ? x - mid : x - (mid - sp);
 }
 
-// An empty asm that reads a slot's position and velocity: placed before the
-// slot's activity test it keeps the compiler from moving these six loads below
-// the test, so they are issued with the activity load and share its memory
-// round trip instead of waiting for it.
-__device__ inline void loads_together(const float (&x)[3], const float (&u)[3]) {
-    asm volatile("" ::"v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(u[0]), "v"(u[1]), "v"(u[2]));
-}
-
 // Grid constants of the tile kernels.  Anchors are found relative to the first
 // node of the tile's field box: an FP32 estimate that is never too small
 // (isp_up or bias) and at most one too large, corrected by one comparison with
@@ -130,9 +122,10 @@ __device__ inline bool tile_anchor(const TileGrid& tg, int a, float x, float nb,
     } else {
         f = floorf(fmaf(x - nb, tg.isp[a], tg.bias[a]));
         double dd = (double)x - node_at(f + fo, tg.sp64[a], tg.org64[a]);
-        const bool below = dd < 0.0;
-        f -= below ? 1.0f : 0.0f;
-        dd += below ? tg.sp64[a] : 0.0;
+        if (dd < 0.0) {
+            f -= 1.0f;
+            dd = (double)x - node_at(f + fo, tg.sp64[a], tg.org64[a]);
+        }
         const double q64 = dd - tg.half64[a];
         dc = (float)dd;
         q = (float)q64;

@@ -243,6 +243,88 @@ __device__ inline void flush_moments(T* p, const float m[12]) {
     }
 }
 
+// A thread's group of kP consecutive slots from s0, loaded at once: one kP-wide
+// vector load per plane where the group lies inside [begin, end) and the planes
+// are aligned (`full`; the lanes of a wave then read contiguous memory, and all
+// loads share one round trip).  Slots outside the range are inactive.
+template <int kP, bool kGather>
+__device__ inline void load_group(const PicParticles& in, const int32_t* __restrict__ gather, int64_t s0,
+                                  int64_t begin, int64_t end, bool full, float (&PX)[3][kP], float (&PU)[3][kP],
+                                  uint32_t& pact) {
+    pact = 0u;
+    if (!kGather && full) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            load_vec<kP>(in.x[a] + s0, PX[a]);
+            load_vec<kP>(in.u[a] + s0, PU[a]);
+        }
+        pact = *reinterpret_cast<const uint32_t*>(in.active + s0);
+    } else if (kGather && full) {
+        // slot i's input is in.*[gather[i]]: the permutation of a re-bin,
+        // applied by this launch while it reads.  The flags are loaded
+        // first and combined only after every load has been issued (the
+        // scheduling barrier keeps the combination from being hoisted
+        // between the loads, where each use of a flag would wait for all
+        // loads issued before it)
+        float gf[kP];
+        load_vec<kP>(reinterpret_cast<const float*>(gather + s0), gf);
+        uint32_t ab[kP];
+#pragma unroll
+        for (int j = 0; j < kP; ++j) ab[j] = in.active[__float_as_int(gf[j])];
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+            const int64_t src = __float_as_int(gf[j]);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                PX[a][j] = in.x[a][src];
+                PU[a][j] = in.u[a][src];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < kP; ++j) pact |= (ab[j] != 0u ? 1u : 0u) << (8 * j);
+    } else {
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+            const int64_t i = s0 + j;
+            const bool inr = i >= begin && i < end;
+            const int64_t src = kGather ? (inr ? (int64_t)gather[i] : 0) : i;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                PX[a][j] = inr ? in.x[a][src] : 0.0f;
+                PU[a][j] = inr ? in.u[a][src] : 0.0f;
+            }
+            pact |= (inr && in.active[src] != 0 ? 1u : 0u) << (8 * j);
+        }
+    }
+}
+
+// The group's outputs, likewise.
+template <int kP>
+__device__ inline void store_group(const PicParticles& out, int64_t s0, int64_t begin, int64_t end, bool full,
+                                   const float (&PX)[3][kP], const float (&PU)[3][kP], uint32_t oact) {
+    if (full) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            store_vec<kP>(out.x[a] + s0, PX[a]);
+            store_vec<kP>(out.u[a] + s0, PU[a]);
+        }
+        *reinterpret_cast<uint32_t*>(out.active + s0) = oact;
+    } else {
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+            const int64_t i = s0 + j;
+            if (i < begin || i >= end) continue;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                out.x[a][i] = PX[a][j];
+                out.u[a][i] = PU[a][j];
+            }
+            out.active[i] = (uint8_t)((oact >> (8 * j)) & 0xffu);
+        }
+    }
+}
+
 // Particles of a chunk that do not stay in their cell: slot offset from the
 // chunk base and pushed velocity; the queue's pass reloads the old position.
 // A full queue sends further particles to the rare list.
@@ -277,9 +359,9 @@ struct CrossQueue {
 // traffic overlap them).  Summing cell moments in registers, FP64 box adds in
 // place of ds_add_f32 and a queue of (slot, velocity) took 128^3 with 2 x 16
 // particles per cell from 1963 to 1548 us (43 G particles/s, 2.2 TB/s) and
-// 256^3 with 32 from 12.1 to 9.7 ms; FP64 anchors in the same kernel take a
-// 64^3 step with 8 and 4 per cell from 1132 to 396 us.  kExact: FP32 anchors of
-// an exact grid, else FP64 ones (TileGrid).  kAll: no species has a frozen axis.
+// 256^3 with 32 from 12.1 to 9.7 ms; FP64 anchors in the same kernel take
+// 160 x 96 x 96 with 4 per cell from 1132 to 396 us.  kExact: FP32 anchors of an
+// exact grid, else FP64 ones (TileGrid).  kAll: no species has a frozen axis.
 template <int kT, bool kGather, bool kExact, bool kAll>
 __global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_exact_kernel(
     PicDesc d, PicParticles in, FieldPtrs fp, PicParticles out, float* Jx, float* Jy, float* Jz,
@@ -327,63 +409,13 @@ __global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_exact_ke
         xlo[a] = uniform(__double2float_ru(fmax(fo[a] * sp + org + 0.5 * sp, org) + margin));
         xhi[a] = uniform(__double2float_ru(min(fo[a] + kB - 1, d.dims[a] - 1) * sp + org - margin));
     }
-    // A group's kP slots are loaded at once, with one kP-wide vector load per
-    // plane when the group lies inside the range (the lanes of a wave then read
-    // contiguous memory, and all loads share one round trip).  The first group is
-    // loaded before the field box is filled, so both wait for memory together.
+    // the first group is loaded before the field box is filled: both wait for memory together
     float PX[3][kP], PU[3][kP];
     uint32_t pact;
-    const auto load_group = [&](int64_t s0, bool full) {
-        pact = 0u;
-        if (!kGather && full) {
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                load_vec<kP>(in.x[a] + s0, PX[a]);
-                load_vec<kP>(in.u[a] + s0, PU[a]);
-            }
-            pact = *reinterpret_cast<const uint32_t*>(in.active + s0);
-        } else if (kGather && full) {
-            // slot i's input is in.*[gather[i]]: the permutation of a re-bin,
-            // applied by this launch while it reads.  The flags are loaded
-            // first and combined only after every load has been issued (the
-            // scheduling barrier keeps the combination from being hoisted
-            // between the loads, where each use of a flag would wait for all
-            // loads issued before it)
-            float gf[kP];
-            load_vec<kP>(reinterpret_cast<const float*>(gather + s0), gf);
-            uint32_t ab[kP];
-#pragma unroll
-            for (int j = 0; j < kP; ++j) ab[j] = in.active[__float_as_int(gf[j])];
-#pragma unroll
-            for (int j = 0; j < kP; ++j) {
-                const int64_t src = __float_as_int(gf[j]);
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    PX[a][j] = in.x[a][src];
-                    PU[a][j] = in.u[a][src];
-                }
-            }
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < kP; ++j) pact |= (ab[j] != 0u ? 1u : 0u) << (8 * j);
-        } else {
-#pragma unroll
-            for (int j = 0; j < kP; ++j) {
-                const int64_t i = s0 + j;
-                const bool inr = i >= begin && i < end;
-                const int64_t src = kGather ? (inr ? (int64_t)gather[i] : 0) : i;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    PX[a][j] = inr ? in.x[a][src] : 0.0f;
-                    PU[a][j] = inr ? in.u[a][src] : 0.0f;
-                }
-                pact |= (inr && in.active[src] != 0 ? 1u : 0u) << (8 * j);
-            }
-        }
-    };
     const auto inside = [&](int64_t s0) { return vec_ok && s0 >= begin && s0 + kP <= end; };
     const int64_t first = begin & ~(int64_t)(kP - 1);
-    load_group(first + (int64_t)kP * (int)threadIdx.x, inside(first + (int64_t)kP * (int)threadIdx.x));
+    const int64_t g0 = first + (int64_t)kP * (int)threadIdx.x;
+    load_group<kP, kGather>(in, gather, g0, begin, end, inside(g0), PX, PU, pact);
     for (int e = threadIdx.x; e < 3 * kB3; e += kThreads) box[e] = (Sum)0;
     fill_field_box<kB>(d, fp, fo, fbox);
     const SpeciesK& k = st.k[s];
@@ -397,7 +429,7 @@ __global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_exact_ke
         int cell = -1;
         const int64_t s0 = base + (int64_t)kP * (int)threadIdx.x;
         const bool full = inside(s0);
-        if (base != first) load_group(s0, full);
+        if (base != first) load_group<kP, kGather>(in, gather, s0, begin, end, full, PX, PU, pact);
         // One particle per iteration (the loop stays rolled to bound register
         // pressure): slot j's inputs are taken from the front of PX/PU/pact,
         // which shift by one, and its outputs enter at the back, so after kP
@@ -551,26 +583,7 @@ __global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_exact_ke
             }
             oact = (oact >> 8) | (oa << (8 * (kP - 1)));
         }
-        if (full) {
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                store_vec<kP>(out.x[a] + s0, PX[a]);
-                store_vec<kP>(out.u[a] + s0, PU[a]);
-            }
-            *reinterpret_cast<uint32_t*>(out.active + s0) = oact;
-        } else {
-#pragma unroll
-            for (int j = 0; j < kP; ++j) {
-                const int64_t i = s0 + j;
-                if (i < begin || i >= end) continue;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    out.x[a][i] = PX[a][j];
-                    out.u[a][i] = PU[a][j];
-                }
-                out.active[i] = (uint8_t)((oact >> (8 * j)) & 0xffu);
-            }
-        }
+        store_group<kP>(out, s0, begin, end, full, PX, PU, oact);
         // the thread's last cell: equal cells of four neighbouring lanes are summed
         // first (over sixteen the two further steps cost more than the adds saved)
         if (row_run_sums<4>(cell, acc) && cell >= 0) flush_moments<kB>(box + cell, acc);
@@ -621,318 +634,241 @@ __global__ __launch_bounds__(kThreads) void fused_tile_rare_kernel(PicDesc d, Pi
 __global__ void zero_count_kernel(int32_t* c) { *c = 0; }
 
 // Direct-current branch of time_loop_electrodynamic (evolve.py:44-67) on
-// tile-sorted particles of an exact 3-D first-order grid, fused: gather from
-// the tile's LDS field box, push, x += v dt/2 (FP64, rounded to FP32 like
+// tile-sorted particles of a 3-D first-order grid, fused: gather from the
+// tile's LDS field box, push, x += v dt/2 (FP64, rounded to FP32 like
 // pic_advance_positions), particle boundaries, the J_from_rhov deposit at the
 // half position (J_from_rhov.py:88-200: node weights 1 - dn/d, dn/d and face
 // weights 1 - df/d, df/d with df = dn - d/2 on the 2x2x2 nodes of the centre
-// anchor, summed in registers over a thread's equal-anchor particles and
-// added into an LDS J box), x += v dt/2, boundaries, store.  Particles the
-// fast loop does not cover are listed for fused_direct_rare_kernel.  kVec:
-// a thread's four slots are stored with one 16-byte store per plane at the
-// end (24 more registers); otherwise each slot is stored as it finishes,
-// which keeps the kernel at 128 VGPRs for 4 waves per SIMD.
-template <int kT, int kMinBlocks, bool kVec, int kP = 4, bool kGather = false>
-__global__ __launch_bounds__(kThreads, kMinBlocks) void fused_tile_direct_kernel(
-    PicDesc d, PicSpecies sp, PicParticles in, FieldPtrs fp, PicParticles out, float* Jx, float* Jy, float* Jz,
-    const int32_t* __restrict__ starts, TileGeom tg, ExactGrid eg, int32_t* __restrict__ rare, int vec_ok, SpeciesTable st,
-    const int32_t* __restrict__ gather) {
-    constexpr int kB = kT + 5;
+// anchor), x += v dt/2, boundaries, store.  Slots, boxes and anchors as in
+// fused_tile_exact_kernel; the 24 node values of a cell are summed in registers
+// over a thread's particles and four lanes, then added into the J box, whose
+// one more node per axis takes half positions.  Particles the fast loop does not
+// cover are listed for fused_direct_rare_kernel.
+// Bound by VALU instructions.  13.8M particles on 96 x 80 x 112 cells of 0.1:
+// 392 us with FP64 anchors (1.8 TB/s); as separate push, advance, boundary and
+// deposit launches, whose deposit added with ds_add_f32, 3100 us.
+template <int kT, bool kGather, bool kExact, bool kAll>
+__global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_direct_kernel(
+    PicDesc d, PicParticles in, FieldPtrs fp, PicParticles out, float* Jx, float* Jy, float* Jz,
+    const int32_t* __restrict__ starts, TileGeom tg, TileGrid grid, int32_t* __restrict__ rare, int vec_ok,
+    SpeciesTable st, const int32_t* __restrict__ gather) {
+    constexpr int kP = 4;
+    constexpr int kB = kT + 5;                     // nodes per axis of the current box
     constexpr int kB3 = kB * kB * kB;
-    constexpr int kFB = kT + 4;
-    constexpr int kFV = kFB * kFB * kFB;
+    constexpr int kF = kT + 4;                     // and of the field box
+    constexpr int kF3 = kF * kF * kF;
     constexpr int kChunk = kThreads * kP;
-    __shared__ float box[3 * kB3];
-    __shared__ float fbox[6 * kFV];
+    constexpr int kUnroll = kExact ? kP : 1;       // as in fused_tile_exact_kernel
+    using Sum = BoxSum<kT>;
+    __shared__ Sum box[3 * kB3];
+    __shared__ float fbox[6 * kF3];
     const int b = xcd_block((int)blockIdx.x, (int)gridDim.x);
     const int64_t begin = starts[b], end = starts[b + 1];
     if (begin >= end) return;
     const int t = b % (tg.tiles + 1);
     const int s = b / (tg.tiles + 1);
-    int o[3] = {0, 0, 0}, fo[3] = {0, 0, 0};
+    int fo[3] = {0, 0, 0};
     // interior: a fast-path particle (anchors inside the field box, cells
     // c0 - 2 .. c0 + T + 1) that moves less than a cell per step stays inside
     // [-W/2, W/2) on every axis, so its particle boundaries do nothing
     bool interior = t < tg.tiles;
     if (t < tg.tiles) {
-        const int tx = t / (tg.nt[1] * tg.nt[2]), ty = (t / tg.nt[2]) % tg.nt[1], tz = t % tg.nt[2];
-        const int c0[3] = {tx * kT, ty * kT, tz * kT};
+        const int c0[3] = {(t / (tg.nt[1] * tg.nt[2])) * kT, ((t / tg.nt[2]) % tg.nt[1]) * kT, (t % tg.nt[2]) * kT};
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
-            o[a] = fo[a] = c0[a] + d.g - 2;
+            fo[a] = c0[a] + d.g - 2;
             interior = interior && c0[a] >= 3 && c0[a] + kT + 3 <= d.n[a];
         }
     }
-    const float fdt = (float)d.dt;
-    for (int e = threadIdx.x; e < 3 * kB3; e += kThreads) box[e] = 0.0f;
-    fill_field_box<kFB>(d, fp, fo, fbox);
+    // old positions as in fused_tile_exact_kernel; half positions: centre anchor and the node above in the J box
+    float nb[3], xlo[3], xhi[3], hhi[3];
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+        const double org = d.org_c[a], sp = d.sp_c[a], margin = kExact ? 0.0 : 1.0e-6 * sp;
+        nb[a] = uniform((float)(fo[a] * sp + org));
+        xlo[a] = uniform(__double2float_ru(fmax(fo[a] * sp + org + 0.5 * sp, org) + margin));
+        xhi[a] = uniform(__double2float_ru(min(fo[a] + kF - 1, d.dims[a] - 1) * sp + org - margin));
+        hhi[a] = uniform(__double2float_ru((fo[a] + kB - 1) * sp + org - margin));
+    }
+    const auto inside = [&](int64_t s0) { return vec_ok && s0 >= begin && s0 + kP <= end; };
+    const int64_t first = begin & ~(int64_t)(kP - 1);
+    const int64_t g0 = first + (int64_t)kP * (int)threadIdx.x;
+    float PX[3][kP], PU[3][kP];
+    uint32_t pact;
+    load_group<kP, kGather>(in, gather, g0, begin, end, inside(g0), PX, PU, pact);
+    for (int e = threadIdx.x; e < 3 * kB3; e += kThreads) box[e] = (Sum)0;
+    fill_field_box<kF>(d, fp, fo, fbox);
     __syncthreads();
-    const FieldBox fb{fbox, {fo[0], fo[1], fo[2]}, kFB};
-    const SpeciesK k = st.k[s];
+    const SpeciesK& k = st.k[s];
     const double hdt = 0.5 * d.dt;
-    auto flush = [&](int h0, int h1, int h2, const float* acc) {
-        float* p = box + ((h0 - o[0]) * kB + (h1 - o[1])) * kB + (h2 - o[2]);
+    const auto flush = [&](int cell, const float* acc) {
+        Sum* p = box + cell;
 #pragma unroll
         for (int m = 0; m < 24; ++m) {
-            const int c = m >> 3, n = m & 7;
-            atomicAdd(p + c * kB3 + ((n >> 2) * kB + ((n >> 1) & 1)) * kB + (n & 1), acc[m]);
+            const int n = m & 7;
+            box_add(p + (m >> 3) * kB3 + ((n >> 2) * kB + ((n >> 1) & 1)) * kB + (n & 1), acc[m]);
+            if ((m & 3) == 3) __builtin_amdgcn_sched_barrier(0);   // bound the live FP64 values
         }
     };
 
-    for (int64_t base = begin & ~(int64_t)(kP - 1); base < end; base += kChunk) {
-        const int64_t s0 = base + (int64_t)kP * threadIdx.x;
+    for (int64_t base = first; base < end; base += kChunk) {
+        const int64_t s0 = base + (int64_t)kP * (int)threadIdx.x;
+        const bool full = inside(s0);
+        if (base != first) load_group<kP, kGather>(in, gather, s0, begin, end, full, PX, PU, pact);
         float acc[24];
 #pragma unroll
         for (int m = 0; m < 24; ++m) acc[m] = 0.0f;
-        int h0 = 0, h1 = 0, h2 = 0;
-        bool have = false;
-        // kVec: OX/OU first hold the group's inputs (one kP-wide load per plane
-        // when the group lies inside the range) and take its outputs slot by
-        // slot, as in fused_tile_exact_kernel
-        float OX[3][kP], OU[3][kP];
-        uint32_t pact = 0u, oact = 0u;
-        const bool full = vec_ok && s0 >= begin && s0 + kP <= end;
-        if constexpr (kVec) {
-            if (!kGather && full) {
+        int cell = -1;
+        uint32_t oact = 0u;
+#pragma unroll kUnroll
+        for (int j = 0; j < kP; ++j) {
+            const float xf[3] = {PX[0][0], PX[1][0], PX[2][0]};
+            float v[3] = {PU[0][0], PU[1][0], PU[2][0]};
+            const bool act0 = (pact & 0xffu) != 0u;
+            pact >>= 8;
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    load_vec<kP>(in.x[a] + s0, OX[a]);
-                    load_vec<kP>(in.u[a] + s0, OU[a]);
-                }
-                if constexpr (kP == 4) pact = *reinterpret_cast<const uint32_t*>(in.active + s0);
-                else pact = *reinterpret_cast<const uint16_t*>(in.active + s0);
-            } else if (kGather && full) {
-                // slot i's input is in.*[gather[i]] (a re-bin's permutation)
-                float gf[kP];
-                load_vec<kP>(reinterpret_cast<const float*>(gather + s0), gf);
+            for (int a = 0; a < 3; ++a) {
 #pragma unroll
-                for (int j = 0; j < kP; ++j) {
-                    const int64_t src = __float_as_int(gf[j]);
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        OX[a][j] = in.x[a][src];
-                        OU[a][j] = in.u[a][src];
-                    }
-                    pact |= (in.active[src] != 0 ? 1u : 0u) << (8 * j);
-                }
-            } else {
-#pragma unroll
-                for (int j = 0; j < kP; ++j) {
-                    const int64_t i = s0 + j;
-                    const bool inr = i >= begin && i < end;
-                    const int64_t src = kGather ? (inr ? (int64_t)gather[i] : 0) : i;
-#pragma unroll
-                    for (int a = 0; a < 3; ++a) {
-                        OX[a][j] = inr ? in.x[a][src] : 0.0f;
-                        OU[a][j] = inr ? in.u[a][src] : 0.0f;
-                    }
-                    pact |= (inr && in.active[src] != 0 ? 1u : 0u) << (8 * j);
+                for (int q = 0; q + 1 < kP; ++q) {
+                    PX[a][q] = PX[a][q + 1];
+                    PU[a][q] = PU[a][q + 1];
                 }
             }
-        }
-#pragma unroll 1
-        for (int j = 0; j < kP; ++j) {
-            const int64_t i = s0 + j;
             float ox[3] = {0.0f, 0.0f, 0.0f}, ou[3] = {0.0f, 0.0f, 0.0f};
             uint32_t oa = 0u;
-            float xf[3], v[3];
-            bool act0;
-            if constexpr (kVec) {
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    xf[a] = OX[a][0];
-                    v[a] = OU[a][0];
-#pragma unroll
-                    for (int q = 0; q + 1 < kP; ++q) {
-                        OX[a][q] = OX[a][q + 1];
-                        OU[a][q] = OU[a][q + 1];
-                    }
-                }
-                act0 = (pact & 0xffu) != 0u;
-                pact >>= 8;
-            }
             do {
-            if constexpr (!kVec) {
-                if (i < begin || i >= end) break;
-                const int64_t src = kGather ? (int64_t)gather[i] : i;
-                act0 = in.active[src] != 0;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    xf[a] = in.x[a][src];
-                    v[a] = in.u[a][src];
-                }
-                loads_together(xf, v);
-            }
             if (!act0) break;
-            int anc[3], anv[3];
-            float dc[3], dv[3], nodec[3];
             bool fast = true;
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                fast = fast && xf[a] >= eg.xlo[a] && xf[a] < eg.xhi[a];
-                exact_anchors(xf[a], eg.org_c[a], eg.sp_c[a], eg.isp_c[a], eg.half_sp[a], anc[a], dc[a], nodec[a],
-                              anv[a], dv[a]);
-                fast = fast && (unsigned)(anc[a] - fo[a]) < (unsigned)(kFB - 1) &&
-                       (unsigned)(anv[a] - fo[a]) < (unsigned)(kFB - 1);
-            }
+            for (int a = 0; a < 3; ++a) fast = fast & (xf[a] >= xlo[a]) & (xf[a] < xhi[a]);
+            float f[3], dc[3], qm[3], dv[3];
+            bool up[3];
+#pragma unroll
+            for (int a = 0; a < 3; ++a)
+                fast = tile_anchor<kExact>(grid, a, xf[a], nb[a], (float)fo[a], f[a], dc[a], qm[a], up[a], dv[a]) & fast;
             if (!fast) {
-                rare_push(rare, i);
+                rare_push(rare, s0 + j);
                 break;
             }
-            CicAxis gc[3], gv[3];
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                const float rc = dc[a] * eg.isp_c[a], rv = dv[a] * eg.isp_c[a];
-                gc[a].p0 = gc[a].p1 = gv[a].p0 = gv[a].p1 = 0;
-                gc[a].w0 = 1.0f - rc;
-                gc[a].w1 = rc;
-                gv[a].w0 = 1.0f - rv;
-                gv[a].w1 = rv;
-            }
             float E[3], Bf[3];
-            E[0] = gather_box(fb, 0, anv[0], anc[1], anc[2], gv[0], gc[1], gc[2]);
-            E[1] = gather_box(fb, 1, anc[0], anv[1], anc[2], gc[0], gv[1], gc[2]);
-            E[2] = gather_box(fb, 2, anc[0], anc[1], anv[2], gc[0], gc[1], gv[2]);
-            Bf[0] = gather_box(fb, 3, anc[0], anv[1], anv[2], gc[0], gv[1], gv[2]);
-            Bf[1] = gather_box(fb, 4, anv[0], anc[1], anv[2], gv[0], gc[1], gv[2]);
-            Bf[2] = gather_box(fb, 5, anv[0], anv[1], anc[2], gv[0], gv[1], gc[2]);
+            {
+                const int at = (int)fmaf(f[0], (float)(kF * kF), fmaf(f[1], (float)kF, f[2]));
+                CicAxis gc[3], gv[3];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) {
+                    gc[a].w0 = fmaf(-dc[a], grid.isp[a], 1.0f);
+                    gc[a].w1 = dc[a] * grid.isp[a];
+                    gv[a].w0 = fmaf(-dv[a], grid.isp[a], 1.0f);
+                    gv[a].w1 = dv[a] * grid.isp[a];
+                }
+                // off an exact grid the particles are those of pic_push bit for bit
+                constexpr CicRounding kE1 = kExact ? kPlain : kSecond, kBs = kExact ? kPlain : kMagnetic;
+                const int lx = up[0] ? 0 : kF * kF, ly = up[1] ? 0 : kF, lz = up[2] ? 0 : 1;   // vertex node below
+                E[0] = gather_at<kF>(fbox + at - lx, gv[0], gc[1], gc[2]);
+                E[1] = gather_at<kF, kE1>(fbox + kF3 + at - ly, gc[0], gv[1], gc[2]);
+                E[2] = gather_at<kF>(fbox + 2 * kF3 + at - lz, gc[0], gc[1], gv[2]);
+                Bf[0] = gather_at<kF, kBs>(fbox + 3 * kF3 + at - ly - lz, gc[0], gv[1], gv[2]);
+                Bf[1] = gather_at<kF, kBs>(fbox + 4 * kF3 + at - lx - lz, gv[0], gc[1], gv[2]);
+                Bf[2] = gather_at<kF, kBs>(fbox + 5 * kF3 + at - lx - ly, gv[0], gv[1], gc[2]);
+            }
             float nv[3] = {v[0], v[1], v[2]};
             push_velocity(nv, E, Bf, k.h, d);
 #pragma unroll
             for (int a = 0; a < 3; ++a)
-                if ((k.uu >> a) & 1u) v[a] = nv[a];
+                if (kAll || ((k.uu >> a) & 1u)) v[a] = nv[a];
             // ---- x += v dt/2, boundaries (evolve.py:48-52)
             bool act = true;
             bool skip_bc = interior;
 #pragma unroll
-            for (int a = 0; a < 3; ++a) skip_bc = skip_bc && fabsf(v[a]) * fdt < 0.99f * eg.sp_c[a];
-            float xh[3];
+            for (int a = 0; a < 3; ++a) skip_bc = skip_bc & (fabsf(v[a]) * grid.dt32 < 0.99f * grid.sp[a]);
+            const auto half_step = [&](float (&x)[3]) {
+                double p[3];
 #pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                double t = ((k.ux >> a) & 1u) ? (double)(float)step_pos((double)xf[a], (double)v[a], hdt)
-                                              : (double)xf[a];
+                for (int a = 0; a < 3; ++a)
+                    p[a] = kAll || ((k.ux >> a) & 1u) ? (double)(float)step_pos((double)x[a], (double)v[a], hdt)
+                                                      : (double)x[a];
                 if (!skip_bc) {
-                    if (d.pbc[a] == 0) periodic_wrap(d.wind[a], t);
-                    else apply_axis_boundary(d.pbc[a], d.wind[a], t, v[a], act);
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) {
+                        double wind = d.wind[a];
+                        asm volatile("" : "+s"(wind));      // see fused_tile_exact_kernel
+                        if (d.pbc[a] == 0) periodic_wrap(wind, p[a]);
+                        else apply_axis_boundary(d.pbc[a], wind, p[a], v[a], act);
+                    }
                 }
-                xh[a] = (float)t;
-            }
+#pragma unroll
+                for (int a = 0; a < 3; ++a) x[a] = (float)p[a];
+            };
+            float xh[3] = {xf[0], xf[1], xf[2]};
+            half_step(xh);
             if (act) {
-                // ---- J_from_rhov at the half position (anchors exact in FP32)
-                int an[3];
+                // ---- J_from_rhov at the half position
                 float dn[3];
                 bool inbox = true;
 #pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    int av2;
-                    float nd, dv2;
-                    inbox = inbox && xh[a] >= eg.xlo[a] && xh[a] < eg.xhi[a];
-                    exact_anchors(xh[a], eg.org_c[a], eg.sp_c[a], eg.isp_c[a], eg.half_sp[a], an[a], dn[a], nd, av2,
-                                  dv2);
-                    inbox = inbox && (unsigned)(an[a] - o[a]) <= (unsigned)(kB - 2);
-                }
+                for (int a = 0; a < 3; ++a) inbox = inbox & (xh[a] >= nb[a]) & (xh[a] < hhi[a]);
+#pragma unroll
+                for (int a = 0; a < 3; ++a)
+                    inbox = tile_anchor<kExact>(grid, a, xh[a], nb[a], (float)fo[a], f[a], dn[a], qm[a], up[a], dv[a]) &
+                            inbox & (f[a] >= 0.0f) & (f[a] <= kB - 2.0f);
                 if (!inbox) {
-                    rare_push(rare, i);
+                    rare_push(rare, s0 + j);
                     break;
+                }
+                const int at = (int)fmaf(f[0], (float)(kB * kB), fmaf(f[1], (float)kB, f[2]));
+                if (at != cell) {
+                    if (cell >= 0) flush(cell, acc);
+#pragma unroll
+                    for (int m = 0; m < 24; ++m) acc[m] = 0.0f;
+                    cell = at;
                 }
                 float wn[3][2], wf[3][2];
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    const float r = dn[a] * eg.inv_d[a];
-                    wn[a][0] = 1.0f - r;
-                    wn[a][1] = r;
-                    const float rf = (dn[a] - eg.half_sp[a]) * eg.inv_d[a];
-                    wf[a][0] = 1.0f - rf;
-                    wf[a][1] = rf;
+                    wn[a][1] = dn[a] * grid.inv_d[a];
+                    wn[a][0] = 1.0f - wn[a][1];
+                    wf[a][1] = (dn[a] - grid.half[a]) * grid.inv_d[a];
+                    wf[a][0] = 1.0f - wf[a][1];
                 }
-                const float qv[3] = {k.q_dv * v[0], k.q_dv * v[1], k.q_dv * v[2]};
-                float val[24];
 #pragma unroll
-                for (int n = 0; n < 8; ++n) {
-                    const int xi = n >> 2, yi = (n >> 1) & 1, zi = n & 1;
-                    val[n] = qv[0] * wf[0][xi] * wn[1][yi] * wn[2][zi];
-                    val[8 + n] = qv[1] * wn[0][xi] * wf[1][yi] * wn[2][zi];
-                    val[16 + n] = qv[2] * wn[0][xi] * wn[1][yi] * wf[2][zi];
-                }
-                const bool same = have && an[0] == h0 && an[1] == h1 && an[2] == h2;
-                if (have && !same) flush(h0, h1, h2, acc);
+                for (int c = 0; c < 3; ++c) {
+                    const float qv = k.q_dv * v[c];
 #pragma unroll
-                for (int m = 0; m < 24; ++m) acc[m] = (same ? acc[m] : 0.0f) + val[m];
-                h0 = an[0];
-                h1 = an[1];
-                h2 = an[2];
-                have = true;
-                // ---- x += v dt/2, boundaries (evolve.py:62-66)
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    double t2 = ((k.ux >> a) & 1u) ? (double)(float)step_pos((double)xh[a], (double)v[a], hdt)
-                                                   : (double)xh[a];
-                    if (!skip_bc) {
-                        if (d.pbc[a] == 0) periodic_wrap(d.wind[a], t2);
-                        else apply_axis_boundary(d.pbc[a], d.wind[a], t2, v[a], act);
+                    for (int n = 0; n < 4; ++n) {
+                        const int xi = n >> 1, yi = n & 1;
+                        const float w = qv * (c == 0 ? wf[0][xi] : wn[0][xi]) * (c == 1 ? wf[1][yi] : wn[1][yi]);
+                        acc[8 * c + 2 * n] = fmaf(w, c == 2 ? wf[2][0] : wn[2][0], acc[8 * c + 2 * n]);
+                        acc[8 * c + 2 * n + 1] = fmaf(w, c == 2 ? wf[2][1] : wn[2][1], acc[8 * c + 2 * n + 1]);
                     }
-                    ox[a] = (float)t2;
-                    ou[a] = v[a];
                 }
+                // ---- x += v dt/2, boundaries (evolve.py:62-66)
+                half_step(xh);
 #pragma unroll
                 for (int a = 0; a < 3; ++a) {
-                    ox[a] = act ? ox[a] : 0.0f;
-                    ou[a] = act ? ou[a] : 0.0f;
+                    ox[a] = act ? xh[a] : 0.0f;
+                    ou[a] = act ? v[a] : 0.0f;
                 }
                 oa = act ? 1u : 0u;
             }
             } while (false);
-            if constexpr (kVec) {
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    OX[a][kP - 1] = ox[a];
-                    OU[a][kP - 1] = ou[a];
-                }
-                oact = (oact >> 8) | (oa << (8 * (kP - 1)));
-            } else if (i >= begin && i < end) {
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    out.x[a][i] = ox[a];
-                    out.u[a][i] = ou[a];
-                }
-                out.active[i] = (uint8_t)oa;
-            }
-        }
-        {
-            // the group's last cell, summed over equal cells of neighbouring lanes first
-            const int key = have ? ((h0 - o[0]) * kB + (h1 - o[1])) * kB + (h2 - o[2]) : -1;
-            if (row_run_sums(key, acc) && have) flush(h0, h1, h2, acc);
-        }
-        if constexpr (!kVec) continue;
-        if (full) {
 #pragma unroll
             for (int a = 0; a < 3; ++a) {
-                store_vec<kP>(out.x[a] + s0, OX[a]);
-                store_vec<kP>(out.u[a] + s0, OU[a]);
+                PX[a][kP - 1] = ox[a];
+                PU[a][kP - 1] = ou[a];
             }
-            if constexpr (kP == 4) *reinterpret_cast<uint32_t*>(out.active + s0) = oact;
-            else *reinterpret_cast<uint16_t*>(out.active + s0) = (uint16_t)oact;
-        } else {
-#pragma unroll
-            for (int j = 0; j < kP; ++j) {
-                const int64_t i = s0 + j;
-                if (i < begin || i >= end) continue;
-#pragma unroll
-                for (int a = 0; a < 3; ++a) {
-                    out.x[a][i] = OX[a][j];
-                    out.u[a][i] = OU[a][j];
-                }
-                out.active[i] = (uint8_t)((oact >> (8 * j)) & 0xffu);
-            }
+            oact = (oact >> 8) | (oa << (8 * (kP - 1)));
         }
+        store_group<kP>(out, s0, begin, end, full, PX, PU, oact);
+        if (row_run_sums<4>(cell, acc) && cell >= 0) flush(cell, acc);
     }
     __syncthreads();
-    flush_current_box<kB>(d, o, box, Jx, Jy, Jz);
+    flush_current_box<kB>(d, fo, box, Jx, Jy, Jz);
 }
 
 // The rare list of fused_tile_direct_kernel: each listed particle runs the
 // direct branch through the general route (global gather, FP64 anchors, the
 // 3^3 deposit into J).
+template <bool kExact>
 __global__ __launch_bounds__(kThreads) void fused_direct_rare_kernel(PicDesc d, PicSpecies sp, PicParticles in,
                                                                      FieldPtrs fp, PicParticles out, float* Jx,
                                                                      float* Jy, float* Jz,
@@ -958,11 +894,11 @@ __global__ __launch_bounds__(kThreads) void fused_direct_rare_kernel(PicDesc d, 
                      gv[a], an, dl);
         }
         E[0] = gather_cic(fp.E[0], fp.Ee[0], d, gv[0], gc[1], gc[2]);
-        E[1] = gather_cic(fp.E[1], fp.Ee[1], d, gc[0], gv[1], gc[2]);
+        E[1] = gather_cic<kExact ? kPlain : kSecond>(fp.E[1], fp.Ee[1], d, gc[0], gv[1], gc[2]);
         E[2] = gather_cic(fp.E[2], fp.Ee[2], d, gc[0], gc[1], gv[2]);
-        B[0] = gather_cic(fp.B[0], fp.Be[0], d, gc[0], gv[1], gv[2]);
-        B[1] = gather_cic(fp.B[1], fp.Be[1], d, gv[0], gc[1], gv[2]);
-        B[2] = gather_cic(fp.B[2], fp.Be[2], d, gv[0], gv[1], gc[2]);
+        B[0] = gather_cic<kExact ? kPlain : kMagnetic>(fp.B[0], fp.Be[0], d, gc[0], gv[1], gv[2]);
+        B[1] = gather_cic<kExact ? kPlain : kMagnetic>(fp.B[1], fp.Be[1], d, gv[0], gc[1], gv[2]);
+        B[2] = gather_cic<kExact ? kPlain : kMagnetic>(fp.B[2], fp.Be[2], d, gv[0], gv[1], gc[2]);
         float nv[3] = {v[0], v[1], v[2]};
         push_velocity(nv, E, B, k.h, d);
         for (int a = 0; a < 3; ++a)
@@ -1045,16 +981,29 @@ int pic_fused_push_esirkepov(const PicDesc* desc, const PicSpecies* sp, const Pi
     return 0;
 }
 
+// Vector loads and stores of a thread's slot group need 16-byte aligned planes.
+static int groups_aligned(const PicParticles* in, const PicParticles* out, const int32_t* gather) {
+    int ok = 1;
+    for (int a = 0; a < 3; ++a)
+        ok &= ((((uintptr_t)out->x[a]) | ((uintptr_t)out->u[a]) | ((uintptr_t)in->x[a]) |
+                ((uintptr_t)in->u[a])) & 15u) == 0;
+    ok &= ((((uintptr_t)out->active) | ((uintptr_t)in->active)) & 3u) == 0;
+    ok &= (((uintptr_t)gather) & 15u) == 0;
+    return ok;
+}
+
 static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
                               const float* const E[3], const float* const B[3], const float* const E_ext[3],
                               const float* const B_ext[3], PicParticles* out, float* const J[3], int32_t tile,
                               const int32_t* starts, int32_t min_blocks, int32_t* workspace, const int32_t* gather,
-                              void* stream) {
+                              bool general, void* stream) {
     PIC_REQUIRE(desc_ok(desc) && particles_ok(sp, in) && particles_ok(sp, out) && E && B && J && starts && workspace);
     PIC_REQUIRE(fused_kind(*desc) == 3 && (tile == 4 || tile == 8) && (min_blocks == 1 || min_blocks == 4));
     ExactGrid eg;
-    PIC_REQUIRE(make_exact_grid(*desc, eg));
-    for (int a = 0; a < 3; ++a) PIC_REQUIRE(desc->d[a] == desc->sp_c[a]);
+    TileGrid grid;
+    const bool exact = make_exact_grid(*desc, eg) && desc->d[0] == desc->sp_c[0] && desc->d[1] == desc->sp_c[1] &&
+                       desc->d[2] == desc->sp_c[2];
+    PIC_REQUIRE((exact || general) && make_tile_grid(*desc, grid));
     const bool empty = (int64_t)sp->count * sp->slots == 0;
     for (int a = 0; a < 3; ++a)
         PIC_REQUIRE(E[a] && B[a] && J[a] && (empty || (in->x[a] != out->x[a] && in->u[a] != out->u[a])));
@@ -1071,38 +1020,35 @@ static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const P
     PIC_REQUIRE(blocks < ((int64_t)1 << 31));
     hipStream_t st = as_stream(stream);
     FieldPtrs fp = make_fields(E, B, E_ext, B_ext);
-    int vec_ok = 1;
-    for (int a = 0; a < 3; ++a)
-        vec_ok &= ((((uintptr_t)out->x[a]) | ((uintptr_t)out->u[a]) | ((uintptr_t)in->x[a]) |
-                    ((uintptr_t)in->u[a])) & 15u) == 0;
-    vec_ok &= ((((uintptr_t)out->active) | ((uintptr_t)in->active)) & 3u) == 0;
-    vec_ok &= (((uintptr_t)gather) & 15u) == 0;
+    const int vec_ok = groups_aligned(in, out, gather);
     hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, st, workspace);
     const SpeciesTable stab = species_table(*desc, *sp);
-#define PIC_DIRECT_LAUNCH2(T, MB, V, P)                                                                              \
-    do {                                                                                                             \
-        if (gather)                                                                                                  \
-            hipLaunchKernelGGL((fused_tile_direct_kernel<T, MB, V, P, true>), dim3((unsigned)blocks), dim3(kThreads), \
-                               0, st, *desc, *sp, *in, fp, *out, J[0], J[1], J[2], starts, tg, eg, workspace, vec_ok, \
-                               stab, gather);                                                                        \
-        else                                                                                                         \
-            hipLaunchKernelGGL((fused_tile_direct_kernel<T, MB, V, P, false>), dim3((unsigned)blocks),               \
-                               dim3(kThreads), 0, st, *desc, *sp, *in, fp, *out, J[0], J[1], J[2], starts, tg, eg,   \
-                               workspace, vec_ok, stab, gather);                                                     \
+    bool all = true;
+    for (int s = 0; s < sp->count; ++s) all = all && stab.k[s].ux == 7u && stab.k[s].uu == 7u;
+#define PIC_DIRECT_LAUNCH(T, GA, EX, ALL)                                                                        \
+    hipLaunchKernelGGL((fused_tile_direct_kernel<T, GA, EX, ALL>), dim3((unsigned)blocks), dim3(kThreads), 0, st, \
+                       *desc, *in, fp, *out, J[0], J[1], J[2], starts, tg, grid, workspace, vec_ok, stab, gather)
+#define PIC_DIRECT_ALL(T, GA, EX)                          \
+    do {                                                   \
+        if (all) PIC_DIRECT_LAUNCH(T, GA, EX, true);       \
+        else PIC_DIRECT_LAUNCH(T, GA, EX, false);          \
     } while (0)
-#define PIC_DIRECT_LAUNCH(T, MB, V) PIC_DIRECT_LAUNCH2(T, MB, V, 4)
-    if (tile == 8) {
-        if (min_blocks == 4) PIC_DIRECT_LAUNCH(8, 4, false);
-        else PIC_DIRECT_LAUNCH(8, 1, true);
-    } else {
-        if (min_blocks == 4) PIC_DIRECT_LAUNCH2(4, 4, true, 2);
-        else PIC_DIRECT_LAUNCH(4, 1, true);
-    }
+    // a gathered launch is only made on exact grids
+#define PIC_DIRECT_SHAPE(T)                           \
+    do {                                              \
+        if (!exact) PIC_DIRECT_ALL(T, false, false);  \
+        else if (gather) PIC_DIRECT_ALL(T, true, true); \
+        else PIC_DIRECT_ALL(T, false, true);          \
+    } while (0)
+    if (tile == 8) PIC_DIRECT_SHAPE(8);
+    else PIC_DIRECT_SHAPE(4);
+#undef PIC_DIRECT_SHAPE
+#undef PIC_DIRECT_ALL
 #undef PIC_DIRECT_LAUNCH
-#undef PIC_DIRECT_LAUNCH2
     const int64_t rare_grid = std::min<int64_t>(std::max<int64_t>(grid_1d(n, kThreads), 1), 1024);
-    hipLaunchKernelGGL(fused_direct_rare_kernel, dim3((unsigned)rare_grid), dim3(kThreads), 0, st, *desc, *sp, *in,
-                       fp, *out, J[0], J[1], J[2], workspace, gather);
+    hipLaunchKernelGGL(exact ? fused_direct_rare_kernel<true> : fused_direct_rare_kernel<false>,
+                       dim3((unsigned)rare_grid), dim3(kThreads), 0, st, *desc, *sp, *in, fp, *out, J[0], J[1], J[2],
+                       workspace, gather);
     PIC_CHECK_LAUNCH();
     return 0;
 }
@@ -1112,6 +1058,14 @@ int pic_fused_push_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const
                                 const float* const B_ext[3], PicParticles* out, float* const J[3], int32_t tile,
                                 const int32_t* starts, int32_t min_blocks, int32_t* workspace, void* stream) {
     return fused_direct_tiled(desc, sp, in, E, B, E_ext, B_ext, out, J, tile, starts, min_blocks, workspace, nullptr,
+                              false, stream);
+}
+
+int pic_fused_push_direct_tiled_general(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                        const float* const E[3], const float* const B[3], const float* const E_ext[3],
+                                        const float* const B_ext[3], PicParticles* out, float* const J[3],
+                                        int32_t tile, const int32_t* starts, int32_t* workspace, void* stream) {
+    return fused_direct_tiled(desc, sp, in, E, B, E_ext, B_ext, out, J, tile, starts, 1, workspace, nullptr, true,
                               stream);
 }
 
@@ -1122,7 +1076,12 @@ int pic_fused_push_direct_tiled_gather(const PicDesc* desc, const PicSpecies* sp
                                        int32_t* workspace, void* stream) {
     PIC_REQUIRE(sp && (gather || (int64_t)sp->count * sp->slots == 0));
     return fused_direct_tiled(desc, sp, in, E, B, E_ext, B_ext, out, J, tile, starts, min_blocks, workspace, gather,
-                              stream);
+                              false, stream);
+}
+
+int pic_tile_general_grid(const PicDesc* desc) {
+    TileGrid grid;
+    return desc && desc_ok(desc) && fused_kind(*desc) == 3 && make_tile_grid(*desc, grid) ? 1 : 0;
 }
 
 int pic_tile_exact_grid(const PicDesc* desc) {
@@ -1137,13 +1096,7 @@ static void launch_tile_esirkepov(const PicDesc* desc, const PicSpecies* sp, con
                                   const int32_t* starts, const TileGeom& tg, const TileGrid& grid, bool exact,
                                   int32_t* workspace, const int32_t* gather, int64_t blocks,
                                   hipStream_t st) {
-    // vector loads and stores of a thread's slot group need 16-byte aligned planes
-    int vec_ok = 1;
-    for (int a = 0; a < 3; ++a)
-        vec_ok &= ((((uintptr_t)out->x[a]) | ((uintptr_t)out->u[a]) | ((uintptr_t)in->x[a]) |
-                    ((uintptr_t)in->u[a])) & 15u) == 0;
-    vec_ok &= ((((uintptr_t)out->active) | ((uintptr_t)in->active)) & 3u) == 0;
-    vec_ok &= (((uintptr_t)gather) & 15u) == 0;
+    const int vec_ok = groups_aligned(in, out, gather);
     hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, st, workspace);
     const SpeciesTable stab = species_table(*desc, *sp);
     bool all = true;

@@ -113,18 +113,30 @@ __device__ inline void cic_axis(float x, float org32, float isp32, double org, d
     s.w1 = r;
 }
 
-// Both products rounded in one stated way.  Left to contraction, which of two
-// products is fused differs between kernels that inline the same source; with
-// the fused operations written out every kernel gives a particle the same field.
-__device__ inline float mix(float w0, float a, float w1, float b) { return fmaf(w1, b, w0 * a); }
+// The gather's fused operations are written out.  Left to contraction, which of
+// two products is fused differs between kernels that inline the same source, and
+// an ulp of a velocity can put a particle on the other side of a cell face, where
+// the weights of J_from_rhov jump.  There are two roundings: kPlain, of the
+// Esirkepov kernels and the direct kernel on an exact grid, and the one of the
+// push into slot order (pic_push), whose results are kept bit for bit: kSecond
+// for its E_y, kMagnetic for B, kPlain for E_x and E_z.
+enum CicRounding { kPlain, kSecond, kMagnetic };
 
-__device__ inline float cic_value(float v000, float v001, float v010, float v011, float v100, float v101, float v110,
-                                  float v111, const CicAxis& ax, const CicAxis& ay, const CicAxis& az) {
-    const float c00 = mix(az.w0, v000, az.w1, v001), c01 = mix(az.w0, v010, az.w1, v011);
-    const float c10 = mix(az.w0, v100, az.w1, v101), c11 = mix(az.w0, v110, az.w1, v111);
-    return mix(ax.w0, mix(ay.w0, c00, ay.w1, c01), ax.w1, mix(ay.w0, c10, ay.w1, c11));
+template <bool kSwap>
+__device__ inline float mix(float w0, float a, float w1, float b) {
+    return kSwap ? fmaf(w1, b, w0 * a) : fmaf(w0, a, w1 * b);
 }
 
+template <CicRounding kR>
+__device__ inline float cic_value(float v000, float v001, float v010, float v011, float v100, float v101, float v110,
+                                  float v111, const CicAxis& ax, const CicAxis& ay, const CicAxis& az) {
+    constexpr bool kZ0 = kR != kPlain, kB = kR == kMagnetic;
+    const float c00 = mix<kZ0>(az.w0, v000, az.w1, v001), c01 = mix<kZ0>(az.w0, v010, az.w1, v011);
+    const float c10 = mix<false>(az.w0, v100, az.w1, v101), c11 = mix<false>(az.w0, v110, az.w1, v111);
+    return mix<kB>(ax.w0, mix<kB>(ay.w0, c00, ay.w1, c01), ax.w1, mix<false>(ay.w0, c10, ay.w1, c11));
+}
+
+template <CicRounding kR = kPlain>
 __device__ inline float gather_cic(const float* __restrict__ f, const float* __restrict__ fe, const PicDesc& d,
                                    const CicAxis& ax, const CicAxis& ay, const CicAxis& az) {
     // 32-bit unsigned offsets on a uniform base (field_size < 2^31 is checked at launch)
@@ -144,7 +156,7 @@ __device__ inline float gather_cic(const float* __restrict__ f, const float* __r
         v110 += fe[r11 + z0];
         v111 += fe[r11 + z1];
     }
-    return cic_value(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
+    return cic_value<kR>(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
 }
 
 // Gather stencil of one axis and node line with kN = 2 (first order: points a,
@@ -187,12 +199,33 @@ __device__ inline void point_axis(float x, double org, double sp, int L, int g, 
     }
 }
 
-// Weighted sum of kN values in the order of gather_cic (the roundings of the
-// first-order kernels then agree).
-template <int kN>
-__device__ inline float weighted(const float (&v)[kN], const float (&w)[kN]) {
-    if constexpr (kN == 2) return mix(w[0], v[0], w[1], v[1]);
-    else return v[0] * w[0] + v[1] * w[1] + v[2] * w[2];
+// Weighted sum over a stencil of kN^3 points, rows v[i][j][.] from `row(i, j, v)`:
+// as cic_value for two points, and as the reference's running sum
+// v (w_x w_y w_z) for three (gather3).
+template <int kN, CicRounding kR, class Row>
+__device__ inline float stencil_sum(const float (&wx)[kN], const float (&wy)[kN], const float (&wz)[kN],
+                                    const Row& row) {
+    if constexpr (kN == 2) {
+        float v[4][2];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) row(q >> 1, q & 1, v[q]);
+        const CicAxis ax{0, 0, wx[0], wx[1]}, ay{0, 0, wy[0], wy[1]}, az{0, 0, wz[0], wz[1]};
+        return cic_value<kR>(v[0][0], v[0][1], v[1][0], v[1][1], v[2][0], v[2][1], v[3][0], v[3][1], ax, ay, az);
+    } else {
+        float acc = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+#pragma unroll
+            for (int j = 0; j < kN; ++j) {
+                float v[kN];
+                row(i, j, v);
+                const float wij = wx[i] * wy[j];
+#pragma unroll
+                for (int k = 0; k < kN; ++k) acc = fmaf(v[k], wij * wz[k], acc);
+            }
+        }
+        return acc;
+    }
 }
 
 // kN consecutive floats at p (4-byte aligned): one load instruction.
@@ -205,53 +238,41 @@ __device__ inline void load_run(const float* p, float (&v)[kN]) {
 // (every lane of the wave), so a stencil row is one load instead of kN; a
 // random-order gather is bound by its load instructions (one line per lane
 // each).  Offsets are 32-bit where the component spans under 4 GiB.
-template <int kShape, bool kRun, class Idx>
+template <int kShape, CicRounding kR, bool kRun, class Idx>
 __device__ inline float gather_point(const float* __restrict__ f, const float* __restrict__ fe, Idx sx, Idx sy,
                                      const PointAxis<kShape>& ax, const PointAxis<kShape>& ay,
                                      const PointAxis<kShape>& az) {
     constexpr int kN = PointAxis<kShape>::kN;
-    float sx_[kN];
+    const auto load = [&](const float* __restrict__ p, Idx row, float (&v)[kN]) {
+        if constexpr (kRun) {
+            load_run<kN>(p + (row + (Idx)az.p[0]), v);
+        } else {
 #pragma unroll
-    for (int i = 0; i < kN; ++i) {
-        float sy_[kN];
-#pragma unroll
-        for (int j = 0; j < kN; ++j) {
-            const Idx row = (Idx)ax.p[i] * sx + (Idx)ay.p[j] * sy;
-            float v[kN];
-            if constexpr (kRun) {
-                load_run<kN>(f + (row + (Idx)az.p[0]), v);
-            } else {
-#pragma unroll
-                for (int k = 0; k < kN; ++k) v[k] = f[row + (Idx)az.p[k]];
-            }
-            if (fe) {
-                float e[kN];
-                if constexpr (kRun) {
-                    load_run<kN>(fe + (row + (Idx)az.p[0]), e);
-                } else {
-#pragma unroll
-                    for (int k = 0; k < kN; ++k) e[k] = fe[row + (Idx)az.p[k]];
-                }
-#pragma unroll
-                for (int k = 0; k < kN; ++k) v[k] += e[k];
-            }
-            sy_[j] = weighted<kN>(v, az.w);
+            for (int k = 0; k < kN; ++k) v[k] = p[row + (Idx)az.p[k]];
         }
-        sx_[i] = weighted<kN>(ay.w, sy_);
-    }
-    return weighted<kN>(ax.w, sx_);
+    };
+    return stencil_sum<kN, kR>(ax.w, ay.w, az.w, [&](int i, int j, float (&v)[kN]) {
+        const Idx row = (Idx)ax.p[i] * sx + (Idx)ay.p[j] * sy;
+        load(f, row, v);
+        if (fe) {
+            float e[kN];
+            load(fe, row, e);
+#pragma unroll
+            for (int k = 0; k < kN; ++k) v[k] += e[k];
+        }
+    });
 }
 
 template <int kShape, bool kRun, class Idx>
 __device__ inline void gather_six(const PicDesc& d, const FieldPtrs& fp, const PointAxis<kShape> (&c)[3],
                                   const PointAxis<kShape> (&v)[3], float E[3], float B[3]) {
     const Idx sy = (Idx)d.dims[2], sx = (Idx)d.dims[1] * sy;
-    E[0] = gather_point<kShape, kRun, Idx>(fp.E[0], fp.Ee[0], sx, sy, v[0], c[1], c[2]);
-    E[1] = gather_point<kShape, kRun, Idx>(fp.E[1], fp.Ee[1], sx, sy, c[0], v[1], c[2]);
-    E[2] = gather_point<kShape, kRun, Idx>(fp.E[2], fp.Ee[2], sx, sy, c[0], c[1], v[2]);
-    B[0] = gather_point<kShape, kRun, Idx>(fp.B[0], fp.Be[0], sx, sy, c[0], v[1], v[2]);
-    B[1] = gather_point<kShape, kRun, Idx>(fp.B[1], fp.Be[1], sx, sy, v[0], c[1], v[2]);
-    B[2] = gather_point<kShape, kRun, Idx>(fp.B[2], fp.Be[2], sx, sy, v[0], v[1], c[2]);
+    E[0] = gather_point<kShape, kPlain, kRun, Idx>(fp.E[0], fp.Ee[0], sx, sy, v[0], c[1], c[2]);
+    E[1] = gather_point<kShape, kSecond, kRun, Idx>(fp.E[1], fp.Ee[1], sx, sy, c[0], v[1], c[2]);
+    E[2] = gather_point<kShape, kPlain, kRun, Idx>(fp.E[2], fp.Ee[2], sx, sy, c[0], c[1], v[2]);
+    B[0] = gather_point<kShape, kMagnetic, kRun, Idx>(fp.B[0], fp.Be[0], sx, sy, c[0], v[1], v[2]);
+    B[1] = gather_point<kShape, kMagnetic, kRun, Idx>(fp.B[1], fp.Be[1], sx, sy, v[0], c[1], v[2]);
+    B[2] = gather_point<kShape, kMagnetic, kRun, Idx>(fp.B[2], fp.Be[2], sx, sy, v[0], v[1], c[2]);
 }
 
 // The six staggered components (particle_push.py:63-68) at x, any
@@ -516,11 +537,11 @@ struct FieldBox {
 };
 
 // Value of a component whose box of kB^3 nodes is at p, the stencil's first node.
-template <int kB>
+template <int kB, CicRounding kR = kPlain>
 __device__ inline float gather_at(const float* p, const CicAxis& ax, const CicAxis& ay, const CicAxis& az) {
     const float v000 = p[0], v001 = p[1], v010 = p[kB], v011 = p[kB + 1];
     const float v100 = p[kB * kB], v101 = p[kB * kB + 1], v110 = p[kB * kB + kB], v111 = p[kB * kB + kB + 1];
-    return cic_value(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
+    return cic_value<kR>(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
 }
 
 __device__ inline float gather_box(const FieldBox& fb, int c, int a0, int a1, int a2, const CicAxis& ax,
@@ -529,7 +550,7 @@ __device__ inline float gather_box(const FieldBox& fb, int c, int a0, int a1, in
     const float* p = fb.box + c * B * B * B + ((a0 - fb.o[0]) * B + (a1 - fb.o[1])) * B + (a2 - fb.o[2]);
     const float v000 = p[0], v001 = p[1], v010 = p[B], v011 = p[B + 1];
     const float v100 = p[B * B], v101 = p[B * B + 1], v110 = p[B * B + B], v111 = p[B * B + B + 1];
-    return cic_value(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
+    return cic_value<kPlain>(v000, v001, v010, v011, v100, v101, v110, v111, ax, ay, az);
 }
 
 // Per-block LDS: the face-crossing queue and the species constants.

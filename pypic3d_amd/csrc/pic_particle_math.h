@@ -138,9 +138,19 @@ __device__ inline void cross(const float a[3], const float b[3], float o[3]) {
     o[2] = fmaf(a[0], b[1], -(a[1] * b[0]));
 }
 
-// c + a . a
-__device__ inline float plus_square(float c, const float a[3]) {
-    return fmaf(a[2], a[2], fmaf(a[1], a[1], fmaf(a[0], a[0], c)));
+// A product that stays rounded: the empty asm keeps it out of a later sum's fused operation.
+__device__ inline float rounded(float v) {
+    asm("" : "+v"(v));
+    return v;
+}
+
+__device__ inline float dot(const float a[3], const float b[3]) {
+    return fmaf(a[2], b[2], fmaf(a[0], b[0], a[1] * b[1]));
+}
+
+// 1 + a . a
+__device__ inline float one_plus_square(const float a[3]) {
+    return fmaf(a[2], a[2], fmaf(a[1], a[1], fmaf(a[0], a[0], 1.0f)));
 }
 
 // Boris rotation with hardware reciprocal / reciprocal-square-root (1 ulp),
@@ -151,10 +161,11 @@ __device__ inline void boris_push(float v[3], const float E[3], const float B[3]
                                   float C) {
     float um[3], t[3], up[3], s[3], c1[3];
     const float invC2 = __builtin_amdgcn_rcpf(C * C);
+    const float hE[3] = {h * E[0], h * E[1], h * E[2]};
     if (relativistic) {
-        float gamma = __builtin_amdgcn_rsqf(fmaf(-plus_square(0.0f, v), invC2, 1.0f));
-        for (int a = 0; a < 3; ++a) um[a] = fmaf(h, E[a], v[a] * gamma);
-        float igm = __builtin_amdgcn_rsqf(fmaf(plus_square(0.0f, um), invC2, 1.0f));
+        float gamma = __builtin_amdgcn_rsqf(fmaf(-dot(v, v), invC2, 1.0f));
+        for (int a = 0; a < 3; ++a) um[a] = fmaf(v[a], gamma, hE[a]);
+        float igm = __builtin_amdgcn_rsqf(fmaf(dot(um, um), invC2, 1.0f));
         for (int a = 0; a < 3; ++a) t[a] = h * B[a] * igm;
     } else {
         for (int a = 0; a < 3; ++a) {
@@ -164,13 +175,13 @@ __device__ inline void boris_push(float v[3], const float E[3], const float B[3]
     }
     cross(um, t, c1);
     for (int a = 0; a < 3; ++a) up[a] = um[a] + c1[a];
-    float f = 2.0f * __builtin_amdgcn_rcpf(plus_square(1.0f, t));
+    float f = 2.0f * __builtin_amdgcn_rcpf(one_plus_square(t));
     for (int a = 0; a < 3; ++a) s[a] = t[a] * f;
     cross(up, s, c1);
     float nu[3];
-    for (int a = 0; a < 3; ++a) nu[a] = fmaf(h, E[a], um[a] + c1[a]);
+    for (int a = 0; a < 3; ++a) nu[a] = rounded(hE[a]) + (um[a] + c1[a]);
     if (relativistic) {
-        float ing = __builtin_amdgcn_rsqf(fmaf(plus_square(0.0f, nu), invC2, 1.0f));
+        float ing = __builtin_amdgcn_rsqf(fmaf(dot(nu, nu), invC2, 1.0f));
         for (int a = 0; a < 3; ++a) v[a] = nu[a] * ing;
     } else {
         for (int a = 0; a < 3; ++a) v[a] = nu[a];
@@ -183,27 +194,26 @@ __device__ inline void boris_push(float v[3], const float E[3], const float B[3]
 // u_m = (u_e + (u_e.t) t + u_e x t) / (1 + t^2), u = u_m + hE + u_m x t.
 __device__ inline void higuera_cary_push(float v[3], const float E[3], const float B[3], float h, float C) {
     const float invC2 = __builtin_amdgcn_rcpf(C * C);
-    float v2 = v[0] * v[0] + v[1] * v[1] + v[2] * v[2];
-    float gamma0 = __builtin_amdgcn_rsqf(1.0f - v2 * invC2);
+    float gamma0 = __builtin_amdgcn_rsqf(fmaf(-dot(v, v), invC2, 1.0f));
     float ue[3], beta[3], t[3], um[3], c1[3];
     for (int a = 0; a < 3; ++a) {
-        ue[a] = v[a] * gamma0 + h * E[a];
+        ue[a] = fmaf(h, E[a], v[a] * gamma0);
         beta[a] = h * B[a];
     }
-    float b2 = beta[0] * beta[0] + beta[1] * beta[1] + beta[2] * beta[2];
-    float ustar = (ue[0] * beta[0] + ue[1] * beta[1] + ue[2] * beta[2]) / C;
-    float sigma = (1.0f + (ue[0] * ue[0] + ue[1] * ue[1] + ue[2] * ue[2]) * invC2) - b2;
-    float gam = sqrtf(0.5f * (sigma + sqrtf(sigma * sigma + 4.0f * (b2 + ustar * ustar))));
+    float b2 = dot(beta, beta);
+    float ustar = dot(ue, beta) / C;
+    float sigma = fmaf(dot(ue, ue), invC2, 1.0f) - b2;
+    float gam = sqrtf(0.5f * (sigma + sqrtf(fmaf(sigma, sigma, 4.0f * fmaf(ustar, ustar, b2)))));
     float ig = __builtin_amdgcn_rcpf(gam);
     for (int a = 0; a < 3; ++a) t[a] = beta[a] * ig;
-    float s = __builtin_amdgcn_rcpf(1.0f + t[0] * t[0] + t[1] * t[1] + t[2] * t[2]);
-    float uet = ue[0] * t[0] + ue[1] * t[1] + ue[2] * t[2];
+    float s = __builtin_amdgcn_rcpf(one_plus_square(t));
+    float uet = dot(ue, t);
     cross(ue, t, c1);
-    for (int a = 0; a < 3; ++a) um[a] = s * (ue[a] + uet * t[a] + c1[a]);
+    for (int a = 0; a < 3; ++a) um[a] = s * (fmaf(uet, t[a], ue[a]) + c1[a]);
     cross(um, t, c1);
     float nu[3];
-    for (int a = 0; a < 3; ++a) nu[a] = um[a] + h * E[a] + c1[a];
-    float ing = __builtin_amdgcn_rsqf(1.0f + (nu[0] * nu[0] + nu[1] * nu[1] + nu[2] * nu[2]) * invC2);
+    for (int a = 0; a < 3; ++a) nu[a] = fmaf(h, E[a], um[a]) + c1[a];
+    float ing = __builtin_amdgcn_rsqf(fmaf(dot(nu, nu), invC2, 1.0f));
     for (int a = 0; a < 3; ++a) v[a] = nu[a] * ing;
 }
 

@@ -94,7 +94,7 @@ class ElectrodynamicRunner:
         self.direct_min_blocks = 1
         self.sort_lookahead = None      # tile re-sort keys at x + t u; None: t = sort_every * dt / 2
         self.tile_ws, self.direct_fused = None, False
-        self.defer_permute = self.tile_general = False
+        self.defer_permute = self.tile_general = self.direct_general = False
         if tile is not None:
             self.set_tile(tile)
 
@@ -170,7 +170,7 @@ class ElectrodynamicRunner:
                 ev[1].record()
             ev = self._mark("current_fold")
             finish_current(d, self.J, s)
-        elif self.tile and self.direct_fused:
+        elif self.tile and (self.direct_fused or self.direct_general):
             N.call("pic_zero_fields", d, N.p3(self.J), s)
             ev = self._mark("particles")
             if self._pending:
@@ -178,6 +178,10 @@ class ElectrodynamicRunner:
                        N.p3(self.B), self.Ee, self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts),
                        self.direct_min_blocks, N.ptr(self.tile_ws), s)
                 self._pending = False
+            elif self.direct_general:
+                N.call("pic_fused_push_direct_tiled_general", d, self.sp, self._pp(src), N.p3(E), N.p3(self.B),
+                       self.Ee, self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts),
+                       N.ptr(self.tile_ws), s)
             else:
                 N.call("pic_fused_push_direct_tiled", d, self.sp, self._pp(src), N.p3(E), N.p3(self.B), self.Ee,
                        self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts), self.direct_min_blocks,
@@ -257,7 +261,7 @@ class ElectrodynamicRunner:
         self._materialize()
         if tile is None:
             self.tile, self.starts, self.tile_ws, self.direct_fused = None, None, None, False
-            self.defer_permute = False
+            self.defer_permute = self.tile_general = self.direct_general = False
             return
         d = self.desc
         if self.esirkepov and not (d.shape_factor == 1 and all(d.n[a] > 1 for a in range(3))):
@@ -266,8 +270,8 @@ class ElectrodynamicRunner:
             raise ValueError("tile must be 4 or 8")
         self.tile = int(tile)
         self.direct_min_blocks = 4 if self.tile == 4 else 1
-        # direct branch: one fused tile kernel on exact 3-D first-order grids with cells equal to the node
-        # spacing, the separate push / advance / boundary / tiled-deposit kernels otherwise
+        # direct branch: one fused tile kernel on 3-D first-order grids (FP32 anchors on exact ones with cells
+        # equal to the node spacing), the separate push / advance / boundary / deposit kernels otherwise
         self.direct_fused = (not self.esirkepov and d.shape_factor == 1 and all(d.n[a] > 1 for a in range(3))
                              and bool(N.lib().pic_tile_exact_grid(d))
                              and all(d.d[a] == d.sp_c[a] for a in range(3)))
@@ -275,8 +279,10 @@ class ElectrodynamicRunner:
         # the particles through perm (both branches' fused kernels on exact grids)
         self.defer_permute = self.direct_fused or (self.esirkepov and d.variant != 1
                                                    and bool(N.lib().pic_tile_exact_grid(d)))
-        # other grids take the same kernel with FP64 anchors, which reads its slots directly
+        # other grids take the same kernels with FP64 anchors, which read their slots directly
         self.tile_general = self.esirkepov and not bool(N.lib().pic_tile_exact_grid(d))
+        self.direct_general = (not self.esirkepov and not self.direct_fused
+                               and bool(N.lib().pic_tile_general_grid(d)))
         tiles = int(N.lib().pic_tile_count(d, self.tile))
         self.starts = torch.empty(self.S * (tiles + 1) + 1, dtype=torch.int32, device=self.device)
         # the tiled kernel's list of particles for its general route (1 + slots int32)
