@@ -343,11 +343,13 @@ int64_t pic_cg_workspace_bytes(const PicDesc* desc);
  * r = rho/eps + lapl(phi) in FP64, each correction solved by CG with FP32
  * vectors and FP64 dot products.  Stops when the FP64 ||r|| <= max(tol,
  * rtol*||r0||), when a refinement pass no longer halves ||r||, or after
- * max_iter CG iterations in total.  phi in/out (its boundaries applied as
- * _apply_tiled_phi_constant_boundaries does).  Synchronises the host once
- * per refinement pass and once per 32 iterations to read the convergence
- * flag.  iterations (total CG iterations) and residual_norm (final FP64
- * ||r||) optional. */
+ * max_iter CG iterations in total.  Where max_iter leaves CG room to converge
+ * and no axis is longer than 1024 cells, each correction is solved outright by
+ * FP64 transforms instead.  phi in/out (its boundaries applied as
+ * _apply_tiled_phi_constant_boundaries does).  Synchronises the host once per
+ * two direct passes, or once per refinement pass and per 32 iterations, to read
+ * the convergence flag.  iterations (CG iterations, or direct passes) and
+ * residual_norm (final FP64 ||r||) optional. */
 int pic_poisson_cg(const PicDesc* desc, const float* rho, float* phi, double tol, double rtol,
                    int32_t max_iter, void* workspace, int64_t workspace_bytes,
                    int32_t* iterations, double* residual_norm, void* stream);

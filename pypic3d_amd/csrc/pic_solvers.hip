@@ -29,8 +29,20 @@
 // The scalars live on the device; every iteration kernel returns at once when
 // the device `done` flag is set, so the host queues iterations in batches and
 // reads the flag once per batch.
+//
+// Direct passes.  The operator is separable and its eigenvectors along an axis
+// are known (periodic: real Fourier, self neighbour: DCT-II, zero neighbour:
+// DST-I), so a pass that is to converge can be solved outright: three dense
+// transforms, a division by the eigenvalues and three transforms back, in FP64
+// on the matrix cores.  64^3 with the default limits takes two such passes of
+// six 3.4 us launches, where CG takes 448 iterations of five (an electrostatic
+// step with 8 and 8 particles per cell 12.5 -> 1.25 ms).  CG stays for iteration
+// limits that may end it before it has converged (its unconverged potential is
+// then the answer) and for axes whose dense tables would not pay (kMaxDirect).
 #include "pic_common.h"
 
+#include <algorithm>
+#include <cmath>
 #include <cstdio>
 #include <mutex>
 
@@ -58,6 +70,7 @@ enum NeighbourMode : int { NB_PERIODIC = 0, NB_SELF = 1, NB_ZERO = 2 };
 struct CGScalars {
     double rr, pAp, alpha, beta, tol2, rr_true, mean;
     int32_t done, iter, max_iter, pad;
+    double target, prev;      // of the direct passes
 };
 
 // interior-array geometry and the face-neighbour map
@@ -274,6 +287,173 @@ __global__ void cg_p_kernel(int64_t total, const float* __restrict__ r, float* _
         p[t] = r[t] + beta * p[t];
 }
 
+// ---- direct passes ----
+
+constexpr int kMaxDirect = 1024;    // longest axis: 8 MB per table
+
+// Tables of one axis: Q (eigenvectors in columns, orthonormal), its transpose
+// and the eigenvalues of -d^2/dx^2.
+struct AxisTable {
+    int n, mode;
+    double i2;
+    double *q, *qt, *lam;
+};
+
+struct DirectTables {
+    AxisTable a[3];
+};
+
+__global__ void direct_tables_kernel(DirectTables D) {
+    const AxisTable T = D.a[blockIdx.y];
+    const int n = T.n;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (int64_t)n * n;
+         t += (int64_t)gridDim.x * blockDim.x) {
+        const int j = (int)(t / n), k = (int)(t % n);
+        double q, s;      // eigenvector k at node j; lam = 4 s^2 / d^2
+        if (T.mode == NB_PERIODIC) {
+            const int m = (k + 1) / 2;
+            const double x = (double)((2 * (int64_t)m * j) % (2 * n)) / n;        // angle / pi
+            if (k == 0) q = sqrt(1.0 / n);
+            else if (2 * m == n) q = (j & 1) ? -sqrt(1.0 / n) : sqrt(1.0 / n);
+            else q = sqrt(2.0 / n) * ((k & 1) ? cospi(x) : sinpi(x));
+            s = sinpi((double)m / n);
+        } else if (T.mode == NB_SELF) {
+            const double x = (double)(((2 * (int64_t)j + 1) * k) % (4 * n)) / (2 * n);
+            q = k == 0 ? sqrt(1.0 / n) : sqrt(2.0 / n) * cospi(x);
+            s = sinpi(0.5 * k / n);
+        } else {
+            const double x = (double)(((int64_t)(j + 1) * (k + 1)) % (2 * (n + 1))) / (n + 1);
+            q = sqrt(2.0 / (n + 1)) * sinpi(x);
+            s = sinpi(0.5 * (k + 1) / (n + 1));
+        }
+        T.q[t] = q;
+        T.qt[(int64_t)k * n + j] = q;
+        if (j == 0) T.lam[k] = 4.0 * s * s * T.i2;
+    }
+}
+
+// FP64 residual of a direct pass, its mean removed, and the partials of r.r.
+__global__ void direct_residual_kernel(PicDesc d, LapMap M, const float* __restrict__ rho,
+                                       const double* __restrict__ phid, double* __restrict__ r, double* partials,
+                                       double inv_eps, const CGScalars* sc) {
+    int64_t total = (int64_t)M.n[0] * M.n[1] * M.n[2];
+    const double mean = M.singular ? sc->mean : 0.0;
+    double acc = 0.0;
+    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x) {
+        int i, j, k;
+        split(M, t, i, j, k);
+        double rv = (double)rho[fidx(d, i + d.g, j + d.g, k + d.g)] * inv_eps + lapl_at(phid, M, t, i, j, k) - mean;
+        r[t] = rv;
+        acc += rv * rv;
+    }
+    double s = block_sum(acc);
+    if (threadIdx.x == 0) partials[blockIdx.x] = s;
+}
+
+// Ends the passes by the tests of the CG loop: ||r|| at the target, or a pass
+// that did not halve it.  pass counts the corrections made so far.
+__global__ void direct_check_kernel(const double* partials, int nparts, CGScalars* sc, double tol, double rtol,
+                                    int pass) {
+    if (pass > 0 && sc->done) return;
+    double acc = 0.0;
+    for (int b = threadIdx.x; b < nparts; b += blockDim.x) acc += partials[b];
+    const double rr = block_sum(acc);
+    if (threadIdx.x == 0) {
+        const double last = sqrt(rr);
+        if (pass == 0) sc->target = fmax(tol, rtol * last);
+        sc->rr_true = rr;
+        sc->iter = pass;
+        sc->done = !(last > sc->target) || (pass > 0 && !(last < 0.5 * sc->prev)) ? 1 : 0;
+        sc->prev = last;
+    }
+}
+
+// C = A B per batch (blockIdx.z), all row-major FP64: a transform along the
+// last axis has the data as A (rows of it) and the table as B, one along an
+// earlier axis the table as A and the data as B.  A wave owns kW x kW MFMA tiles
+// of 16 x 16, a block 2 x 2 waves; 16 values of the contraction are in LDS at a
+// time and the next 16 in flight.  kDivide: by the sum of the axes' eigenvalues
+// (zero for the constant of a singular operator); kAdd: C += A B.
+enum TransformEnd { kStore, kDivide, kAdd };
+struct Transform {
+    const double *A, *B;
+    double* C;
+    int M, N, K;
+    int64_t lda, ldb, ldc, batch_b, batch_c;
+};
+typedef double v4d __attribute__((ext_vector_type(4)));
+
+template <int kW, int kEnd>
+__global__ __launch_bounds__(kBlock) void transform_kernel(Transform T, LapMap M, DirectTables D, const CGScalars* sc) {
+    constexpr int kT = 32 * kW, kK = 16, kQ = kT * kK / kBlock;
+    __shared__ double As[kK][kT + 1], Bs[kK][kT];
+    if (sc->done) return;
+    const int m0 = blockIdx.y * kT, n0 = blockIdx.x * kT;
+    const double* __restrict__ B = T.B + blockIdx.z * T.batch_b;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int wm = (wave >> 1) * 16 * kW, wn = (wave & 1) * 16 * kW;
+    v4d acc[kW][kW];
+#pragma unroll
+    for (int a = 0; a < kW; ++a)
+#pragma unroll
+        for (int b = 0; b < kW; ++b) acc[a][b] = v4d{0.0, 0.0, 0.0, 0.0};
+    double ra[kQ], rb[kQ];
+    const auto load = [&](int k0) {
+#pragma unroll
+        for (int q = 0; q < kQ; ++q) {
+            const int e = (int)threadIdx.x + q * kBlock;
+            const int am = m0 + e / kK, ak = k0 + e % kK, bk = k0 + e / kT, bn = n0 + e % kT;
+            ra[q] = am < T.M && ak < T.K ? T.A[am * T.lda + ak] : 0.0;
+            rb[q] = bk < T.K && bn < T.N ? B[bk * T.ldb + bn] : 0.0;
+        }
+    };
+    load(0);
+    for (int k0 = 0; k0 < T.K; k0 += kK) {
+#pragma unroll
+        for (int q = 0; q < kQ; ++q) {
+            const int e = (int)threadIdx.x + q * kBlock;
+            As[e % kK][e / kK] = ra[q];
+            Bs[e / kT][e % kT] = rb[q];
+        }
+        __syncthreads();
+        if (k0 + kK < T.K) load(k0 + kK);
+#pragma unroll
+        for (int kk = 0; kk < kK; kk += 4) {
+            double a[kW], b[kW];
+#pragma unroll
+            for (int q = 0; q < kW; ++q) {
+                a[q] = As[kk + (lane >> 4)][wm + 16 * q + (lane & 15)];
+                b[q] = Bs[kk + (lane >> 4)][wn + 16 * q + (lane & 15)];
+            }
+#pragma unroll
+            for (int p = 0; p < kW; ++p)
+#pragma unroll
+                for (int q = 0; q < kW; ++q)
+                    acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[p], b[q], acc[p][q], 0, 0, 0);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int p = 0; p < kW; ++p)
+#pragma unroll
+        for (int q = 0; q < kW; ++q)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int m = m0 + wm + 16 * p + 4 * v + (lane >> 4), n = n0 + wn + 16 * q + (lane & 15);
+                if (m >= T.M || n >= T.N) continue;
+                const int64_t t = blockIdx.z * T.batch_c + m * T.ldc + n;
+                double c = acc[p][q][v];
+                if constexpr (kEnd == kDivide) {
+                    int i, j, k;
+                    split(M, t, i, j, k);
+                    const double lam = D.a[0].lam[i] + D.a[1].lam[j] + D.a[2].lam[k];
+                    c = M.singular && i + j + k == 0 ? 0.0 : c / lam;
+                }
+                if constexpr (kEnd == kAdd) c += T.C[t];
+                T.C[t] = c;
+            }
+}
+
 // phi_d += e (FP64 accumulation of the FP32 correction)
 __global__ void cg_accumulate_kernel(int64_t total, double* __restrict__ phid, const float* __restrict__ e) {
     for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total; t += (int64_t)gridDim.x * blockDim.x)
@@ -412,11 +592,31 @@ int phi_bc(const PicDesc* d, float* f, hipStream_t s) {
 }
 
 struct CGLayout {
-    int64_t phid_off, p_off, r_off, ap_off, e_off, part_off, sc_off, total;
+    int64_t phid_off, p_off, r_off, ap_off, e_off, part_off, sc_off, table_off, total;
 };
 
+// Longest axis and the square root of the operator's condition number.
+bool direct_possible(const LapMap& M, double& kappa) {
+    double top = 0.0, zero = 0.0, low = 0.0;
+    bool active = false;
+    for (int a = 0; a < 3; ++a) {
+        const int n = M.n[a];
+        if (n > kMaxDirect) return false;
+        active = active || n > 1;
+        if (n > 1 || M.mode[a] == NB_ZERO) top += 4.0 * M.i2[a];
+        const double angle = M.mode[a] == NB_ZERO ? 0.5 / (n + 1) : (M.mode[a] == NB_SELF ? 0.5 / n : 1.0 / n);
+        const double s = std::sin(M_PI * angle), lam = 4.0 * s * s * M.i2[a];
+        if (M.mode[a] == NB_ZERO) zero += lam;
+        else if (n > 1 && (low == 0.0 || lam < low)) low = lam;
+    }
+    if (!active) return false;
+    kappa = std::sqrt(top / (zero > 0.0 ? zero : low));
+    return true;
+}
+
 // workspace: phi_d (FP64) and p, r, Ap, e (FP32) over the interior, FP64
-// partial sums, the scalar block
+// partial sums, the scalar block, the axis tables of the direct passes (whose
+// two FP64 arrays lie over p, r and Ap, e)
 CGLayout cg_layout(const PicDesc* d) {
     auto up = [](int64_t b) { return ((b + 255) / 256) * 256; };
     const int64_t n = (int64_t)d->n[0] * d->n[1] * d->n[2];
@@ -428,7 +628,11 @@ CGLayout cg_layout(const PicDesc* d) {
     L.e_off = L.ap_off + up(n * 4);
     L.part_off = L.e_off + up(n * 4);
     L.sc_off = L.part_off + kMaxPartials * 8;
-    L.total = L.sc_off + 256;
+    L.table_off = L.sc_off + 256;
+    L.total = L.table_off;
+    double kappa;
+    if (direct_possible(lap_map(d), kappa))
+        for (int a = 0; a < 3; ++a) L.total += up((int64_t)d->n[a] * (2 * d->n[a] + 1) * 8);
     return L;
 }
 
@@ -474,6 +678,67 @@ int scratch_address(double** out) {
         g_scratch_ptr[dev] = static_cast<double*>(p);
     }
     *out = g_scratch_ptr[dev];
+    return 0;
+}
+
+// One direct pass, phi_d += solution of -lapl e = r: forward along z, y, x, back along x, y, z,
+// between r and tmp.  Axes of one cell have nothing to transform.
+int direct_solve(const LapMap& M, const DirectTables& D, double* r, double* tmp, double* phid, const CGScalars* sc,
+                 hipStream_t s) {
+    int axes[6], n = 0;
+    for (int a = 2; a >= 0; --a)
+        if (M.n[a] > 1) axes[n++] = a;
+    for (int q = n - 1, f = n; q >= 0; --q) axes[f++] = axes[q];
+    double *src = r, *dst = tmp;
+    for (int q = 0; q < 2 * n; ++q) {
+        const int a = axes[q];
+        const bool back = q >= n, last = q == 2 * n - 1, divide = q == n - 1;
+        const AxisTable& X = D.a[a];
+        int64_t inner = 1, outer = 1;
+        for (int b = a + 1; b < 3; ++b) inner *= M.n[b];
+        for (int b = 0; b < a; ++b) outer *= M.n[b];
+        Transform T;
+        int batches = 1;
+        T.C = last ? phid : dst;
+        if (inner == 1) {          // rows of data times the table
+            T.A = src;
+            T.B = back ? X.qt : X.q;
+            T.M = (int)outer;
+            T.N = T.K = X.n;
+            T.lda = T.ldb = T.ldc = X.n;
+            T.batch_b = T.batch_c = 0;
+        } else {                   // the table times columns of data
+            T.A = back ? X.q : X.qt;
+            T.B = src;
+            T.M = T.K = X.n;
+            T.N = (int)inner;
+            T.lda = X.n;
+            T.ldb = T.ldc = inner;
+            T.batch_b = T.batch_c = X.n * inner;
+            batches = (int)outer;
+        }
+        // 64 x 64 tiles where they make a block for every second CU at least; smaller problems
+        // take 32 x 32 tiles to fill the chip
+        const auto grid = [&](int tile) {
+            return dim3((T.N + tile - 1) / tile, (T.M + tile - 1) / tile, batches);
+        };
+        const dim3 g64 = grid(64), g32 = grid(32);
+        const bool wide = (int64_t)g64.x * g64.y * g64.z >= 128;
+#define PIC_TRANSFORM(W, END) \
+    hipLaunchKernelGGL((transform_kernel<W, END>), W == 2 ? g64 : g32, dim3(kBlock), 0, s, T, M, D, sc)
+#define PIC_TRANSFORM_END(END)              \
+    do {                                    \
+        if (wide) PIC_TRANSFORM(2, END);    \
+        else PIC_TRANSFORM(1, END);         \
+    } while (0)
+        if (last) PIC_TRANSFORM_END(kAdd);
+        else if (divide) PIC_TRANSFORM_END(kDivide);
+        else PIC_TRANSFORM_END(kStore);
+#undef PIC_TRANSFORM_END
+#undef PIC_TRANSFORM
+        PIC_CHECK_LAUNCH();
+        std::swap(src, dst);
+    }
     return 0;
 }
 
@@ -523,7 +788,54 @@ int pic_poisson_cg(const PicDesc* desc, const float* rho, float* phi, double tol
     CGScalars host;
     int total_iter = 0;
     double target = tol, prev = 0.0, last = 0.0;
-    for (int outer = 0; outer < kMaxOuter; ++outer) {
+    // CG reduces the residual by e^-2 in kappa iterations at least: 16 kappa cover the FP64 range and the restarts
+    // of its passes (64^3 periodic: 448 iterations, 12.7 kappa).  Under smaller limits CG itself runs
+    double kappa = 0.0;
+    const bool direct = direct_possible(M, kappa) && (double)max_iter >= 16.0 * kappa + 64.0;
+    if (direct) {
+        double *r64 = reinterpret_cast<double*>(base + Lw.p_off), *t64 = reinterpret_cast<double*>(base + Lw.ap_off);
+        DirectTables D;
+        int64_t off = Lw.table_off;
+        int longest = 1;
+        for (int a = 0; a < 3; ++a) {
+            const int n = M.n[a];
+            double* q = reinterpret_cast<double*>(base + off);
+            D.a[a] = AxisTable{n, M.mode[a], M.i2[a], q, q + (int64_t)n * n, q + 2 * (int64_t)n * n};
+            off += (((int64_t)n * (2 * n + 1) * 8 + 255) / 256) * 256;
+            longest = std::max(longest, n);
+        }
+        hipLaunchKernelGGL(direct_tables_kernel, dim3(grid_1d((int64_t)longest * longest, kBlock), 3), dim3(kBlock), 0,
+                           s, D);
+        PIC_CHECK_LAUNCH();
+        const auto check = [&](int pass) {
+            if (M.singular) {
+                hipLaunchKernelGGL(cg_residual_sum_kernel, dim3(nb), dim3(kBlock), 0, s, *desc, M, rho, phid, partials,
+                                   inv_eps);
+                hipLaunchKernelGGL(cg_mean_kernel, dim3(1), dim3(kBlock), 0, s, partials, nb, sc,
+                                   1.0 / (double)interior);
+            }
+            hipLaunchKernelGGL(direct_residual_kernel, dim3(nb), dim3(kBlock), 0, s, *desc, M, rho, phid, r64, partials,
+                               inv_eps, sc);
+            hipLaunchKernelGGL(direct_check_kernel, dim3(1), dim3(kBlock), 0, s, partials, nb, sc, tol, rtol, pass);
+        };
+        // one pass brings the residual to the rounding of FP64, the second to its floor: both are
+        // queued before the flag is read, the second returning at once if the first was enough
+        check(0);
+        int pass = 0;
+        do {
+            for (int q = 0; q < 2; ++q) {
+                rc = direct_solve(M, D, r64, t64, phid, sc, s);
+                if (rc) return rc;
+                check(++pass);
+            }
+            PIC_CHECK_LAUNCH();
+            rc = read_scalars(&host, sc, s);
+            if (rc) return rc;
+        } while (!host.done && pass < kMaxOuter);
+        total_iter = host.iter;
+        last = sqrt(host.rr_true);
+    }
+    for (int outer = 0; !direct && outer < kMaxOuter; ++outer) {
         if (M.singular) {
             hipLaunchKernelGGL(cg_residual_sum_kernel, dim3(nb), dim3(kBlock), 0, s, *desc, M, rho, phid, partials,
                                inv_eps);

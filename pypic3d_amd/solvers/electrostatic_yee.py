@@ -6,8 +6,10 @@ vectors and FP64 dot products (mixed-precision iterative refinement).  It
 stops at the reference's test ||r|| <= tol (absolute, default 1e-12) on the
 FP64 residual, optionally relaxed to ``rtol * ||r0||``, when a refinement pass
 no longer halves ||r|| (the FP64 rounding floor of a large grid), or after
-``max_iter`` CG iterations in total.  ``last_solve_info`` holds the iteration
-count and final FP64 residual norm of the most recent solve.
+``max_iter`` CG iterations in total.  Where ``max_iter`` leaves CG room to
+converge and no axis exceeds 1024 cells, each correction is solved outright by
+FP64 transforms.  ``last_solve_info`` holds the iteration count (CG iterations,
+or direct passes) and final FP64 residual norm of the most recent solve.
 """
 
 from __future__ import annotations
