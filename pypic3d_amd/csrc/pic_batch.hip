@@ -18,7 +18,7 @@
 // barriers between the passes left three quarters of the chip idle at 64
 // members (647 us per step of 64 members of up to 256 x 32 cells).
 #include "pic_field_ops.h"
-#include "pic_fused_block.h"
+#include "pic_planar.h"
 
 namespace {
 
@@ -61,8 +61,53 @@ struct BatchParticleArgs {
     float* J[3];
 };
 
-// Each work item runs fused_block_boxed (J accumulated in an LDS box sized to
-// the item's particles).
+// A member's table entry as constant memory: the kernels do not write the
+// table, and without saying so each of its values is loaded again, by vector
+// loads, after every store.
+__device__ inline const PicBatchSim& member(const PicBatchSim* sims, int sim) {
+    typedef const __attribute__((address_space(4))) PicBatchSim ConstSim;
+    return *(const PicBatchSim*)((ConstSim*)(sims + __builtin_amdgcn_readfirstlane(sim)));
+}
+
+// Whether any of the block's work items (every gridDim.x-th) is left by the planar kernel.
+__device__ inline bool any_item(const PicBatchSim* __restrict__ sims, const int32_t* __restrict__ work,
+                                int32_t n_work) {
+    bool any = false;
+    for (int64_t w = blockIdx.x + (int64_t)threadIdx.x * gridDim.x; w < n_work; w += (int64_t)kThreads * gridDim.x)
+        any = any || !planar_covers(sims[work[2 * w]].desc);
+    return __syncthreads_or(any) != 0;
+}
+
+// The items of first-order 1-D and 2-D members, a block each: the chunks of planar_kernel.
+template <int kRounds>
+__global__ __launch_bounds__(kPlanarBlock, 2) void batch_planar_kernel(const PicBatchSim* __restrict__ sims,
+                                                                   const int32_t* __restrict__ work, int32_t n_work,
+                                                                   BatchParticleArgs args) {
+    constexpr int kP = kRounds == 2 ? 1 : 2, kChunk = kPlanarBlock * kP;
+    __shared__ PlanarShared<kP, kPlanarBlock> sh;
+    const int32_t w = blockIdx.x;
+    const PicBatchSim& bs = member(sims, work[2 * w]);
+    const PicDesc& d = bs.desc;
+    const int kind = fused_kind(d);
+    if (kind == 1 || kind == 2) {
+        const int64_t poff = bs.particle_offset, foff = bs.field_offset;
+        const int64_t n = (int64_t)bs.species.count * bs.species.slots;
+        const PicParticles in = offset_particles(args.in, poff);
+        const PicParticles out = offset_particles(args.out, poff);
+        const FieldPtrs fp = batch_field_ptrs(args.E, args.B, foff);
+        float* const J[3] = {args.J[0] + foff, args.J[1] + foff, args.J[2] + foff};
+        const bool vec_ok = groups_aligned(in, out);
+        for (int r = 0; r < kThreads * kRounds / kChunk; ++r) {
+            const uint32_t base = (uint32_t)work[2 * w + 1] * (uint32_t)(kThreads * kRounds) + (uint32_t)(r * kChunk);
+            if (base >= n) break;
+            if (kind == 2) planar_chunk<2, kP, kPlanarBlock>(d, bs.species, in, fp, out, J, n, base, vec_ok, sh);
+            else planar_chunk<1, kP, kPlanarBlock>(d, bs.species, in, fp, out, J, n, base, vec_ok, sh);
+        }
+    }
+}
+
+// The other items: fused_block_boxed (J accumulated in an LDS box sized to the
+// item's particles).
 template <int kRounds>
 __global__ __launch_bounds__(kThreads, 1) void batch_fused_kernel(const PicBatchSim* __restrict__ sims,
                                                                   const int32_t* __restrict__ work, int32_t n_work,
@@ -70,11 +115,13 @@ __global__ __launch_bounds__(kThreads, 1) void batch_fused_kernel(const PicBatch
     __shared__ FusedShared<kRounds> sh;
     __shared__ float box[kRangeBoxCap];
     __shared__ int bmin[3], bmax[3];
+    if (!any_item(sims, work, n_work)) return;
     for (int32_t w = blockIdx.x; w < n_work; w += gridDim.x) {
         const int sim = work[2 * w];
         const uint32_t blk = (uint32_t)work[2 * w + 1];
         const PicBatchSim& bs = sims[sim];
         const PicDesc& d = bs.desc;
+        if (planar_covers(d)) continue;
         const int64_t poff = bs.particle_offset, foff = bs.field_offset;
         const int64_t n = (int64_t)bs.species.count * bs.species.slots;
         const PicParticles in = offset_particles(args.in, poff);
@@ -184,10 +231,13 @@ int pic_batch_fused_push_esirkepov(const PicBatchSim* sims, const int32_t* work,
     hipStream_t st = as_stream(stream);
     const int g = grid < n_work ? grid : n_work;
     if (rounds == 2) {
+        hipLaunchKernelGGL(batch_planar_kernel<2>, dim3(n_work), dim3(kPlanarBlock), 0, st, sims, work, n_work, args);
         hipLaunchKernelGGL(batch_fused_kernel<2>, dim3(g), dim3(kThreads), 0, st, sims, work, n_work, args);
     } else if (rounds == 4) {
+        hipLaunchKernelGGL(batch_planar_kernel<4>, dim3(n_work), dim3(kPlanarBlock), 0, st, sims, work, n_work, args);
         hipLaunchKernelGGL(batch_fused_kernel<4>, dim3(g), dim3(kThreads), 0, st, sims, work, n_work, args);
     } else {
+        hipLaunchKernelGGL(batch_planar_kernel<8>, dim3(n_work), dim3(kPlanarBlock), 0, st, sims, work, n_work, args);
         hipLaunchKernelGGL(batch_fused_kernel<8>, dim3(g), dim3(kThreads), 0, st, sims, work, n_work, args);
     }
     PIC_CHECK_LAUNCH();

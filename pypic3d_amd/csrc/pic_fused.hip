@@ -6,6 +6,7 @@
 
 #include "pic_exact_grid.h"
 #include "pic_fused_block.h"
+#include "pic_planar.h"
 
 namespace {
 
@@ -92,28 +93,6 @@ __global__ __launch_bounds__(kThreads, kMinBlocks) void fused_tiled_kernel(PicDe
     }
 }
 
-// Periodic wrap of wrap_periodic_position (grid_and_stencil.py:14-35) with
-// the one-period cases done without fmod (fmod(s, W) = s - W exactly for
-// W <= s < 2W, and = s for -W < s < 0); anything else takes the general form.
-__device__ inline void periodic_wrap(double wind, double& x) {
-    const double half = 0.5 * wind;
-    if (x >= half || x < -half) {
-        const double s = x + half;
-        double m;
-        if (s >= wind && s < 2.0 * wind) {
-            m = s - wind;
-        } else if (s < 0.0 && s > -wind) {
-            m = s + wind;
-        } else {
-            m = fmod(s, wind);
-            if (m != 0.0 && ((m < 0.0) != (wind < 0.0))) m += wind;
-        }
-        double w = m - half;
-        if (w == -half && x >= half) w = half;
-        x = w;
-    }
-}
-
 // One particle of the tile kernel through the general route: global gather
 // with FP64 anchors, push, 3-slot (or 5-slot) Esirkepov deposit, position
 // update, boundaries and store.  Run by fused_tile_rare_kernel for the rare
@@ -175,11 +154,6 @@ __device__ inline void tile_particle_general(const PicDesc& d, const SpeciesK& k
     out.active[i] = act ? 1 : 0;
 }
 
-// A block-uniform value computed by vector instructions, moved to a scalar register.
-__device__ inline float uniform(float v) {
-    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
-}
-
 __device__ inline void rare_push(int32_t* rare, int64_t i) {
     const int p = atomicAdd(rare, 1);
     rare[1 + p] = (int32_t)i;
@@ -190,11 +164,6 @@ __device__ inline void rare_push(int32_t* rare, int64_t i) {
 // 8-cell tiles keep FP32, whose box leaves room for two blocks per CU.
 template <int kT>
 using BoxSum = std::conditional_t<kT == 4, double, float>;
-
-template <class T>
-__device__ inline void box_add(T* p, float v) {
-    unsafeAtomicAdd(p, (T)v);
-}
 
 // Face-crossing deposit (the 54 terms of crossing_deposit) straight into the
 // LDS box when the particle's 3x3x3 frame lies inside it: one base address,
@@ -240,88 +209,6 @@ __device__ inline void flush_moments(T* p, const float m[12]) {
         box_add(p + c * kB3 + sp, v10);
         box_add(p + c * kB3 + sp + sq, m[4 * c + 3]);
         __builtin_amdgcn_sched_barrier(0);   // bound the live FP64 values to one component
-    }
-}
-
-// A thread's group of kP consecutive slots from s0, loaded at once: one kP-wide
-// vector load per plane where the group lies inside [begin, end) and the planes
-// are aligned (`full`; the lanes of a wave then read contiguous memory, and all
-// loads share one round trip).  Slots outside the range are inactive.
-template <int kP, bool kGather>
-__device__ inline void load_group(const PicParticles& in, const int32_t* __restrict__ gather, int64_t s0,
-                                  int64_t begin, int64_t end, bool full, float (&PX)[3][kP], float (&PU)[3][kP],
-                                  uint32_t& pact) {
-    pact = 0u;
-    if (!kGather && full) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            load_vec<kP>(in.x[a] + s0, PX[a]);
-            load_vec<kP>(in.u[a] + s0, PU[a]);
-        }
-        pact = *reinterpret_cast<const uint32_t*>(in.active + s0);
-    } else if (kGather && full) {
-        // slot i's input is in.*[gather[i]]: the permutation of a re-bin,
-        // applied by this launch while it reads.  The flags are loaded
-        // first and combined only after every load has been issued (the
-        // scheduling barrier keeps the combination from being hoisted
-        // between the loads, where each use of a flag would wait for all
-        // loads issued before it)
-        float gf[kP];
-        load_vec<kP>(reinterpret_cast<const float*>(gather + s0), gf);
-        uint32_t ab[kP];
-#pragma unroll
-        for (int j = 0; j < kP; ++j) ab[j] = in.active[__float_as_int(gf[j])];
-#pragma unroll
-        for (int j = 0; j < kP; ++j) {
-            const int64_t src = __float_as_int(gf[j]);
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                PX[a][j] = in.x[a][src];
-                PU[a][j] = in.u[a][src];
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int j = 0; j < kP; ++j) pact |= (ab[j] != 0u ? 1u : 0u) << (8 * j);
-    } else {
-#pragma unroll
-        for (int j = 0; j < kP; ++j) {
-            const int64_t i = s0 + j;
-            const bool inr = i >= begin && i < end;
-            const int64_t src = kGather ? (inr ? (int64_t)gather[i] : 0) : i;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                PX[a][j] = inr ? in.x[a][src] : 0.0f;
-                PU[a][j] = inr ? in.u[a][src] : 0.0f;
-            }
-            pact |= (inr && in.active[src] != 0 ? 1u : 0u) << (8 * j);
-        }
-    }
-}
-
-// The group's outputs, likewise.
-template <int kP>
-__device__ inline void store_group(const PicParticles& out, int64_t s0, int64_t begin, int64_t end, bool full,
-                                   const float (&PX)[3][kP], const float (&PU)[3][kP], uint32_t oact) {
-    if (full) {
-#pragma unroll
-        for (int a = 0; a < 3; ++a) {
-            store_vec<kP>(out.x[a] + s0, PX[a]);
-            store_vec<kP>(out.u[a] + s0, PU[a]);
-        }
-        *reinterpret_cast<uint32_t*>(out.active + s0) = oact;
-    } else {
-#pragma unroll
-        for (int j = 0; j < kP; ++j) {
-            const int64_t i = s0 + j;
-            if (i < begin || i >= end) continue;
-#pragma unroll
-            for (int a = 0; a < 3; ++a) {
-                out.x[a][i] = PX[a][j];
-                out.u[a][i] = PU[a][j];
-            }
-            out.active[i] = (uint8_t)((oact >> (8 * j)) & 0xffu);
-        }
     }
 }
 
@@ -926,8 +813,18 @@ __global__ __launch_bounds__(kThreads) void fused_direct_rare_kernel(PicDesc d, 
     }
 }
 
-// Slot-ordered launch for 1-D and 2-D first-order runs (and the general
-// path): each block accumulates J in an LDS box sized to its particles.
+// 1-D and 2-D first-order runs: a chunk of slots per block.
+template <int kDims, int kP, int kBlk>
+__global__ __launch_bounds__(kBlk, 1024 / kBlk) void planar_kernel(PicDesc d, PicSpecies sp, PicParticles in, FieldPtrs fp,
+                                                             PicParticles out, float* Jx, float* Jy, float* Jz,
+                                                             int64_t n, int vec_ok) {
+    __shared__ PlanarShared<kP, kBlk> sh;
+    float* const J[3] = {Jx, Jy, Jz};
+    planar_chunk<kDims, kP, kBlk>(d, sp, in, fp, out, J, n, blockIdx.x * (uint32_t)(kBlk * kP), vec_ok != 0, sh);
+}
+
+// Slot-ordered launch of the general path (any shape and reduced axes): each
+// block accumulates J in an LDS box sized to its particles.
 template <int kRounds>
 __global__ __launch_bounds__(kThreads, 1) void fused_boxed_kernel(PicDesc d, PicSpecies sp, PicParticles in,
                                                                   FieldPtrs fp, PicParticles out, float* Jx,
@@ -972,6 +869,19 @@ int pic_fused_push_esirkepov(const PicDesc* desc, const PicSpecies* sp, const Pi
             case 5: PIC_FUSED_LAUNCH(3, 8, 3); break;
             default: PIC_FUSED_LAUNCH(3, 4, 1); break;
         }
+    } else if (kind != 0 && planar_covers(*desc)) {
+        // chunks of 1024 slots amortise ranges and boxes once they still make four blocks a CU; smaller
+        // sets take 256, for more blocks (262k slots: 1024 of them, all resident at once)
+        const bool large = n >= (int64_t)1 << 20;
+        const int vec_ok = groups_aligned(*in, *out);
+#define PIC_PLANAR(DIMS, P, BLK)                                                                                  \
+    hipLaunchKernelGGL((planar_kernel<DIMS, P, BLK>), dim3(grid_1d(n, BLK * P)), dim3(BLK), 0, st, *desc, *sp, *in, \
+                       fp, *out, J[0], J[1], J[2], n, vec_ok)
+        if (kind == 2 && large) PIC_PLANAR(2, 2, kPlanarBlock);
+        else if (kind == 2) PIC_PLANAR(2, 1, kThreads);
+        else if (large) PIC_PLANAR(1, 2, kPlanarBlock);
+        else PIC_PLANAR(1, 1, kThreads);
+#undef PIC_PLANAR
     } else {
         hipLaunchKernelGGL(fused_boxed_kernel<4>, dim3(grid_1d(n, kThreads * 4)), dim3(kThreads), 0, st, *desc, *sp,
                            *in, fp, *out, J[0], J[1], J[2], n);
@@ -979,17 +889,6 @@ int pic_fused_push_esirkepov(const PicDesc* desc, const PicSpecies* sp, const Pi
 #undef PIC_FUSED_LAUNCH
     PIC_CHECK_LAUNCH();
     return 0;
-}
-
-// Vector loads and stores of a thread's slot group need 16-byte aligned planes.
-static int groups_aligned(const PicParticles* in, const PicParticles* out, const int32_t* gather) {
-    int ok = 1;
-    for (int a = 0; a < 3; ++a)
-        ok &= ((((uintptr_t)out->x[a]) | ((uintptr_t)out->u[a]) | ((uintptr_t)in->x[a]) |
-                ((uintptr_t)in->u[a])) & 15u) == 0;
-    ok &= ((((uintptr_t)out->active) | ((uintptr_t)in->active)) & 3u) == 0;
-    ok &= (((uintptr_t)gather) & 15u) == 0;
-    return ok;
 }
 
 static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
@@ -1020,7 +919,7 @@ static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const P
     PIC_REQUIRE(blocks < ((int64_t)1 << 31));
     hipStream_t st = as_stream(stream);
     FieldPtrs fp = make_fields(E, B, E_ext, B_ext);
-    const int vec_ok = groups_aligned(in, out, gather);
+    const int vec_ok = groups_aligned(*in, *out, gather);
     hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, st, workspace);
     const SpeciesTable stab = species_table(*desc, *sp);
     bool all = true;
@@ -1096,7 +995,7 @@ static void launch_tile_esirkepov(const PicDesc* desc, const PicSpecies* sp, con
                                   const int32_t* starts, const TileGeom& tg, const TileGrid& grid, bool exact,
                                   int32_t* workspace, const int32_t* gather, int64_t blocks,
                                   hipStream_t st) {
-    const int vec_ok = groups_aligned(in, out, gather);
+    const int vec_ok = groups_aligned(*in, *out, gather);
     hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, st, workspace);
     const SpeciesTable stab = species_table(*desc, *sp);
     bool all = true;

@@ -396,19 +396,25 @@ struct BoxSink {
     }
 };
 
+template <class T>
+__device__ inline void box_add(T* p, float v) {
+    unsafeAtomicAdd(p, (T)v);
+}
+
 // LDS box with per-axis extents e[] from origin o[] (array indices), three
 // components; used when a block's particles cover a small, data-dependent
 // range of cells.  Nodes outside (or `on` false) go to the global arrays.
+template <class T>
 struct RangeBoxSink {
     float* J[3];
-    float* box;
+    T* box;
     int o[3], e[3];
     bool on;
     __device__ inline void add(const PicDesc& d, int c, int i, int j, int k, float v) const {
         if (v == 0.0f) return;
         const int bi = i - o[0], bj = j - o[1], bk = k - o[2];
         if (on && (unsigned)bi < (unsigned)e[0] && (unsigned)bj < (unsigned)e[1] && (unsigned)bk < (unsigned)e[2])
-            atomicAdd(&box[((c * e[0] + bi) * e[1] + bj) * e[2] + bk], v);
+            box_add(&box[((c * e[0] + bi) * e[1] + bj) * e[2] + bk], v);
         else
             deposit_at(J[c], d, i, j, k, v);
     }
@@ -981,7 +987,7 @@ __device__ inline void fused_block_boxed(const PicDesc& d, const PicSpecies& sp,
         }
     }
     __syncthreads();
-    RangeBoxSink sink;
+    RangeBoxSink<float> sink;
     for (int c = 0; c < 3; ++c) sink.J[c] = J[c];
     sink.box = box;
     sink.on = bmax[0] >= bmin[0];
@@ -1083,6 +1089,126 @@ __device__ inline void flush_current_box(const PicDesc& d, const int o[3], const
             if (v != 0.0f) atomic_add_f32(J[c] + off[q], v);
         }
     }
+}
+
+// Periodic wrap of wrap_periodic_position (grid_and_stencil.py:14-35) with
+// the one-period cases done without fmod (fmod(s, W) = s - W exactly for
+// W <= s < 2W, and = s for -W < s < 0); anything else takes the general form.
+__device__ inline void periodic_wrap(double wind, double& x) {
+    const double half = 0.5 * wind;
+    if (x >= half || x < -half) {
+        const double s = x + half;
+        double m;
+        if (s >= wind && s < 2.0 * wind) {
+            m = s - wind;
+        } else if (s < 0.0 && s > -wind) {
+            m = s + wind;
+        } else {
+            m = fmod(s, wind);
+            if (m != 0.0 && ((m < 0.0) != (wind < 0.0))) m += wind;
+        }
+        double w = m - half;
+        if (w == -half && x >= half) w = half;
+        x = w;
+    }
+}
+
+// A block-uniform value computed by vector instructions, moved to a scalar register.
+__device__ inline float uniform(float v) {
+    return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v)));
+}
+
+// A thread's group of kP consecutive slots from s0, loaded at once: one kP-wide
+// vector load per plane where the group lies inside [begin, end) and the planes
+// are aligned (`full`; the lanes of a wave then read contiguous memory, and all
+// loads share one round trip).  Slots outside the range are inactive.
+template <int kP, bool kGather>
+__device__ inline void load_group(const PicParticles& in, const int32_t* __restrict__ gather, int64_t s0,
+                                  int64_t begin, int64_t end, bool full, float (&PX)[3][kP], float (&PU)[3][kP],
+                                  uint32_t& pact) {
+    pact = 0u;
+    if (kP > 1 && !kGather && full) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            load_vec<kP>(in.x[a] + s0, PX[a]);
+            load_vec<kP>(in.u[a] + s0, PU[a]);
+        }
+        if constexpr (kP == 4) pact = *reinterpret_cast<const uint32_t*>(in.active + s0);
+        else pact = *reinterpret_cast<const uint16_t*>(in.active + s0);
+    } else if (kP > 1 && kGather && full) {
+        // slot i's input is in.*[gather[i]]: the permutation of a re-bin,
+        // applied by this launch while it reads.  The flags are loaded
+        // first and combined only after every load has been issued (the
+        // scheduling barrier keeps the combination from being hoisted
+        // between the loads, where each use of a flag would wait for all
+        // loads issued before it)
+        float gf[kP];
+        load_vec<kP>(reinterpret_cast<const float*>(gather + s0), gf);
+        uint32_t ab[kP];
+#pragma unroll
+        for (int j = 0; j < kP; ++j) ab[j] = in.active[__float_as_int(gf[j])];
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+            const int64_t src = __float_as_int(gf[j]);
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                PX[a][j] = in.x[a][src];
+                PU[a][j] = in.u[a][src];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < kP; ++j) pact |= (ab[j] != 0u ? 1u : 0u) << (8 * j);
+    } else {
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+            const int64_t i = s0 + j;
+            const bool inr = i >= begin && i < end;
+            const int64_t src = kGather ? (inr ? (int64_t)gather[i] : 0) : i;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                PX[a][j] = inr ? in.x[a][src] : 0.0f;
+                PU[a][j] = inr ? in.u[a][src] : 0.0f;
+            }
+            pact |= (inr && in.active[src] != 0 ? 1u : 0u) << (8 * j);
+        }
+    }
+}
+
+// The group's outputs, likewise.
+template <int kP>
+__device__ inline void store_group(const PicParticles& out, int64_t s0, int64_t begin, int64_t end, bool full,
+                                   const float (&PX)[3][kP], const float (&PU)[3][kP], uint32_t oact) {
+    if (full) {
+#pragma unroll
+        for (int a = 0; a < 3; ++a) {
+            store_vec<kP>(out.x[a] + s0, PX[a]);
+            store_vec<kP>(out.u[a] + s0, PU[a]);
+        }
+        if constexpr (kP == 4) *reinterpret_cast<uint32_t*>(out.active + s0) = oact;
+        else *reinterpret_cast<uint16_t*>(out.active + s0) = (uint16_t)oact;
+    } else {
+#pragma unroll
+        for (int j = 0; j < kP; ++j) {
+            const int64_t i = s0 + j;
+            if (i < begin || i >= end) continue;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                out.x[a][i] = PX[a][j];
+                out.u[a][i] = PU[a][j];
+            }
+            out.active[i] = (uint8_t)((oact >> (8 * j)) & 0xffu);
+        }
+    }
+}
+
+// Vector loads and stores of a thread's slot group need 16-byte aligned planes.
+__host__ __device__ inline bool groups_aligned(const PicParticles& in, const PicParticles& out,
+                                               const int32_t* gather = nullptr) {
+    uintptr_t planes = (uintptr_t)gather, flags = (uintptr_t)in.active | (uintptr_t)out.active;
+    for (int a = 0; a < 3; ++a)
+        planes |= (uintptr_t)in.x[a] | (uintptr_t)in.u[a] | (uintptr_t)out.x[a] | (uintptr_t)out.u[a];
+    return (planes & 15u) == 0 && (flags & 3u) == 0;
 }
 
 }  // namespace
