@@ -99,6 +99,10 @@ int pic_filter_bilinear(const PicDesc* desc, const float* in, float* out, void* 
  * nonzero, tangential E zero on the conducting walls (first_order_yee.py:76-92);
  * those walls alone, in place.  Guard cells of in must be refreshed. */
 int pic_zero_fields(const PicDesc* desc, float* const f[3], void* stream);
+/* flags[0] = 1 where any value of a's components is not zero, else 0; flags[1]
+ * likewise of b's. */
+int pic_any_nonzero(const PicDesc* desc, const float* const a[3], const float* const b[3], int32_t* flags,
+                    void* stream);
 int pic_finish_current(const PicDesc* desc, float* const f[3], int bc_type, void* stream);
 int pic_filter_refresh(const PicDesc* desc, const float* const in[3], float* const out[3], int bilinear,
                        double alpha, int bc_type, int walls, void* stream);
@@ -404,6 +408,8 @@ int pic_constant_boundary_f64(const PicDesc* desc, double* field, int axis, void
 int pic_filter_digital_f64(const PicDesc* desc, const double* in, double* out, double alpha, void* stream);
 int pic_filter_bilinear_f64(const PicDesc* desc, const double* in, double* out, void* stream);
 int pic_zero_fields_f64(const PicDesc* desc, double* const f[3], void* stream);
+int pic_any_nonzero_f64(const PicDesc* desc, const double* const a[3], const double* const b[3], int32_t* flags,
+                        void* stream);
 int pic_finish_current_f64(const PicDesc* desc, double* const f[3], int bc_type, void* stream);
 int pic_filter_refresh_f64(const PicDesc* desc, const double* const in[3], double* const out[3], int bilinear,
                            double alpha, int bc_type, int walls, void* stream);

@@ -70,6 +70,8 @@ SIGNATURES = {
     "pic_filter_digital": (c_int, [DP, c_vp, c_vp, c_dbl, c_vp]),
     "pic_filter_bilinear": (c_int, [DP, c_vp, c_vp, c_vp]),
     "pic_zero_fields": (c_int, [DP, P3, c_vp]),
+    "pic_any_nonzero": (c_int, [DP, P3, P3, c_vp, c_vp]),
+    "pic_any_nonzero_f64": (c_int, [DP, P3, P3, c_vp, c_vp]),
     "pic_finish_current": (c_int, [DP, P3, c_int, c_vp]),
     "pic_filter_refresh": (c_int, [DP, P3, P3, c_int, c_dbl, c_int, c_int, c_vp]),
     "pic_conducting_walls": (c_int, [DP, P3, c_vp]),

@@ -7,6 +7,8 @@
 // input arrays are never modified -- the reference is functional.
 #include "pic_field_ops.h"
 
+#include <algorithm>
+
 namespace {
 
 using namespace pic;
@@ -320,6 +322,43 @@ bool desc_ok(const PicDesc* d) {
     return true;
 }
 
+// flags[0], flags[1]: whether any value of f[0..2], of f[3..5] is not zero (NaN is not).  flags are cleared before.
+template <class T>
+struct Six {
+    const T* f[6];
+};
+
+template <class T>
+__global__ void any_nonzero_kernel(Six<T> p, int64_t n, int32_t* flags) {
+    bool any[2] = {false, false};
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+#pragma unroll
+        for (int c = 0; c < 6; ++c) any[c / 3] = any[c / 3] | (p.f[c][i] != (T)0);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+        if (__any(any[q]) && (threadIdx.x & 63) == 0) flags[q] = 1;
+}
+
+__global__ void clear_flags_kernel(int32_t* flags) { flags[threadIdx.x] = 0; }
+
+template <class T>
+int any_nonzero_t(const PicDesc* desc, const T* const a[3], const T* const b[3], int32_t* flags, hipStream_t s) {
+    PIC_REQUIRE(desc_ok(desc) && a && b && flags);
+    Six<T> p;
+    for (int c = 0; c < 3; ++c) {
+        PIC_REQUIRE(a[c] && b[c]);
+        p.f[c] = a[c];
+        p.f[3 + c] = b[c];
+    }
+    const int64_t n = field_size(*desc);
+    hipLaunchKernelGGL(clear_flags_kernel, dim3(1), dim3(2), 0, s, flags);
+    const int64_t blocks = std::min<int64_t>((n + 1023) / 1024, 2048);
+    hipLaunchKernelGGL(any_nonzero_kernel<T>, dim3((unsigned)blocks), dim3(256), 0, s, p, n, flags);
+    PIC_CHECK_LAUNCH();
+    return 0;
+}
+
 }  // namespace
 
 // Host-side launch sequences, for the FP32 (float) and FP64 (double) fields.
@@ -578,6 +617,16 @@ int pic_zero_fields(const PicDesc* desc, float* const f[3], void* stream) {
 
 int pic_zero_fields_f64(const PicDesc* desc, double* const f[3], void* stream) {
     return zero_fields_t(desc, f, as_stream(stream));
+}
+
+int pic_any_nonzero(const PicDesc* desc, const float* const a[3], const float* const b[3], int32_t* flags,
+                    void* stream) {
+    return any_nonzero_t(desc, a, b, flags, as_stream(stream));
+}
+
+int pic_any_nonzero_f64(const PicDesc* desc, const double* const a[3], const double* const b[3], int32_t* flags,
+                        void* stream) {
+    return any_nonzero_t(desc, a, b, flags, as_stream(stream));
 }
 
 int pic_finish_current(const PicDesc* desc, float* const f[3], int bc_type, void* stream) {

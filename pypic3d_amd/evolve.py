@@ -8,7 +8,8 @@ the individual kernels in the reference's order.  float64 particles and
 fields run the FP64 path (the reference's precision): the same sequence with
 the FP64 kernels, the Esirkepov branch as separate push, deposit, advance and
 boundary launches.  Inputs are never modified; new tensors are returned.
-External fields that are all zero are skipped (their sum is the identity).
+External fields that are all zero are skipped in large sets (their sum is the
+identity).
 """
 
 from __future__ import annotations
@@ -24,19 +25,28 @@ from .particles.particle_class import TiledParticles
 from .pusher.particle_push import check_pusher, push_into
 from .solvers.electrostatic_yee import electrostatic_fields_into
 from .solvers.first_order_yee import _check_pml, _pml_args, yee_b, yee_e
-from .utils import is_all_zero
 
 __all__ = ["time_loop_electrodynamic", "time_loop_electrostatic"]
 
 
-def _external(desc, external_fields, dtype):
+# Below these sizes the external fields are read as they are: asking the device whether they are zero costs a host
+# synchronisation (64 x 64 with 262k slots: 345 us a step with six of them, 159 without), adding zeros to the gather
+# a few microseconds.  Larger sets ask, once for the six components.
+_ASK_SLOTS, _ASK_NODES = 1 << 18, 1 << 18
+
+
+def _external(desc, external_fields, dtype, slots):
     ext_E, ext_B = external_fields
     e = [as_field3(c, "external E") for c in ext_E]
     b = [as_field3(c, "external B") for c in ext_B]
     check_fields(desc, *e, *b, dtype=dtype)
-    Ee = None if all(is_all_zero(c) for c in e) else N.p3(e)
-    Be = None if all(is_all_zero(c) for c in b) else N.p3(b)
-    return Ee, Be
+    Ee, Be = N.p3(e), N.p3(b)
+    if slots <= _ASK_SLOTS and e[0].numel() <= _ASK_NODES:
+        return Ee, Be, e + b
+    flags = torch.empty(2, dtype=torch.int32, device=e[0].device)
+    N.call(N.op("pic_any_nonzero", dtype == torch.float64), desc, Ee, Be, N.ptr(flags), N.stream_handle())
+    some_E, some_B = flags.tolist()
+    return (Ee if some_E else None), (Be if some_B else None), e + b
 
 
 def _advance(desc, sp, xp, up, act, scale, stream):
@@ -63,7 +73,7 @@ def time_loop_electrodynamic(particles, species_config, fields, static_parameter
     dtype = xp[0].dtype
     f64 = dtype == torch.float64
     check_fields(desc, *E3, *B3, *J_t, dtype=dtype)
-    Ee, Be = _external(desc, external_fields, dtype)
+    Ee, Be, _keep = _external(desc, external_fields, dtype, S * P)
     dev = xp[0].device
 
     if static_parameters.current_deposition == "esirkepov" and f64:
@@ -146,7 +156,7 @@ def time_loop_electrostatic(particles, species_config, fields, static_parameters
     E3 = [as_field3(c, "E") for c in E]
     B3 = [as_field3(c, "B") for c in B]
     check_fields(desc, *E3, *B3, dtype=torch.float32)
-    Ee, Be = _external(desc, external_fields, torch.float32)
+    Ee, Be, _keep = _external(desc, external_fields, torch.float32, S * P)
     dev = xp[0].device
     us, uv = new_soa(S, P, dev)
     u_planes = [us[0], us[1], us[2]]
