@@ -227,8 +227,8 @@ struct CrossQueue {
 // one (species, tile) pair: the particles that were in that T^3-cell tile at the
 // last sort.  Fields are gathered from an LDS box of the (T+4)^3 nodes around
 // the tile, J is summed in an LDS box of the same nodes and added into the
-// arrays once per block.  Thread t of a chunk owns four
-// consecutive slots, loaded and stored with one 16-byte access per plane;
+// arrays once per block.  Thread t of a chunk owns kP
+// consecutive slots, loaded and stored with one access per plane (16 bytes of four);
 // sorted slots of one cell are contiguous, so a thread's particles mostly share
 // a cell and their twelve moments (flush_moments) are summed in registers, added
 // into the box when the cell changes and, after a sum over equal cells of
@@ -247,14 +247,13 @@ struct CrossQueue {
 // place of ds_add_f32 and a queue of (slot, velocity) took 128^3 with 2 x 16
 // particles per cell from 1963 to 1548 us (43 G particles/s, 2.2 TB/s) and
 // 256^3 with 32 from 12.1 to 9.7 ms; FP64 anchors in the same kernel take
-// 160 x 96 x 96 with 4 per cell from 1132 to 396 us.  kExact: FP32 anchors of an
+// 160 x 96 x 96 with 4 per cell from 1132 to 396 us, one slot a thread there to 315.  kExact: FP32 anchors of an
 // exact grid, else FP64 ones (TileGrid).  kAll: no species has a frozen axis.
-template <int kT, bool kGather, bool kExact, bool kAll>
+template <int kT, bool kGather, bool kExact, bool kAll, int kP>
 __global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_exact_kernel(
     PicDesc d, PicParticles in, FieldPtrs fp, PicParticles out, float* Jx, float* Jy, float* Jz,
     const int32_t* __restrict__ starts, TileGeom tg, TileGrid grid, int32_t* __restrict__ rare, int vec_ok,
     SpeciesTable st, const int32_t* __restrict__ gather) {
-    constexpr int kP = 4;
     constexpr int kB = kT + 4;                     // nodes per axis of both boxes
     constexpr int kB3 = kB * kB * kB;
     constexpr int kChunk = kThreads * kP;          // a thread owns kP consecutive slots
@@ -299,7 +298,7 @@ __global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_exact_ke
     // the first group is loaded before the field box is filled: both wait for memory together
     float PX[3][kP], PU[3][kP];
     uint32_t pact;
-    const auto inside = [&](int64_t s0) { return vec_ok && s0 >= begin && s0 + kP <= end; };
+    const auto inside = [&](int64_t s0) { return kP > 1 && vec_ok && s0 >= begin && s0 + kP <= end; };
     const int64_t first = begin & ~(int64_t)(kP - 1);
     const int64_t g0 = first + (int64_t)kP * (int)threadIdx.x;
     load_group<kP, kGather>(in, gather, g0, begin, end, inside(g0), PX, PU, pact);
@@ -988,8 +987,8 @@ int pic_tile_exact_grid(const PicDesc* desc) {
     return desc && desc_ok(desc) && make_exact_grid(*desc, eg) ? 1 : 0;
 }
 
-// The tile kernel has one launch shape: rounds and min_blocks are those of the
-// strided kernel.
+// The tile kernel chooses its launch shape by the slots of a tile: rounds and
+// min_blocks are those of the strided kernel.
 static void launch_tile_esirkepov(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
                                   const FieldPtrs& fp, const PicParticles* out, float* const J[3],
                                   const int32_t* starts, const TileGeom& tg, const TileGrid& grid, bool exact,
@@ -1000,9 +999,19 @@ static void launch_tile_esirkepov(const PicDesc* desc, const PicSpecies* sp, con
     const SpeciesTable stab = species_table(*desc, *sp);
     bool all = true;
     for (int s = 0; s < sp->count; ++s) all = all && stab.k[s].ux == 7u && stab.k[s].uu == 7u;
-#define PIC_EXACT_LAUNCH(T, GA, EX, ALL)                                                                        \
-    hipLaunchKernelGGL((fused_tile_exact_kernel<T, GA, EX, ALL>), dim3((unsigned)blocks), dim3(kThreads), 0, st, \
+    // Slots per thread by the mean of a block: with four a block of few slots ran in one or two of its waves.
+    // 96^3, 2 / 4 / 8 / 10 per cell (128 / 256 / 512 / 640 slots): 285 / 301 / 348 / 370 us a step with four,
+    // 215 / 255 / 335 / 371 by this rule (FP64 anchors 304 / 322 / 384 / 413 and 221 / 262 / 357 / 418)
+    const int64_t mean = (int64_t)sp->count * sp->slots / blocks;
+#define PIC_EXACT_SLOTS(T, GA, EX, ALL, P)                                                                      \
+    hipLaunchKernelGGL((fused_tile_exact_kernel<T, GA, EX, ALL, P>), dim3((unsigned)blocks), dim3(kThreads), 0, st, \
                        *desc, *in, fp, *out, J[0], J[1], J[2], starts, tg, grid, workspace, vec_ok, stab, gather)
+#define PIC_EXACT_LAUNCH(T, GA, EX, ALL)                                \
+    do {                                                                \
+        if (mean <= kThreads) PIC_EXACT_SLOTS(T, GA, EX, ALL, 1);       \
+        else if (mean <= 2 * kThreads) PIC_EXACT_SLOTS(T, GA, EX, ALL, 2); \
+        else PIC_EXACT_SLOTS(T, GA, EX, ALL, 4);                        \
+    } while (0)
 #define PIC_EXACT_ALL(T, GA, EX)                          \
     do {                                                     \
         if (all) PIC_EXACT_LAUNCH(T, GA, EX, true);       \
@@ -1020,6 +1029,7 @@ static void launch_tile_esirkepov(const PicDesc* desc, const PicSpecies* sp, con
 #undef PIC_EXACT_SHAPE
 #undef PIC_EXACT_ALL
 #undef PIC_EXACT_LAUNCH
+#undef PIC_EXACT_SLOTS
 }
 
 static int fused_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,

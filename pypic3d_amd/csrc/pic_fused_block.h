@@ -1179,7 +1179,7 @@ __device__ inline void load_group(const PicParticles& in, const int32_t* __restr
 template <int kP>
 __device__ inline void store_group(const PicParticles& out, int64_t s0, int64_t begin, int64_t end, bool full,
                                    const float (&PX)[3][kP], const float (&PU)[3][kP], uint32_t oact) {
-    if (full) {
+    if (kP > 1 && full) {
 #pragma unroll
         for (int a = 0; a < 3; ++a) {
             store_vec<kP>(out.x[a] + s0, PX[a]);
