@@ -222,6 +222,34 @@ struct CrossQueue {
     int n;
 };
 
+// Slots of a block of a tile kernel, whose grid has a block per (species, tile)
+// and, in front of them, kOutside for the slots of each species that no tile
+// holds: empty ones for the most part, whose number grows where an open box
+// absorbs particles.  One block per species took longer over them than the tiles
+// (160 x 96 x 96 with 4 per cell and PML, six steps: 2.9 ms on new particles, 3.7
+// on a plasma that had lost some, 2.9 shared out).
+constexpr int kOutside = 128;           // a multiple of 8: the tiles' blocks keep their XCDs
+
+__device__ inline bool tile_slots(const int32_t* __restrict__ starts, const TileGeom& tg, int& s, int& t,
+                                  int64_t& begin, int64_t& end) {
+    const int bx = (int)blockIdx.x, ranges = tg.tiles + 1, count = (int)gridDim.x / (ranges + kOutside);
+    if (bx < count * kOutside) {
+        s = bx / kOutside;
+        t = tg.tiles;
+        const int64_t b0 = starts[s * ranges + t], b1 = starts[s * ranges + t + 1], lo = b0 & ~(int64_t)3;
+        const int64_t share = ((b1 - lo + kOutside - 1) / kOutside + 3) & ~(int64_t)3;
+        begin = max(b0, lo + share * (bx % kOutside));
+        end = min(b1, lo + share * (bx % kOutside + 1));
+    } else {
+        const int b = xcd_block(bx - count * kOutside, count * ranges);
+        s = b / ranges;
+        t = b % ranges;
+        begin = starts[b];
+        end = t < tg.tiles ? starts[b + 1] : begin;
+    }
+    return begin < end;
+}
+
 // Tile-ordered launch: gather + push + Esirkepov + position update +
 // boundaries.  Block b owns the sorted slot range [starts[b], starts[b+1]) of
 // one (species, tile) pair: the particles that were in that T^3-cell tile at the
@@ -264,11 +292,9 @@ __global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_exact_ke
     __shared__ CrossQueue sh;
     __shared__ Sum box[3 * kB3];
     __shared__ float fbox[6 * kB3];
-    const int b = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    const int64_t begin = starts[b], end = starts[b + 1];
-    if (begin >= end) return;
-    const int t = b % (tg.tiles + 1);
-    const int s = b / (tg.tiles + 1);          // blocks are grouped per species
+    int s, t;
+    int64_t begin, end;
+    if (!tile_slots(starts, tg, s, t, begin, end)) return;
     int fo[3] = {0, 0, 0};
     // interior: every particle the fast path handles (anchors inside the field
     // box, cells c0 - 2 .. c0 + T + 1, an anchor step of at most one) stays
@@ -548,11 +574,9 @@ __global__ __launch_bounds__(kThreads, kT == 4 ? 4 : 2) void fused_tile_direct_k
     using Sum = BoxSum<kT>;
     __shared__ Sum box[3 * kB3];
     __shared__ float fbox[6 * kF3];
-    const int b = xcd_block((int)blockIdx.x, (int)gridDim.x);
-    const int64_t begin = starts[b], end = starts[b + 1];
-    if (begin >= end) return;
-    const int t = b % (tg.tiles + 1);
-    const int s = b / (tg.tiles + 1);
+    int s, t;
+    int64_t begin, end;
+    if (!tile_slots(starts, tg, s, t, begin, end)) return;
     int fo[3] = {0, 0, 0};
     // interior: a fast-path particle (anchors inside the field box, cells
     // c0 - 2 .. c0 + T + 1) that moves less than a cell per step stays inside
@@ -915,7 +939,7 @@ static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const P
     for (int a = 0; a < 3; ++a) tg.nt[a] = (desc->n[a] + tile - 1) / tile;
     tg.tiles = tg.nt[0] * tg.nt[1] * tg.nt[2];
     const int64_t blocks = (int64_t)sp->count * (tg.tiles + 1);
-    PIC_REQUIRE(blocks < ((int64_t)1 << 31));
+    PIC_REQUIRE(blocks + kOutside * sp->count < ((int64_t)1 << 31));
     hipStream_t st = as_stream(stream);
     FieldPtrs fp = make_fields(E, B, E_ext, B_ext);
     const int vec_ok = groups_aligned(*in, *out, gather);
@@ -924,7 +948,7 @@ static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const P
     bool all = true;
     for (int s = 0; s < sp->count; ++s) all = all && stab.k[s].ux == 7u && stab.k[s].uu == 7u;
 #define PIC_DIRECT_LAUNCH(T, GA, EX, ALL)                                                                        \
-    hipLaunchKernelGGL((fused_tile_direct_kernel<T, GA, EX, ALL>), dim3((unsigned)blocks), dim3(kThreads), 0, st, \
+    hipLaunchKernelGGL((fused_tile_direct_kernel<T, GA, EX, ALL>), dim3((unsigned)(blocks + kOutside * sp->count)), dim3(kThreads), 0, st, \
                        *desc, *in, fp, *out, J[0], J[1], J[2], starts, tg, grid, workspace, vec_ok, stab, gather)
 #define PIC_DIRECT_ALL(T, GA, EX)                          \
     do {                                                   \
@@ -1004,7 +1028,7 @@ static void launch_tile_esirkepov(const PicDesc* desc, const PicSpecies* sp, con
     // 215 / 255 / 335 / 371 by this rule (FP64 anchors 304 / 322 / 384 / 413 and 221 / 262 / 357 / 418)
     const int64_t mean = (int64_t)sp->count * sp->slots / blocks;
 #define PIC_EXACT_SLOTS(T, GA, EX, ALL, P)                                                                      \
-    hipLaunchKernelGGL((fused_tile_exact_kernel<T, GA, EX, ALL, P>), dim3((unsigned)blocks), dim3(kThreads), 0, st, \
+    hipLaunchKernelGGL((fused_tile_exact_kernel<T, GA, EX, ALL, P>), dim3((unsigned)(blocks + kOutside * sp->count)), dim3(kThreads), 0, st, \
                        *desc, *in, fp, *out, J[0], J[1], J[2], starts, tg, grid, workspace, vec_ok, stab, gather)
 #define PIC_EXACT_LAUNCH(T, GA, EX, ALL)                                \
     do {                                                                \
@@ -1054,7 +1078,7 @@ static int fused_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, cons
     for (int a = 0; a < 3; ++a) tg.nt[a] = (desc->n[a] + tile - 1) / tile;
     tg.tiles = tg.nt[0] * tg.nt[1] * tg.nt[2];
     const int64_t blocks = (int64_t)sp->count * (tg.tiles + 1);
-    PIC_REQUIRE(blocks < ((int64_t)1 << 31));
+    PIC_REQUIRE(blocks + kOutside * sp->count < ((int64_t)1 << 31));
     hipStream_t st = as_stream(stream);
     FieldPtrs fp = make_fields(E, B, E_ext, B_ext);
 #define PIC_TILED_LAUNCH(R, T, MB)                                                                              \
