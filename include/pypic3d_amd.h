@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define PIC_ABI_VERSION 13
+#define PIC_ABI_VERSION 14
 #define PIC_MAX_SPECIES 16
 
 /* Scalar run description: StaticParameters + DynamicParameters fields the hot
@@ -189,6 +189,14 @@ int pic_fused_push_esirkepov(const PicDesc* desc, const PicSpecies* sp, const Pi
                              const float* const E[3], const float* const B[3],
                              const float* const E_ext[3], const float* const B_ext[3],
                              PicParticles* out, float* const J[3], void* stream);
+/* pic_fused_push_esirkepov with every node value of J formed particle by
+ * particle on all grids (1-D and 2-D first-order sets otherwise form them from
+ * a cell's moments, which rounds differently): the forward phase of the
+ * adjoint. */
+int pic_fused_push_esirkepov_nodes(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                   const float* const E[3], const float* const B[3],
+                                   const float* const E_ext[3], const float* const B_ext[3],
+                                   PicParticles* out, float* const J[3], void* stream);
 
 /* Tile-ordered variant for particles sorted by pic_tile_keys (3-D first-order
  * case only): one block per (species, tile) slot range [starts[b], starts[b+1])

@@ -17,7 +17,7 @@ LIB_PATH = os.path.join(HERE, "libpypic3d_hip.so")
 MAX_SPECIES = 16
 PUSHERS = {"boris": 0, "higuera_cary": 1}
 FUSED_VARIANTS = 6
-ABI_VERSION = 13
+ABI_VERSION = 14
 
 c_int = ctypes.c_int
 c_i32 = ctypes.c_int32
@@ -96,6 +96,7 @@ SIGNATURES = {
     "pic_push_binned": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, P3, c_vp, c_i64, c_vp]),
     "pic_fused_push_esirkepov_binned": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_vp, c_i64, c_vp]),
     "pic_fused_push_esirkepov": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_vp]),
+    "pic_fused_push_esirkepov_nodes": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_vp]),
     "pic_fused_push_esirkepov_tiled": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_i32, c_vp, c_i32, c_i32,
                                                c_vp, c_vp]),
     "pic_fused_push_esirkepov_tiled_general": (c_int, [DP, SP, PP, P3, P3, c_vp, c_vp, PP, P3, c_i32, c_vp, c_i32,

@@ -20,6 +20,13 @@ Scope: periodic field and particle boundaries, no PML, the Esirkepov current
 (the branch ``current_deposition == "esirkepov"``), any pusher, shape factor
 and reduced axes.  Adjoint quantities are FP64; the forward state is the FP32
 state of the forward kernels.
+
+The derivative of first-order weights jumps where a particle crosses a node
+line, so a rounding of J that puts one particle on the other side of a line
+changes single entries of the gradient visibly.  The forward phase here forms
+each node value of J by itself (``node_values``), the phase the gradients have
+always been taken through, not from a cell's moments as other 1-D and 2-D runs
+do.
 """
 
 from __future__ import annotations
@@ -105,6 +112,7 @@ class AdjointRun:
                                active=self.active.reshape(1, 1, 1, S, P))
         self.runner = ElectrodynamicRunner(parts, self.cfg, self._fields(E0, B0), self.static, self.dynamic,
                                            sort_every=0)
+        self.runner.node_values = True
         d = self.runner.desc
         if any(d.bc[a] != 0 or d.pbc[a] != 0 for a in range(3)):
             raise NotImplementedError("the adjoint covers periodic field and particle boundaries")

@@ -864,9 +864,11 @@ __global__ __launch_bounds__(kThreads, 1) void fused_boxed_kernel(PicDesc d, Pic
 
 extern "C" {
 
-int pic_fused_push_esirkepov(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
-                             const float* const E[3], const float* const B[3], const float* const E_ext[3],
-                             const float* const B_ext[3], PicParticles* out, float* const J[3], void* stream) {
+// node_values: 1-D and 2-D first-order sets too form J's node values particle by particle.
+static int fused_esirkepov(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                           const float* const E[3], const float* const B[3], const float* const E_ext[3],
+                           const float* const B_ext[3], PicParticles* out, float* const J[3], bool node_values,
+                           void* stream) {
     PIC_REQUIRE(desc_ok(desc) && particles_ok(sp, in) && particles_ok(sp, out) && E && B && J);
     PIC_REQUIRE(desc->n[0] > 1 || desc->n[1] > 1 || desc->n[2] > 1);
     const bool empty = (int64_t)sp->count * sp->slots == 0;
@@ -892,7 +894,7 @@ int pic_fused_push_esirkepov(const PicDesc* desc, const PicSpecies* sp, const Pi
             case 5: PIC_FUSED_LAUNCH(3, 8, 3); break;
             default: PIC_FUSED_LAUNCH(3, 4, 1); break;
         }
-    } else if (kind != 0 && planar_covers(*desc)) {
+    } else if (kind != 0 && !node_values && planar_covers(*desc)) {
         // chunks of 1024 slots amortise ranges and boxes once they still make four blocks a CU; smaller
         // sets take 256, for more blocks (262k slots: 1024 of them, all resident at once)
         const bool large = n >= (int64_t)1 << 20;
@@ -912,6 +914,18 @@ int pic_fused_push_esirkepov(const PicDesc* desc, const PicSpecies* sp, const Pi
 #undef PIC_FUSED_LAUNCH
     PIC_CHECK_LAUNCH();
     return 0;
+}
+
+int pic_fused_push_esirkepov(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                             const float* const E[3], const float* const B[3], const float* const E_ext[3],
+                             const float* const B_ext[3], PicParticles* out, float* const J[3], void* stream) {
+    return fused_esirkepov(desc, sp, in, E, B, E_ext, B_ext, out, J, false, stream);
+}
+
+int pic_fused_push_esirkepov_nodes(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
+                                   const float* const E[3], const float* const B[3], const float* const E_ext[3],
+                                   const float* const B_ext[3], PicParticles* out, float* const J[3], void* stream) {
+    return fused_esirkepov(desc, sp, in, E, B, E_ext, B_ext, out, J, true, stream);
 }
 
 static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,

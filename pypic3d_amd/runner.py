@@ -84,6 +84,7 @@ class ElectrodynamicRunner:
             pml_state = (e_new, b_new, pml_state[2])
         self.rest = (rho, phi, external_fields, pml_state, overflow)
         self.sort_every = int(sort_every)
+        self.node_values = False        # the adjoint's forward phase (adjoint.py)
         self.steps_done = 0
         self.events = None
         self.keys = None
@@ -164,8 +165,9 @@ class ElectrodynamicRunner:
                        self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts), self.rounds,
                        self.min_blocks, N.ptr(self.tile_ws), s)
             else:
-                N.call("pic_fused_push_esirkepov", d, self.sp, self._pp(src), N.p3(E), N.p3(self.B), self.Ee,
-                       self.Be, self._pp(dst), N.p3(self.J), s)
+                N.call("pic_fused_push_esirkepov_nodes" if self.node_values else "pic_fused_push_esirkepov", d,
+                       self.sp, self._pp(src), N.p3(E), N.p3(self.B), self.Ee, self.Be, self._pp(dst), N.p3(self.J),
+                       s)
             if ev:
                 ev[1].record()
             ev = self._mark("current_fold")
