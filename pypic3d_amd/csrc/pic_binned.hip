@@ -635,18 +635,23 @@ __global__ __launch_bounds__(kWide) void bin_esirkepov_kernel(PicDesc d, BinGeom
     extern __shared__ double esir_box[];
     double* const box = esir_box;
     __shared__ uint16_t queue[kShape == 1 ? kQueue : 1];
-    __shared__ int nq;
+    __shared__ int added[3];
     Item it;
     if (!find_item(d, g, w, blockIdx.x, it)) return;
     for (int e = threadIdx.x; e < 3 * g.box; e += kWide) box[e] = 0.0;
-    if (threadIdx.x == 0) nq = 0;
+    if (threadIdx.x < 3) added[threadIdx.x] = 0;
     __syncthreads();
     const TileBox<3> sink{{Jx, Jy, Jz}, box, {it.o[0], it.o[1], it.o[2]}, {g.e[0], g.e[1], g.e[2]}, g.box};
     const float fdt = (float)d.dt;
-    // deposits the queued particles; every thread of the block calls it
+    // Queued particles, the same number in every thread: those of the passes before
+    // (held) and of this one, counted in added[pass].  After a pass's barrier every
+    // wave reads that count and, held being equal, drains or goes on with the others.
+    // A wave that goes on adds to the next count, and clears the one after it, which
+    // was last read before the barrier it has just passed; the third was read by
+    // waves that may not have read it yet, so two counts would not do.
+    int held = 0, pass = 0;
     const auto drain = [&]() {
-        const int m = nq;
-        for (int q = threadIdx.x; q < m; q += kWide) {
+        for (int q = threadIdx.x; q < held; q += kWide) {
             const int64_t r = it.begin + queue[q];
             const float4 a = w.rec[2 * r], b = w.rec[2 * r + 1];
             const SpeciesK& k = st.k[__float_as_int(a.w)];
@@ -710,7 +715,9 @@ __global__ __launch_bounds__(kWide) void bin_esirkepov_kernel(PicDesc d, BinGeom
             const bool in = (unsigned)bi < (unsigned)(g.e[0] - 1) && (unsigned)bj < (unsigned)(g.e[1] - 1) &&
                             (unsigned)bk < (unsigned)(g.e[2] - 1);
             const int at = (bi * g.e[1] + bj) * g.e[2] + bk;
-            if (live && !regular) queue[atomicAdd(&nq, 1)] = (uint16_t)(r - it.begin);
+            const int next = pass == 2 ? 0 : pass + 1;
+            if (threadIdx.x == 0) added[next] = 0;
+            if (live && !regular) queue[held + atomicAdd(&added[pass], 1)] = (uint16_t)(r - it.begin);
             const int key = !regular ? -1 - (int)(threadIdx.x & 63u) : (in ? at : -128 - (int)(threadIdx.x & 63u));
             if (row_run_sums(key, val) && regular) {
 #pragma unroll
@@ -722,12 +729,13 @@ __global__ __launch_bounds__(kWide) void bin_esirkepov_kernel(PicDesc d, BinGeom
                 }
             }
             __syncthreads();
+            held += added[pass];
+            pass = next;
             const bool last = r0 + kWide >= it.end;
-            if (last || nq > kQueue - kWide) {      // room for a whole pass
+            if (last || held > kQueue - kWide) {    // room for a whole pass
                 drain();
-                __syncthreads();
-                if (threadIdx.x == 0) nq = 0;
-                __syncthreads();
+                __syncthreads();                    // before the next pass queues over what was read
+                held = 0;
             }
         } else if (live) {
             double xo[3], xn[3];
