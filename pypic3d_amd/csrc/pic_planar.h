@@ -371,7 +371,9 @@ __device__ __forceinline__ void planar_chunk(const PicDesc& d, const PicSpecies&
     }
     __syncthreads();
     if (!sh.ok[0] || !sh.ok[1]) return;      // (the general kernel's)
-    // ---- range of the centre anchors (FP32 estimate)
+    // ---- range of the centre anchors (FP32 estimate, within one of the anchor below kFar, four times the longest
+    // axis; a chunk with a particle beyond gets no box, so no anchor is taken relative to a clamped range)
+    constexpr int kFar = 1 << 22;
     int lo[2] = {INT_MAX, INT_MAX}, hi[2] = {INT_MIN, INT_MIN};
 #pragma unroll
     for (int a = 0; a < kDims; ++a) {
@@ -379,7 +381,7 @@ __device__ __forceinline__ void planar_chunk(const PicDesc& d, const PicSpecies&
 #pragma unroll
         for (int j = 0; j < kP; ++j) {
             if (((pact >> (8 * j)) & 0xffu) == 0u) continue;
-            const int c = (int)fminf(fmaxf(floorf((PX[a][j] - org) * isp), -1.0e6f), 1.0e6f);
+            const int c = (int)fminf(fmaxf(floorf((PX[a][j] - org) * isp), -(float)kFar), (float)kFar);
             lo[a] = min(lo[a], c);
             hi[a] = max(hi[a], c);
         }
@@ -398,12 +400,15 @@ __device__ __forceinline__ void planar_chunk(const PicDesc& d, const PicSpecies&
     int o[2] = {0, d.g}, e[2] = {1, 1};
     int64_t vol = 1;
     const bool any = sh.lo[0] <= sh.hi[0];
+    bool far = false;
 #pragma unroll
     for (int a = 0; a < kDims; ++a) {
+        far = far || (any && (sh.lo[a] <= -kFar || sh.hi[a] >= kFar));
         o[a] = __builtin_amdgcn_readfirstlane(any ? sh.lo[a] - 2 : 0);
         e[a] = __builtin_amdgcn_readfirstlane(any ? sh.hi[a] - sh.lo[a] + 6 : 6);
         vol *= e[a];
     }
+    if (far) vol = INT64_MAX / 64;
     if (vol <= kPlanarNodes<kP, kBlk>) {
         float* fbox = reinterpret_cast<float*>(sh.box);
         double* box = reinterpret_cast<double*>(sh.box + 24 * kPlanarNodes<kP, kBlk>);
