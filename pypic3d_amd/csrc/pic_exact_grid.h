@@ -66,14 +66,17 @@ struct TileGrid {
 
 // False where a grid's vertex line is not the centre line shifted by half a
 // spacing up to rounding (no grid of the solver; the slot-ordered kernel takes
-// any lines).
-bool make_tile_grid(const PicDesc& d, TileGrid& t) {
+// any lines), or an origin so far that the FP32 estimate may be off by two.  An
+// exact grid (make_exact_grid) takes every part: its anchors are exact.
+bool make_tile_grid(const PicDesc& d, bool exact, TileGrid& t) {
     for (int a = 0; a < 3; ++a) {
         const double org = d.org_c[a], sp = d.sp_c[a];
-        if (!(sp > 0.0) || d.dims[a] > (1 << 20) || !(d.d[a] > 0.0)) return false;
-        const double off = d.org_v[a] - org - 0.5 * sp;
-        if (std::fabs(off) > 1.0e-7 * sp || std::fabs(d.sp_v[a] - sp) * d.dims[a] > 1.0e-7 * sp) return false;
-        if (std::fabs(org) > 4.0e6 * sp) return false;
+        if (!exact) {
+            if (!(sp > 0.0) || d.dims[a] > (1 << 20) || !(d.d[a] > 0.0)) return false;
+            const double off = d.org_v[a] - org - 0.5 * sp;
+            if (std::fabs(off) > 1.0e-7 * sp || std::fabs(d.sp_v[a] - sp) * d.dims[a] > 1.0e-7 * sp) return false;
+            if (std::fabs(org) > 4.0e6 * sp) return false;
+        }
         t.sp[a] = (float)sp;
         t.isp[a] = (float)(1.0 / sp);
         t.isp_up[a] = t.isp[a] * (1.0f + 0x1p-21f);

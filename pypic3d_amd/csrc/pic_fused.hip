@@ -939,7 +939,7 @@ static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const P
     TileGrid grid;
     const bool exact = make_exact_grid(*desc, eg) && desc->d[0] == desc->sp_c[0] && desc->d[1] == desc->sp_c[1] &&
                        desc->d[2] == desc->sp_c[2];
-    PIC_REQUIRE((exact || general) && make_tile_grid(*desc, grid));
+    PIC_REQUIRE((exact || general) && make_tile_grid(*desc, exact, grid));
     const bool empty = (int64_t)sp->count * sp->slots == 0;
     for (int a = 0; a < 3; ++a)
         PIC_REQUIRE(E[a] && B[a] && J[a] && (empty || (in->x[a] != out->x[a] && in->u[a] != out->u[a])));
@@ -1017,7 +1017,7 @@ int pic_fused_push_direct_tiled_gather(const PicDesc* desc, const PicSpecies* sp
 
 int pic_tile_general_grid(const PicDesc* desc) {
     TileGrid grid;
-    return desc && desc_ok(desc) && fused_kind(*desc) == 3 && make_tile_grid(*desc, grid) ? 1 : 0;
+    return desc && desc_ok(desc) && fused_kind(*desc) == 3 && make_tile_grid(*desc, false, grid) ? 1 : 0;
 }
 
 int pic_tile_exact_grid(const PicDesc* desc) {
@@ -1107,7 +1107,7 @@ static int fused_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, cons
     ExactGrid eg;
     TileGrid grid;
     const bool exact = desc->variant != 1 && make_exact_grid(*desc, eg);
-    if ((exact || general) && make_tile_grid(*desc, grid)) {
+    if ((exact || general) && make_tile_grid(*desc, exact, grid)) {
         PIC_REQUIRE(workspace);
         launch_tile_esirkepov(desc, sp, in, fp, out, J, starts, tg, grid, exact, workspace, gather, blocks, st);
         const int64_t rare_grid = std::min<int64_t>(std::max<int64_t>(grid_1d(n, kThreads), 1), 1024);
