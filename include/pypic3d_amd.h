@@ -283,7 +283,7 @@ int pic_fused_push_direct_tiled_gather(const PicDesc* desc, const PicSpecies* sp
  * slot order through cell bins (pic_binned.hip): kind 0 rho, 1 J_from_rhov,
  * 2 Esirkepov (deposit or fused phase), 3 push.  The workspace query returns -1
  * where the grid is not covered (an axis of one cell, or more cells than the
- * bins hold) and, for the push, for small sets.  pic_push_binned samples the
+ * bins hold), from 2^31 - 2048 slots on and, for the push, for small sets.  pic_push_binned samples the
  * slot order on the device and pushes sorted sets in slot order. */
 int64_t pic_binned_workspace_bytes(const PicDesc* desc, const PicSpecies* sp, int32_t kind);
 int pic_deposit_rho_binned(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in, float* rho,

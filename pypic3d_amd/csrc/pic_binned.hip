@@ -795,6 +795,9 @@ int bin_scatter(const PicDesc* desc, const PicSpecies* sp, const PicParticles* i
 
 unsigned item_grid(const BinGeom& g, int64_t n) { return (unsigned)(g.tiles + n / kItem + 1); }
 
+// Slots are numbered in 32 bits; larger sets keep the slot-ordered kernels.
+constexpr int64_t kMaxSlots = ((int64_t)1 << 31) - 8 * kThreads;
+
 // The six field components and the three current components of a box are held
 // one after the other, never together.
 bool binned_ok(const PicDesc* d, int kind, BinGeom& g) {
@@ -834,7 +837,7 @@ int node_deposit(const PicDesc* desc, const PicSpecies* sp, const PicParticles* 
     PIC_REQUIRE(ws_bytes >= pic_binned_workspace_bytes(desc, sp, kKind));
     const int64_t n = (int64_t)sp->count * sp->slots;
     if (n == 0) return 0;
-    PIC_REQUIRE(n < ((int64_t)1 << 31));
+    PIC_REQUIRE(n < kMaxSlots);
     const BinWork w = bin_work(ws, g.tiles, kKind, n);
     const int rc = bin_scatter<kKind>(desc, sp, in, g, w, n, s);
     if (rc) return rc;
@@ -901,7 +904,7 @@ int64_t pic_binned_workspace_bytes(const PicDesc* desc, const PicSpecies* sp, in
     BinGeom g;
     if (!desc || !sp || kind < 0 || kind > 3 || !binned_ok(desc, kind, g)) return -1;
     const int64_t n = (int64_t)sp->count * sp->slots;
-    if (kind == REC_PUSH && !tile_push_ok(g, n)) return -1;
+    if (n >= kMaxSlots || (kind == REC_PUSH && !tile_push_ok(g, n))) return -1;
     return bin_tables(g.tiles) + bin_records(kind, n) + (kind >= REC_ESIRKEPOV && tile_push_ok(g, n) ? 4 * n : 0);
 }
 
@@ -925,7 +928,7 @@ int pic_deposit_esirkepov_binned(const PicDesc* desc, const PicSpecies* sp, cons
     PIC_REQUIRE(workspace_bytes >= pic_binned_workspace_bytes(desc, sp, REC_ESIRKEPOV));
     const int64_t n = (int64_t)sp->count * sp->slots;
     if (n == 0) return 0;
-    PIC_REQUIRE(n < ((int64_t)1 << 31));
+    PIC_REQUIRE(n < kMaxSlots);
     hipStream_t s = as_stream(stream);
     const BinWork w = bin_work(workspace, g.tiles, REC_ESIRKEPOV, n);
     const int rc = bin_scatter<REC_ESIRKEPOV>(desc, sp, in, g, w, n, s);
@@ -939,7 +942,7 @@ int pic_push_binned(const PicDesc* desc, const PicSpecies* sp, const PicParticle
     PIC_REQUIRE(binned_ok(desc, REC_PUSH, g) && particles_ok(sp, in) && E && B && u_out && workspace);
     for (int a = 0; a < 3; ++a) PIC_REQUIRE(E[a] && B[a] && u_out[a]);
     const int64_t need = pic_binned_workspace_bytes(desc, sp, REC_PUSH), n = (int64_t)sp->count * sp->slots;
-    PIC_REQUIRE(need > 0 && workspace_bytes >= need && n < ((int64_t)1 << 31) - 8 * kThreads);
+    PIC_REQUIRE(need > 0 && workspace_bytes >= need && n < kMaxSlots);
     hipStream_t s = as_stream(stream);
     const BinWork w = bin_work(workspace, g.tiles, REC_PUSH, n);
     const FieldPtrs fp = make_fields(E, B, E_ext, B_ext);
@@ -971,7 +974,7 @@ int pic_fused_push_esirkepov_binned(const PicDesc* desc, const PicSpecies* sp, c
     for (int a = 0; a < 3; ++a)
         PIC_REQUIRE(E[a] && B[a] && J[a] && (n == 0 || (in->x[a] != out->x[a] && in->u[a] != out->u[a])));
     PIC_REQUIRE(n == 0 || in->active != out->active);
-    PIC_REQUIRE(n < ((int64_t)1 << 31) - 8 * kThreads);
+    PIC_REQUIRE(n < kMaxSlots);
     PIC_REQUIRE(workspace_bytes >= pic_binned_workspace_bytes(desc, sp, REC_ESIRKEPOV));
     if (n == 0) return 0;
     hipStream_t s = as_stream(stream);
