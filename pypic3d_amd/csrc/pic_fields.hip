@@ -47,10 +47,17 @@ struct Modes {
 // three components instead of three: 27 us less of a 64 x 64 x 1 step.
 constexpr int kRowThreads = 64, kRows = 4;
 
+// Row of a thread of a row_grid launch; its index fits 32 bits where it is below rows.
+__device__ inline bool grid_row(int64_t rows, int& row) {
+    const int64_t r = ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * kRows + threadIdx.y;
+    row = (int)r;
+    return r < rows;
+}
+
 template <class T>
 __global__ void refresh_kernel(PicDesc d, Modes md, T* f0, T* f1, T* f2) {
-    const int row = blockIdx.x * kRows + threadIdx.y;
-    if (row >= d.dims[0] * d.dims[1]) return;
+    int row;
+    if (!grid_row((int64_t)d.dims[0] * d.dims[1], row)) return;
     const int i = row / d.dims[1], j = row % d.dims[1];
     const int si = ghost_source(i, d.n[0], d.g, md.mode[0]), sj = ghost_source(j, d.n[1], d.g, md.mode[1]);
     const bool through = si == i && sj == j;      // an interior row: only its ends are ghosts
@@ -107,8 +114,8 @@ __global__ void finish_kernel(PicDesc d, Modes md, T* f0, T* f1, T* f2, uint32_t
 // (first_order_yee.py:80-92 and the refresh after it).
 template <class T>
 __global__ void walls_kernel(PicDesc d, Modes md, T* f0, T* f1, T* f2) {
-    const int row = blockIdx.x * kRows + threadIdx.y;
-    if (row >= d.n[0] * d.n[1]) return;
+    int row;
+    if (!grid_row((int64_t)d.n[0] * d.n[1], row)) return;
     const int i = row / d.n[1] + d.g, j = row % d.n[1] + d.g;
     const bool all = (d.bc[0] == 1 && (i == d.g || i == d.n[0] + d.g - 1)) ||
                      (d.bc[1] == 1 && (j == d.g || j == d.n[1] + d.g - 1));
@@ -371,10 +378,16 @@ static Modes modes(const PicDesc* d, int bc_type) {
     return m;
 }
 
-static dim3 row_grid(int64_t rows) { return dim3((unsigned)((rows + kRows - 1) / kRows)); }
+// Blocks of kRows rows, in two grid axes: one alone would pass 2^32 threads from 2^28 rows on (a 2-D run of
+// 16384^2 cells).
+static dim3 row_grid(int64_t rows) {
+    const int64_t blocks = (rows + kRows - 1) / kRows, x = std::min<int64_t>(blocks, 1 << 20);
+    return dim3((unsigned)x, (unsigned)((blocks + x - 1) / x));
+}
 
 template <class T>
 static int refresh_t(const PicDesc* d, T* f0, T* f1, T* f2, int bc_type, hipStream_t s) {
+    PIC_REQUIRE((int64_t)d->dims[0] * d->dims[1] < ((int64_t)1 << 31));
     hipLaunchKernelGGL(refresh_kernel<T>, row_grid((int64_t)d->dims[0] * d->dims[1]), dim3(kRowThreads, kRows), 0, s,
                        *d, modes(d, bc_type), f0, f1, f2);
     PIC_CHECK_LAUNCH();
@@ -410,6 +423,7 @@ template <class T>
 static int walls_t(const PicDesc* desc, T* const E[3], hipStream_t s) {
     PIC_REQUIRE(desc_ok(desc) && E && E[0] && E[1] && E[2]);
     if (desc->bc[0] != 1 && desc->bc[1] != 1 && desc->bc[2] != 1) return 0;
+    PIC_REQUIRE((int64_t)desc->n[0] * desc->n[1] < ((int64_t)1 << 31));
     hipLaunchKernelGGL(walls_kernel<T>, row_grid((int64_t)desc->n[0] * desc->n[1]), dim3(kRowThreads, kRows), 0, s,
                        *desc, modes(desc, 0), E[0], E[1], E[2]);
     PIC_CHECK_LAUNCH();
