@@ -864,6 +864,11 @@ __global__ __launch_bounds__(kThreads, 1) void fused_boxed_kernel(PicDesc d, Pic
 
 extern "C" {
 
+// A launch of 2^32 threads or more would run the remainder only, without an error (tiles of 4^3 cells: 1024^3).
+static bool tile_grid_ok(int64_t blocks, int32_t species) {
+    return (blocks + (int64_t)kOutside * species) * kThreads < ((int64_t)1 << 32);
+}
+
 // node_values: 1-D and 2-D first-order sets too form J's node values particle by particle.
 static int fused_esirkepov(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
                            const float* const E[3], const float* const B[3], const float* const E_ext[3],
@@ -953,7 +958,7 @@ static int fused_direct_tiled(const PicDesc* desc, const PicSpecies* sp, const P
     for (int a = 0; a < 3; ++a) tg.nt[a] = (desc->n[a] + tile - 1) / tile;
     tg.tiles = tg.nt[0] * tg.nt[1] * tg.nt[2];
     const int64_t blocks = (int64_t)sp->count * (tg.tiles + 1);
-    PIC_REQUIRE(blocks + kOutside * sp->count < ((int64_t)1 << 31));
+    PIC_REQUIRE(tile_grid_ok(blocks, sp->count));
     hipStream_t st = as_stream(stream);
     FieldPtrs fp = make_fields(E, B, E_ext, B_ext);
     const int vec_ok = groups_aligned(*in, *out, gather);
@@ -1092,7 +1097,7 @@ static int fused_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, cons
     for (int a = 0; a < 3; ++a) tg.nt[a] = (desc->n[a] + tile - 1) / tile;
     tg.tiles = tg.nt[0] * tg.nt[1] * tg.nt[2];
     const int64_t blocks = (int64_t)sp->count * (tg.tiles + 1);
-    PIC_REQUIRE(blocks + kOutside * sp->count < ((int64_t)1 << 31));
+    PIC_REQUIRE(tile_grid_ok(blocks, sp->count));
     hipStream_t st = as_stream(stream);
     FieldPtrs fp = make_fields(E, B, E_ext, B_ext);
 #define PIC_TILED_LAUNCH(R, T, MB)                                                                              \
