@@ -25,14 +25,17 @@ from .particles.particle_class import TiledParticles
 from .pusher.particle_push import check_pusher, push_into
 from .solvers.electrostatic_yee import electrostatic_fields_into
 from .solvers.first_order_yee import _check_pml, _pml_args, yee_b, yee_e
+from .utils import is_all_zero
 
 __all__ = ["time_loop_electrodynamic", "time_loop_electrostatic"]
 
 
-# Below these sizes the external fields are read as they are: asking the device whether they are zero costs a host
-# synchronisation (64 x 64 with 262k slots: 345 us a step with six of them, 159 without), adding zeros to the gather
-# a few microseconds.  Larger sets ask, once for the six components.
-_ASK_SLOTS, _ASK_NODES = 1 << 18, 1 << 18
+# Up to these sizes the external fields are read as they are: asking the device whether they are zero costs a host
+# synchronisation, adding zeros to the gather less.  A step on zero fields, read / asked about:
+#   64 x 64, 2^18 slots 171 / 200 us, 2^20 168 / 200, 2^22 203 / 225, 2^23 400 / 380
+#   3-D in cell order, 2^19 slots 186 / 216 us, 2^20 192 / 226, 2^21 292 / 233, 2^22 602 / 428 (random order 583 / 618)
+#   3-D direct current, 2^20 slots 230 / 257 us, 2^22 635 / 535
+_ASK_SLOTS, _ASK_NODES = 1 << 20, 1 << 18
 
 
 def _external(desc, external_fields, dtype, slots):
@@ -43,9 +46,14 @@ def _external(desc, external_fields, dtype, slots):
     Ee, Be = N.p3(e), N.p3(b)
     if slots <= _ASK_SLOTS and e[0].numel() <= _ASK_NODES:
         return Ee, Be, e + b
-    flags = torch.empty(2, dtype=torch.int32, device=e[0].device)
-    N.call(N.op("pic_any_nonzero", dtype == torch.float64), desc, Ee, Be, N.ptr(flags), N.stream_handle())
-    some_E, some_B = flags.tolist()
+    if all(p is q for p, q in zip(e + b, [*ext_E, *ext_B])):
+        # the caller's own 3-D tensors: counted when they are new or were written to, so later steps do not
+        # synchronise (and can be captured); the views of tile-shaped ones are new on every step
+        some_E, some_B = not all(is_all_zero(c) for c in e), not all(is_all_zero(c) for c in b)
+    else:
+        flags = torch.empty(2, dtype=torch.int32, device=e[0].device)
+        N.call(N.op("pic_any_nonzero", dtype == torch.float64), desc, Ee, Be, N.ptr(flags), N.stream_handle())
+        some_E, some_B = flags.tolist()
     return (Ee if some_E else None), (Be if some_B else None), e + b
 
 
