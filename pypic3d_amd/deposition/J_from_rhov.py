@@ -12,34 +12,39 @@ from .. import _native as N
 from .._tensors import DIRECT, as_field3, binned_workspace, check_fields, is_f64, like_input, make_desc, make_species, particle_planes, pic_particles
 
 
+def raw_direct_current(J3, current_filter, scratch=None):
+    """The arrays that take the raw deposit: J3, or, as the filter reads it from
+    other arrays than it writes, scratch (new ones where it is None)."""
+    if current_filter not in ("bilinear", "digital"):
+        return J3
+    return scratch if scratch is not None else [c.new_empty(c.shape) for c in J3]
+
+
 def deposit_direct_into(desc, sp, pp, J3, current_filter, stream, scratch=None, tile=None, starts=None):
     """tile/starts: tile-ordered deposit for particles sorted by pic_tile_keys
     (FP32 only); float64 J runs the FP64 path."""
     f64 = is_f64(J3[0])
-    N.call(N.op("pic_zero_fields", f64), desc, N.p3(J3), stream)
+    raw = raw_direct_current(J3, current_filter, scratch)
+    N.call(N.op("pic_zero_fields", f64), desc, N.p3(raw), stream)
     if tile and not f64:
-        N.call("pic_deposit_direct_tiled", desc, sp, pp, N.p3(J3), int(tile), N.ptr(starts), stream)
+        N.call("pic_deposit_direct_tiled", desc, sp, pp, N.p3(raw), int(tile), N.ptr(starts), stream)
     else:
         ws = None if f64 else binned_workspace(desc, sp, DIRECT, J3[0].device)
         if ws is not None:
-            N.call("pic_deposit_direct_binned", desc, sp, pp, N.p3(J3), N.ptr(ws), ws.numel(), stream)
+            N.call("pic_deposit_direct_binned", desc, sp, pp, N.p3(raw), N.ptr(ws), ws.numel(), stream)
         else:
-            N.call(N.op("pic_deposit_direct", f64), desc, sp, pp, N.p3(J3), stream)
-    finish_direct_current(desc, J3, current_filter, stream, scratch)
+            N.call(N.op("pic_deposit_direct", f64), desc, sp, pp, N.p3(raw), stream)
+    finish_direct_current(desc, raw, J3, current_filter, stream)
 
 
-def finish_direct_current(desc, J3, current_filter, stream, scratch=None):
-    """Fold + refresh of the raw direct deposit, then the optional filter
-    (J_from_rhov.py:224-258).  The filter writes the other set of arrays, which
-    J3 then holds (scratch, if given, holds the raw deposit's)."""
+def finish_direct_current(desc, raw, J3, current_filter, stream):
+    """Fold + refresh of the raw direct deposit (raw_direct_current), then the
+    optional filter into J3 (J_from_rhov.py:224-258)."""
     f64 = is_f64(J3[0])
-    N.call(N.op("pic_finish_current", f64), desc, N.p3(J3), 1, stream)
-    if current_filter in ("bilinear", "digital"):
-        tmp = scratch if scratch is not None else [c.new_empty(c.shape) for c in J3]
-        N.call(N.op("pic_filter_refresh", f64), desc, N.p3(J3), N.p3(tmp), int(current_filter == "bilinear"),
+    N.call(N.op("pic_finish_current", f64), desc, N.p3(raw), 1, stream)
+    if raw is not J3:
+        N.call(N.op("pic_filter_refresh", f64), desc, N.p3(raw), N.p3(J3), int(current_filter == "bilinear"),
                float(desc.alpha), 1, 0, stream)
-        for c in range(3):
-            J3[c], tmp[c] = tmp[c], J3[c]
 
 
 def J_from_rhov(particles, species_config, J, static_parameters, dynamic_parameters):

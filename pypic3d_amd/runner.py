@@ -20,7 +20,7 @@ import torch
 from . import _native as N
 from ._tensors import as_field3, check_fields, make_desc, make_species, particle_planes, pic_particles, soa_view
 from .deposition.Esirkepov import finish_current
-from .deposition.J_from_rhov import deposit_direct_into, finish_direct_current
+from .deposition.J_from_rhov import deposit_direct_into, finish_direct_current, raw_direct_current
 from .particles.particle_class import TiledParticles
 from .solvers.first_order_yee import _check_pml, _pml_args, yee_b, yee_e
 from .sorting import key_bits
@@ -173,25 +173,26 @@ class ElectrodynamicRunner:
             ev = self._mark("current_fold")
             finish_current(d, self.J, s)
         elif self.tile and (self.direct_fused or self.direct_general):
-            N.call("pic_zero_fields", d, N.p3(self.J), s)
+            raw = raw_direct_current(self.J, self.filter, self.scratch)
+            N.call("pic_zero_fields", d, N.p3(raw), s)
             ev = self._mark("particles")
             if self._pending:
                 N.call("pic_fused_push_direct_tiled_gather", d, self.sp, self._pp(src), N.ptr(self.perm), N.p3(E),
-                       N.p3(self.B), self.Ee, self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts),
+                       N.p3(self.B), self.Ee, self.Be, self._pp(dst), N.p3(raw), self.tile, N.ptr(self.starts),
                        self.direct_min_blocks, N.ptr(self.tile_ws), s)
                 self._pending = False
             elif self.direct_general:
                 N.call("pic_fused_push_direct_tiled_general", d, self.sp, self._pp(src), N.p3(E), N.p3(self.B),
-                       self.Ee, self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts),
+                       self.Ee, self.Be, self._pp(dst), N.p3(raw), self.tile, N.ptr(self.starts),
                        N.ptr(self.tile_ws), s)
             else:
                 N.call("pic_fused_push_direct_tiled", d, self.sp, self._pp(src), N.p3(E), N.p3(self.B), self.Ee,
-                       self.Be, self._pp(dst), N.p3(self.J), self.tile, N.ptr(self.starts), self.direct_min_blocks,
+                       self.Be, self._pp(dst), N.p3(raw), self.tile, N.ptr(self.starts), self.direct_min_blocks,
                        N.ptr(self.tile_ws), s)
             if ev:
                 ev[1].record()
             ev = self._mark("current_fold")
-            finish_direct_current(d, self.J, self.filter, s, scratch=self.scratch)
+            finish_direct_current(d, raw, self.J, self.filter, s)
         else:
             ev = self._mark("particles")
             uo = [self.vel[dst][0], self.vel[dst][1], self.vel[dst][2]]
