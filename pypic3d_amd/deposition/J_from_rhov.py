@@ -20,16 +20,18 @@ def raw_direct_current(J3, current_filter, scratch=None):
     return scratch if scratch is not None else [c.new_empty(c.shape) for c in J3]
 
 
-def deposit_direct_into(desc, sp, pp, J3, current_filter, stream, scratch=None, tile=None, starts=None):
+def deposit_direct_into(desc, sp, pp, J3, current_filter, stream, scratch=None, tile=None, starts=None,
+                        workspace=binned_workspace):
     """tile/starts: tile-ordered deposit for particles sorted by pic_tile_keys
-    (FP32 only); float64 J runs the FP64 path."""
+    (FP32 only); float64 J runs the FP64 path.  workspace(desc, sp, kind, device):
+    where the scratch of a deposit in any order comes from."""
     f64 = is_f64(J3[0])
     raw = raw_direct_current(J3, current_filter, scratch)
     N.call(N.op("pic_zero_fields", f64), desc, N.p3(raw), stream)
     if tile and not f64:
         N.call("pic_deposit_direct_tiled", desc, sp, pp, N.p3(raw), int(tile), N.ptr(starts), stream)
     else:
-        ws = None if f64 else binned_workspace(desc, sp, DIRECT, J3[0].device)
+        ws = None if f64 else workspace(desc, sp, DIRECT, J3[0].device)
         if ws is not None:
             N.call("pic_deposit_direct_binned", desc, sp, pp, N.p3(raw), N.ptr(ws), ws.numel(), stream)
         else:

@@ -18,7 +18,8 @@ from __future__ import annotations
 import torch
 
 from . import _native as N
-from ._tensors import as_field3, check_fields, make_desc, make_species, particle_planes, pic_particles, soa_view
+from ._tensors import (as_field3, binned_workspace, check_fields, make_desc, make_species, particle_planes, pic_particles,
+                       soa_view)
 from .deposition.Esirkepov import finish_current
 from .deposition.J_from_rhov import deposit_direct_into, finish_direct_current, raw_direct_current
 from .particles.particle_class import TiledParticles
@@ -94,7 +95,7 @@ class ElectrodynamicRunner:
         # (two slots per thread) at tile 4, one at tile 8
         self.direct_min_blocks = 1
         self.sort_lookahead = None      # tile re-sort keys at x + t u; None: t = sort_every * dt / 2
-        self.tile_ws, self.direct_fused = None, False
+        self.tile_ws, self.direct_fused, self._deposit_ws = None, False, None
         self.defer_permute = self.tile_general = self.direct_general = False
         if tile is not None:
             self.set_tile(tile)
@@ -206,7 +207,7 @@ class ElectrodynamicRunner:
                 ev[1].record()
             ev = self._mark("current_fold")
             deposit_direct_into(d, self.sp, self._pp(dst), self.J, self.filter, s, scratch=self.scratch,
-                                tile=self.tile, starts=self.starts)
+                                tile=self.tile, starts=self.starts, workspace=self._deposit_workspace)
             N.call("pic_advance_positions", d, self.sp, self._pp(dst), 0.5, N.p3(xd), s)
             N.call("pic_particle_boundaries", d, self.sp, self._pp(dst), s)
         if ev:
@@ -243,6 +244,12 @@ class ElectrodynamicRunner:
         self.desc.variant = best
         return best, times
 
+    def _deposit_workspace(self, *args):
+        """binned_workspace, taken at the first step that needs it and kept."""
+        if self._deposit_ws is None:
+            self._deposit_ws = (binned_workspace(*args),)
+        return self._deposit_ws[0]
+
     def _sort_buffers(self):
         n = self.S * self.P
         dev = self.device
@@ -271,7 +278,7 @@ class ElectrodynamicRunner:
             raise ValueError("the tile-ordered Esirkepov kernel needs the 3-D first-order path")
         if tile not in (4, 8):
             raise ValueError("tile must be 4 or 8")
-        self.tile = int(tile)
+        self.tile, self._deposit_ws = int(tile), None
         self.direct_min_blocks = 4 if self.tile == 4 else 1
         # direct branch: one fused tile kernel on 3-D first-order grids (FP32 anchors on exact ones with cells
         # equal to the node spacing), the separate push / advance / boundary / deposit kernels otherwise
