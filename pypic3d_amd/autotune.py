@@ -47,21 +47,28 @@ def tune_fused(desc, sp, pp_in, E3, B3, Ee, Be, pp_out, J3, reps=3, variants=Non
     return best, times
 
 
-def tune_tiled(desc, sp, pp_in, E3, B3, Ee, Be, pp_out, J3, tile, starts, workspace, reps=3, rounds=(4,),
-               min_blocks=(4,)):
-    """Launch shape of the tile-ordered kernel, which has one; candidates matter to the strided kernel only:
-    ((rounds, min_blocks), {"rounds/min_blocks": mean ms})."""
+def tune_tiled(desc, sp, pp_in, E3, B3, Ee, Be, pp_out, J3, tile, starts, workspace, reps=3, rounds=(2, 4, 8),
+               min_blocks=(1, 3, 4), general=False):
+    """Launch shape of the tile-ordered phase: ((rounds, min_blocks), {"rounds/min_blocks": mean ms}).  The tile
+    kernel (exact grids, any grid where general is set, as the runner's steps do) has one launch shape, which is timed
+    alone; the candidates are those of the strided kernel (other grids, desc.variant 1)."""
     s = N.stream_handle()
+    exact = bool(N.lib().pic_tile_exact_grid(desc))
+    if desc.variant != 1 and (exact or general):
+        rounds = (4,) if 4 in rounds else rounds[:1]
+        min_blocks = (4,) if 4 in min_blocks else min_blocks[:1]
+    general = general and not exact and desc.variant != 1
+    name = "pic_fused_push_esirkepov_tiled_general" if general else "pic_fused_push_esirkepov_tiled"
     times = {}
     for r in rounds:
         for mb in min_blocks:
-            args = (desc, sp, pp_in, N.p3(E3), N.p3(B3), Ee, Be, pp_out, N.p3(J3), tile, N.ptr(starts), r, mb,
-                    N.ptr(workspace), s)
-            N.call("pic_fused_push_esirkepov_tiled", *args)
+            args = (desc, sp, pp_in, N.p3(E3), N.p3(B3), Ee, Be, pp_out, N.p3(J3), tile, N.ptr(starts), r,
+                    *(() if general else (mb,)), N.ptr(workspace), s)
+            N.call(name, *args)
             a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             a.record()
             for _ in range(reps):
-                N.call("pic_fused_push_esirkepov_tiled", *args)
+                N.call(name, *args)
             b.record()
             torch.cuda.synchronize()
             times[(r, mb)] = a.elapsed_time(b) / reps

@@ -226,9 +226,10 @@ class ElectrodynamicRunner:
 
     def autotune(self, reps=3):
         """Pick the fastest launch shape of the fused kernel on the current
-        state: the slot-ordered kernel's variants, or in tile mode the tiled
-        kernel's slots per thread.  The timed launches write the inactive
-        particle set and J, which the next step overwrites."""
+        state: the slot-ordered kernel's variants, or in tile mode the strided
+        kernel's slots per thread where that kernel runs (the tile kernel has
+        one shape).  The timed launches write the inactive particle set and J,
+        which the next step overwrites."""
         from .autotune import tune_fused, tune_tiled
         if not self.esirkepov:
             return None, {}
@@ -236,7 +237,7 @@ class ElectrodynamicRunner:
         E = self.E[self.ecur]
         if self.tile:
             best, times = tune_tiled(self.desc, self.sp, self._pp(src), E, self.B, self.Ee, self.Be, self._pp(dst),
-                                     self.J, self.tile, self.starts, self.tile_ws, reps=reps)
+                                     self.J, self.tile, self.starts, self.tile_ws, reps=reps, general=self.tile_general)
             self.rounds, self.min_blocks = best
             return best, times
         best, times = tune_fused(self.desc, self.sp, self._pp(src), E, self.B, self.Ee, self.Be, self._pp(dst),
