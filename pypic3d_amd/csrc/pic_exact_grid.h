@@ -20,11 +20,6 @@ struct ExactGrid {
     float org_c[3], sp_c[3], isp_c[3], half_sp[3];
     float inv_d[3];
     float xlo[3], xhi[3];
-    double tol[3];      // band around a face inside which a new FP64 position takes the queue
-    // FP32 form of the same test: an FP32 offset (x - node) + v dt in
-    // [band_lo, band_hi) puts the FP64 new position in [node + tol, node + sp - tol)
-    // (the FP32 offset is within 2^-23 sp of the FP64 one; the band is 2 tol wide)
-    float band_lo[3], band_hi[3];
 };
 
 // Center-line anchor and offset of x (xlo <= x < xhi): the FP32 estimate is
@@ -56,7 +51,10 @@ __device__ inline void exact_anchors(float x, float org, float sp, float isp, fl
 struct TileGrid {
     float sp[3], isp[3], isp_up[3], half[3], inv_d[3];
     float bias[3], edge[3];
-    float lim[3];       // a new offset from the cell's middle below lim stays in the cell (ExactGrid::band_*)
+    // a new FP32 offset from the cell's middle below lim stays in the cell: it is within 2^-22 spacings of the FP64
+    // one, and FP64 floor((x - org)/sp) differs from the exact bracket only within a few ulps of a quotient below
+    // 2^22, so a band of 2^-19 spacings along the faces covers both
+    float lim[3];
     double sp64[3], org64[3], half64[3];
     // the rest of cross_axis' arguments, and the time step: scalar kernel arguments, where
     // a division or conversion in the kernel would hold a vector register across its loops
@@ -159,14 +157,6 @@ bool make_exact_grid(const PicDesc& d, ExactGrid& eg) {
         eg.inv_d[a] = (float)(1.0 / d.d[a]);
         eg.xlo[a] = std::fma((float)lo, s32, o32);
         eg.xhi[a] = std::fma((float)hi, s32, o32);
-        // floor((x - org)/sp) in FP64 can differ from the exact bracket only within a
-        // few FP64 ulps of the quotient (|quotient| < 2^22 here): a band of 2^-20 sp is ample
-        eg.tol[a] = std::ldexp(sp, -20);
-        eg.band_lo[a] = (float)std::ldexp(sp, -19);                      // exact
-        const double hd = sp - std::ldexp(sp, -19);
-        float hf = (float)hd;
-        if ((double)hf > hd) hf = std::nextafter(hf, 0.0f);                // rounded down
-        eg.band_hi[a] = hf;
     }
     return true;
 }

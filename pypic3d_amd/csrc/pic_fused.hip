@@ -1044,7 +1044,9 @@ static void launch_tile_esirkepov(const PicDesc* desc, const PicSpecies* sp, con
     for (int s = 0; s < sp->count; ++s) all = all && stab.k[s].ux == 7u && stab.k[s].uu == 7u;
     // Slots per thread by the mean of a block: with four a block of few slots ran in one or two of its waves.
     // 96^3, 2 / 4 / 8 / 10 per cell (128 / 256 / 512 / 640 slots): 285 / 301 / 348 / 370 us a step with four,
-    // 215 / 255 / 335 / 371 by this rule (FP64 anchors 304 / 322 / 384 / 413 and 221 / 262 / 357 / 418)
+    // 215 / 255 / 335 / 371 by this rule (FP64 anchors 304 / 322 / 384 / 413 and 221 / 262 / 357 / 418).  Tiles of 8^3
+    // cells, the phase alone, 64 / 128 / 256 / 384 / 512 slots: 105 / 118 / 137 / 144 / 150 us with four, 85 / 100 /
+    // 119 / 126 / 146 by the rule (FP64 anchors 106 / 120 / 138 / 145 / 151 and 86 / 98 / 120 / 128 / 146)
     const int64_t mean = (int64_t)sp->count * sp->slots / blocks;
 #define PIC_EXACT_SLOTS(T, GA, EX, ALL, P)                                                                      \
     hipLaunchKernelGGL((fused_tile_exact_kernel<T, GA, EX, ALL, P>), dim3((unsigned)(blocks + kOutside * sp->count)), dim3(kThreads), 0, st, \

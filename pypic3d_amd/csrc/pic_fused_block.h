@@ -453,8 +453,6 @@ __device__ inline bool cross_axis(double xo, double xn, double org, double sp, d
     return true;
 }
 
-__device__ inline float sel3(int k, float a0, float a1, float a2) { return k == 0 ? a0 : (k == 1 ? a1 : a2); }
-
 // All 54 terms (component c, differenced slot i in {0,1}, 3x3 slots (j, k) of
 // the other two axes) of one particle, fully unrolled so every per-axis value
 // stays in registers.

@@ -17,27 +17,6 @@ struct GatherAxis {
     int k0, k1;     // live stencil slots [k0, k1)
 };
 
-__device__ inline void gather_axis(double pos, double org, double sp, int sf, int L, bool active, int g,
-                                   GatherAxis& s) {
-    int a = anchor_of(pos, org, sp, sf);
-    double delta = pos - node_coord(a, sp, org);
-    double w[3];
-    shape3(delta / sp, sf, w);
-    if (active) {
-        for (int q = 0; q < 3; ++q) {
-            s.p[q] = pmod(a - 1 + q, L);
-            s.w[q] = (float)w[q];
-        }
-        s.k0 = sf == 1 ? 1 : 0;   // CIC weight of point -1 is exactly 0 (shapes.py:46-48)
-        s.k1 = 3;
-    } else {
-        s.p[0] = g;
-        s.w[0] = (float)(w[0] + w[1] + w[2]);
-        s.k0 = 0;
-        s.k1 = 1;
-    }
-}
-
 __device__ inline float gather3(const float* __restrict__ f, const float* __restrict__ fext, const PicDesc& d,
                                 const GatherAxis& ax, const GatherAxis& ay, const GatherAxis& az) {
     float acc = 0.0f;
@@ -105,24 +84,6 @@ inline SpeciesTable species_table(const PicDesc& d, const PicSpecies& sp) {
     SpeciesTable t{};
     for (int s = 0; s < sp.count && s < PIC_MAX_SPECIES; ++s) t.k[s] = species_constants(d, sp, s);
     return t;
-}
-
-// Six staggered components (particle_push.py:63-68): Ex (v,c,c), Ey (c,v,c),
-// Ez (c,c,v), Bx (c,v,v), By (v,c,v), Bz (v,v,c).
-__device__ inline void gather_EB(const PicDesc& d, const FieldPtrs& fp, const double pos[3], float E[3],
-                                 float B[3]) {
-    GatherAxis c[3], v[3];
-    for (int a = 0; a < 3; ++a) {
-        bool act = d.n[a] > 1;
-        gather_axis(pos[a], d.org_c[a], d.sp_c[a], d.shape_factor, d.dims[a], act, d.g, c[a]);
-        gather_axis(pos[a], d.org_v[a], d.sp_v[a], d.shape_factor, d.dims[a], act, d.g, v[a]);
-    }
-    E[0] = gather3(fp.E[0], fp.Ee[0], d, v[0], c[1], c[2]);
-    E[1] = gather3(fp.E[1], fp.Ee[1], d, c[0], v[1], c[2]);
-    E[2] = gather3(fp.E[2], fp.Ee[2], d, c[0], c[1], v[2]);
-    B[0] = gather3(fp.B[0], fp.Be[0], d, c[0], v[1], v[2]);
-    B[1] = gather3(fp.B[1], fp.Be[1], d, v[0], c[1], v[2]);
-    B[2] = gather3(fp.B[2], fp.Be[2], d, v[0], v[1], c[2]);
 }
 
 // ------------------------------------------------------------------------
