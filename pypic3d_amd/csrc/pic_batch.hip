@@ -12,18 +12,22 @@
 // function as the single-simulation kernel (fast paths chosen per item).
 //
 // Field phase: the grid part of time_loop_electrodynamic's Esirkepov branch
-// (evolve.py:70-97) as four launches over all members: J fold + refresh with
-// the particle codes, B half step, E step, B half step, each point stored with
-// its ghost images, so no pass needs a barrier inside.  A block per member with
-// barriers between the passes left three quarters of the chip idle at 64
-// members (647 us per step of 64 members of up to 256 x 32 cells).
+// (evolve.py:70-97) as four launches over all members: J fold, B half step with
+// J's guard cells, E step, B half step, none of which needs a barrier inside.
 #include "pic_field_ops.h"
 #include "pic_planar.h"
+
+#include <algorithm>
 
 namespace {
 
 constexpr int kFieldThreads = 256;
-constexpr int kFieldBlocks = 16;       // per member and pass
+// Blocks of a pass, shared out over the members.  A block costs 3.6 ns to start
+// whether it has points or not, and four a CU hide the latency: the four passes
+// of 2048 members of 64 cells take 161 us with one block a member, 304 with four
+// and 717 with sixteen; 256 of 32 x 32 167 / 87 / 128; one of 512 x 512 69 with
+// 1024, 466 with 64.
+constexpr int kFieldBlocks = 1024;
 
 struct BatchFields {
     const float* E[3];
@@ -134,22 +138,38 @@ __global__ __launch_bounds__(kThreads, 1) void batch_fused_kernel(const PicBatch
     }
 }
 
-__device__ inline void interior_ijk(const PicDesc& d, int64_t t, int& i, int& j, int& k) {
-    k = (int)(t % d.n[2]) + d.g;
-    int64_t r = t / d.n[2];
-    j = (int)(r % d.n[1]) + d.g;
-    i = (int)(r / d.n[1]) + d.g;
+// Array point of number t in a box of e[] points from index o.
+__device__ inline void box_point(const int e1, const int e2, int o, uint32_t t, int& i, int& j, int& k) {
+    const uint32_t r = t / (uint32_t)e2;
+    k = (int)(t - r * (uint32_t)e2) + o;
+    j = (int)(r % (uint32_t)e1) + o;
+    i = (int)(r / (uint32_t)e1) + o;
 }
 
-// Pass 0: J fold + refresh with the particle codes (Esirkepov.py:357-359);
-// 1: B_h = B - (dt/2) curl E (evolve.py:88); 2: E' = E + dt (C^2 curl B_h -
-// J/eps) (:92); 3: B = B_h - (dt/2) curl E' (:96).  gridDim.x blocks share a
-// member's points; blockIdx.y is the member.
+// Pass 0: J's guard cells folded into the interior with the particle codes
+// (Esirkepov.py:357-359); 1: B_h = B - (dt/2) curl E (evolve.py:88) and J's
+// guard cells; 2: E' = E + dt (C^2 curl B_h - J/eps) (:92); 3: B = B_h - (dt/2)
+// curl E' (:96).  gridDim.x blocks share a member's points; blockIdx.y is the
+// member.  Pass 0 has a thread per interior cell and component (a guard cell
+// belongs to one cell, so nothing it reads is written by another); the others
+// have a thread per array point, which stores the value of the interior point
+// its coordinates map to.  1-D and 2-D members have 25 and 5 points a cell along
+// their reduced axes, contiguous in memory: stored by the cell's own thread they
+// took a strided store each, and the four passes of 2048 members of 64 cells
+// 2.6 ms (a block per member with barriers between the passes: 397 us; now 161),
+// of 64 members of 256 x 32 cells 152 (646, 141), of one of 512 x 512 1505 (15685,
+// 69).
 template <int kPass>
 __global__ __launch_bounds__(kFieldThreads) void batch_field_kernel(const PicBatchSim* __restrict__ sims,
                                                                      BatchFields bf) {
-    const PicDesc& d = sims[blockIdx.y].desc;
-    const int64_t off = sims[blockIdx.y].field_offset;
+    const PicDesc& d = member(sims, blockIdx.y).desc;
+    const int64_t off = member(sims, blockIdx.y).field_offset;
+    const uint32_t points = kPass == 0 ? (uint32_t)(d.n[0] * d.n[1] * d.n[2]) : (uint32_t)field_size(d);
+    const uint32_t t0 = blockIdx.x * kFieldThreads + threadIdx.x, step = gridDim.x * kFieldThreads;
+    if (blockIdx.x * kFieldThreads >= points) return;
+    // FP64 divisions: by one thread of the block
+    __shared__ YeeConst y;
+    if (kPass != 0 && threadIdx.x == 0) y = yee_const(d);
     const float* E[3];
     float *B[3], *Bh[3], *J[3], *Eo[3];
     for (int c = 0; c < 3; ++c) {
@@ -159,25 +179,39 @@ __global__ __launch_bounds__(kFieldThreads) void batch_field_kernel(const PicBat
         J[c] = bf.J[c] + off;
         Eo[c] = bf.Eo[c] + off;
     }
-    const YeeConst y = yee_const(d);
-    int mode[3], sign[3];
-    for (int a = 0; a < 3; ++a) {
-        mode[a] = refresh_mode(d, a, 1);
-        sign[a] = fold_sign(d, a, 1);
-    }
-    const int64_t ni = (int64_t)d.n[0] * d.n[1] * d.n[2];
-    for (int64_t t = (int64_t)blockIdx.x * kFieldThreads + threadIdx.x; t < ni;
-         t += (int64_t)gridDim.x * kFieldThreads) {
-        int i, j, k;
-        interior_ijk(d, t, i, j, k);
-        if constexpr (kPass == 0) {
-            for (int c = 0; c < 3; ++c) finish_point(d, mode, sign, J[c], i, j, k);
-        } else if constexpr (kPass == 1) {
-            yee_b_point(d, y, E, B, Bh, i, j, k);
-        } else if constexpr (kPass == 2) {
-            yee_e_point(d, y, E, Bh, J, Eo, i, j, k);
-        } else {
-            yee_b_point(d, y, Eo, Bh, B, i, j, k);
+    int mode[3], i, j, k;
+    for (int a = 0; a < 3; ++a) mode[a] = refresh_mode(d, a, 1);
+    if constexpr (kPass == 0) {
+        int sign[3];
+        for (int a = 0; a < 3; ++a) sign[a] = fold_sign(d, a, 1);
+        float* const f = blockIdx.z == 0 ? J[0] : (blockIdx.z == 1 ? J[1] : J[2]);
+        for (uint32_t t = t0; t < points; t += step) {
+            box_point(d.n[1], d.n[2], d.g, t, i, j, k);
+            if (has_images(d, 0, i) || has_images(d, 1, j) || has_images(d, 2, k))
+                f[fidx(d, i, j, k)] = folded_at(d, mode, sign, f, i, j, k);
+        }
+    } else {
+        __syncthreads();
+        for (uint32_t t = t0; t < points; t += step) {
+            box_point(d.dims[1], d.dims[2], 0, t, i, j, k);
+            const int si = ghost_source(i, d.n[0], d.g, y.mode[0]), sj = ghost_source(j, d.n[1], d.g, y.mode[1]);
+            const int sk = ghost_source(k, d.n[2], d.g, y.mode[2]);
+            float v[3] = {0.0f, 0.0f, 0.0f};
+            if (si >= 0 && sj >= 0 && sk >= 0) {
+                if constexpr (kPass == 1) yee_b_value(d, y, E, B, v, si, sj, sk);
+                else if constexpr (kPass == 2) yee_e_value(d, y, E, Bh, J, v, si, sj, sk);
+                else yee_b_value(d, y, Eo, Bh, v, si, sj, sk);
+            }
+            float* const* out = kPass == 1 ? Bh : (kPass == 2 ? Eo : B);
+            for (int c = 0; c < 3; ++c) out[c][t] = v[c];
+            if constexpr (kPass == 1) {
+                const int pi = ghost_source(i, d.n[0], d.g, mode[0]), pj = ghost_source(j, d.n[1], d.g, mode[1]);
+                const int pk = ghost_source(k, d.n[2], d.g, mode[2]);
+                if (pi == i && pj == j && pk == k) continue;
+                const bool zero = pi < 0 || pj < 0 || pk < 0;
+                const int64_t src = zero ? t : fidx(d, pi, pj, pk);
+                for (int c = 0; c < 3; ++c) J[c][t] = zero ? 0.0f : J[c][src];
+            }
         }
     }
 }
@@ -262,8 +296,10 @@ int pic_batch_field_step(const PicBatchSim* sims, int32_t n_sims, const float* c
     constexpr int kRowsMax = 65535;      // members per launch (grid rows)
     for (int32_t first = 0; first < n_sims; first += kRowsMax) {
         const PicBatchSim* part = sims + first;
-        const dim3 grid(kFieldBlocks, (unsigned)(n_sims - first < kRowsMax ? n_sims - first : kRowsMax));
-        hipLaunchKernelGGL(batch_field_kernel<0>, grid, dim3(kFieldThreads), 0, st, part, bf);
+        const int members = n_sims - first < kRowsMax ? n_sims - first : kRowsMax;
+        const int per = std::max(kFieldBlocks / members, 1);
+        const dim3 grid((unsigned)per, (unsigned)members), fold((unsigned)per, (unsigned)members, 3);
+        hipLaunchKernelGGL(batch_field_kernel<0>, fold, dim3(kFieldThreads), 0, st, part, bf);
         hipLaunchKernelGGL(batch_field_kernel<1>, grid, dim3(kFieldThreads), 0, st, part, bf);
         hipLaunchKernelGGL(batch_field_kernel<2>, grid, dim3(kFieldThreads), 0, st, part, bf);
         hipLaunchKernelGGL(batch_field_kernel<3>, grid, dim3(kFieldThreads), 0, st, part, bf);

@@ -288,11 +288,10 @@ __host__ __device__ inline YeeConstT<T> yee_const(const PicDesc& d) {
 }
 
 // first_order_yee.py:96-142 at interior array point (i, j, k):
-// B_out = B_in - (dt/2) curl E with forward differences, guard cells refreshed
-// (out may be B: only the point itself is read from it).
+// v = B_in - (dt/2) curl E with forward differences.
 template <class T>
-__device__ inline void yee_b_point(const PicDesc& d, const YeeConstT<T>& y, const T* const E[3], const T* const B[3],
-                                   T* const out[3], int i, int j, int k) {
+__device__ inline void yee_b_value(const PicDesc& d, const YeeConstT<T>& y, const T* const E[3], const T* const B[3],
+                                   T v[3], int i, int j, int k) {
     int64_t c = fidx(d, i, j, k);
     T ex = E[0][c], ey = E[1][c], ez = E[2][c];
     T ez_yp = refreshed_at(E[2], d, y.mode, i, j + 1, k, 1);
@@ -304,16 +303,25 @@ __device__ inline void yee_b_point(const PicDesc& d, const YeeConstT<T>& y, cons
     T curl_x = (ez_yp - ez) * y.id[1] - (ey_zp - ey) * y.id[2];
     T curl_y = (ex_zp - ex) * y.id[2] - (ez_xp - ez) * y.id[0];
     T curl_z = (ey_xp - ey) * y.id[0] - (ex_yp - ex) * y.id[1];
-    const T v[3] = {B[0][c] - y.hdt * curl_x, B[1][c] - y.hdt * curl_y, B[2][c] - y.hdt * curl_z};
+    v[0] = B[0][c] - y.hdt * curl_x;
+    v[1] = B[1][c] - y.hdt * curl_y;
+    v[2] = B[2][c] - y.hdt * curl_z;
+}
+
+// The point stored with its guard images (out may be B: only the point itself is read from it).
+template <class T>
+__device__ inline void yee_b_point(const PicDesc& d, const YeeConstT<T>& y, const T* const E[3], const T* const B[3],
+                                   T* const out[3], int i, int j, int k) {
+    T v[3];
+    yee_b_value(d, y, E, B, v, i, j, k);
     store_refreshed<3>(d, y.mode, out, i, j, k, v);
 }
 
 // first_order_yee.py:12-72 at interior array point (i, j, k):
-// E_out = E_in + dt (C^2 curl B - J/eps) with backward differences, guard
-// cells refreshed.
+// v = E_in + dt (C^2 curl B - J/eps) with backward differences.
 template <class T>
-__device__ inline void yee_e_point(const PicDesc& d, const YeeConstT<T>& y, const T* const E[3], const T* const B[3],
-                                   const T* const J[3], T* const out[3], int i, int j, int k) {
+__device__ inline void yee_e_value(const PicDesc& d, const YeeConstT<T>& y, const T* const E[3], const T* const B[3],
+                                   const T* const J[3], T v[3], int i, int j, int k) {
     int64_t c = fidx(d, i, j, k);
     T bx = B[0][c], by = B[1][c], bz = B[2][c];
     T bz_ym = refreshed_at(B[2], d, y.mode, i, j - 1, k, 1);
@@ -325,9 +333,16 @@ __device__ inline void yee_e_point(const PicDesc& d, const YeeConstT<T>& y, cons
     T curl_x = (bz - bz_ym) * y.id[1] - (by - by_zm) * y.id[2];
     T curl_y = (bx - bx_zm) * y.id[2] - (bz - bz_xm) * y.id[0];
     T curl_z = (by - by_xm) * y.id[0] - (bx - bx_ym) * y.id[1];
-    const T v[3] = {E[0][c] + (y.c2 * curl_x - J[0][c] * y.inv_eps) * y.dt,
-                    E[1][c] + (y.c2 * curl_y - J[1][c] * y.inv_eps) * y.dt,
-                    E[2][c] + (y.c2 * curl_z - J[2][c] * y.inv_eps) * y.dt};
+    v[0] = E[0][c] + (y.c2 * curl_x - J[0][c] * y.inv_eps) * y.dt;
+    v[1] = E[1][c] + (y.c2 * curl_y - J[1][c] * y.inv_eps) * y.dt;
+    v[2] = E[2][c] + (y.c2 * curl_z - J[2][c] * y.inv_eps) * y.dt;
+}
+
+template <class T>
+__device__ inline void yee_e_point(const PicDesc& d, const YeeConstT<T>& y, const T* const E[3], const T* const B[3],
+                                   const T* const J[3], T* const out[3], int i, int j, int k) {
+    T v[3];
+    yee_e_value(d, y, E, B, J, v, i, j, k);
     store_refreshed<3>(d, y.mode, out, i, j, k, v);
 }
 
