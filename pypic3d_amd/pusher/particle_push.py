@@ -20,12 +20,30 @@ def check_pusher(static_parameters):
         raise ValueError(f"Unknown particle_pusher: {static_parameters.particle_pusher}")
 
 
+# The push through tiles brings the launches of the binning (20 us of host time), so first-order sets take it from
+# 2^20 slots on.  us in slot order / through tiles, random order: 2^18 slots 58 / 76, 2^19 60 to 96 / 90 to 97, 2^20 114,
+# 186, 329 / 119, 142, 192 (32, 4, 1 particles a cell), 2^21 371, 787 / 181, 304; cell order 56 to 80 / 75 to 83
+# throughout.  Second order, 2^18: random 170 to 195 / 92 to 97, cell order 89 / 82, but with 40 work items (16^3 cells)
+# 98 / 118: a tile's 8192 records are an item and an item a block, and fewer than 64 leave most CUs idle.
+_TILE_SLOTS_1, _TILE_SLOTS_2, _TILE_ITEMS = 1 << 20, 1 << 18, 64
+
+
+def _through_tiles(desc, slots):
+    tiles = 1
+    for a in range(3):
+        tiles *= -(-desc.n[a] // 8)
+    least = _TILE_SLOTS_1 if desc.shape_factor == 1 else _TILE_SLOTS_2
+    return slots >= least and tiles + slots // 8192 >= _TILE_ITEMS
+
+
 def push_into(desc, sp, xp, up, act, E3, B3, Ee, Be, u_planes, stream):
     """Pushed velocities into u_planes; E3, B3 are 3-D components, Ee, Be the
     external fields' pointers or None."""
     f64 = is_f64(xp[0])
     pp = pic_particles(xp, up, act)
-    ws = None if f64 else binned_workspace(desc, sp, PUSH, xp[0].device)
+    ws = None
+    if not f64 and _through_tiles(desc, xp[0].numel()):
+        ws = binned_workspace(desc, sp, PUSH, xp[0].device)
     if ws is not None:
         N.call("pic_push_binned", desc, sp, pp, N.p3(E3), N.p3(B3), Ee, Be, N.p3(u_planes), N.ptr(ws), ws.numel(),
                stream)
