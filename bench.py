@@ -429,7 +429,6 @@ def main():
         sys.exit(2)
 
     import torch
-    from pypic3d_amd import _native as N
     from pypic3d_amd import workloads
     from pypic3d_amd.runner import ElectrodynamicRunner
 
@@ -476,8 +475,7 @@ def main():
     print(f"[bench] timed {args.steps} steps in {elapsed:.3f} s; phases {phases}", file=sys.stderr, flush=True)
 
     if runner.tile:
-        exact = bool(N.lib().pic_tile_exact_grid(runner.desc)) and runner.desc.variant != 1
-        kernel_name = "fused_tile_exact_kernel" if exact else "fused_tiled_kernel"
+        kernel_name = "fused_tile_exact_kernel" if runner.desc.variant != 1 else "fused_tiled_kernel"
     else:
         kernel_name = "fused_push_esirkepov_v2"
     traffic, traffic_src = measured_traffic(kernel_name, args.n, args.ppc)

@@ -204,14 +204,16 @@ int pic_fused_push_esirkepov_nodes(const PicDesc* desc, const PicSpecies* sp, co
  * tile and adds the box into J once.  Same results as
  * pic_fused_push_esirkepov up to FP32 summation order.  E+E_ext and B+B_ext
  * around the tile are staged in LDS for the gather.  tile: 4 or 8 cells per
- * axis; rounds: 2 or 4 particle slots per thread per pass; min_blocks: 1, 3
- * or 4 resident blocks per CU requested from the register allocator.
- * On an exact grid (every node origin + a*spacing an FP32 number, e.g. integer
- * or dyadic spacings and origins) a thread takes `rounds` consecutive sorted
- * slots and sums equal-cell deposits in registers; particles its fast loop does
- * not cover are listed in workspace (1 + count*slots int32: workspace[0] is
- * the list length) and finished by a second kernel in the same call.
- * desc->variant = 1 selects the strided kernel on every grid (comparison).
+ * axis.  On an exact grid (every node origin + a*spacing an FP32 number, e.g.
+ * integer or dyadic spacings and origins) a thread takes one, two or four
+ * consecutive sorted slots, by the mean number of a tile, and sums equal-cell
+ * deposits in registers; particles its fast loop does not cover are listed in
+ * workspace (1 + count*slots int32: workspace[0] is the list length) and
+ * finished by a second kernel in the same call.  Other grids, and every grid
+ * with desc->variant = 1, take the strided kernel (comparison), shaped by rounds
+ * (2, 4 or 8: slots per thread per pass) and min_blocks (1, 3 or 4 resident
+ * blocks per CU requested from the register allocator).  A tiled launch of
+ * 2^32 threads or more (256 a tile: tile 4 on 1024^3 cells) is refused.
  * pic_tile_exact_grid returns 1 when desc is such an exact grid. */
 int pic_tile_exact_grid(const PicDesc* desc);
 int pic_fused_push_esirkepov_tiled(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in,
@@ -283,8 +285,9 @@ int pic_fused_push_direct_tiled_gather(const PicDesc* desc, const PicSpecies* sp
  * slot order through cell bins (pic_binned.hip): kind 0 rho, 1 J_from_rhov,
  * 2 Esirkepov (deposit or fused phase), 3 push.  The workspace query returns -1
  * where the grid is not covered (an axis of one cell, or more cells than the
- * bins hold), from 2^31 - 2048 slots on and, for the push, for small sets.  pic_push_binned samples the
- * slot order on the device and pushes sorted sets in slot order. */
+ * bins hold: some 8 million, second order 4 million; rho goes beyond 256^3), from
+ * 2^31 - 2048 slots on and, for the push, for small sets.  pic_push_binned samples the slot order on the
+ * device and pushes sorted sets in slot order. */
 int64_t pic_binned_workspace_bytes(const PicDesc* desc, const PicSpecies* sp, int32_t kind);
 int pic_deposit_rho_binned(const PicDesc* desc, const PicSpecies* sp, const PicParticles* in, float* rho,
                            void* workspace, int64_t workspace_bytes, void* stream);
@@ -466,13 +469,12 @@ typedef struct PicBatchSim {
 int pic_batch_check(const PicBatchSim* sims, int32_t n_sims, int64_t particle_slots, int64_t field_elems);
 /* Fused particle phase of every member: `sims` and `work` are device arrays;
  * work holds n_work (member, block) pairs covering each member's slots in
- * blocks of 256 * rounds (rounds 2, 4 or 8); `grid` persistent blocks walk
- * the list.  J (batch arrays) must be zero on entry.  out must not alias in. */
+ * blocks of 256 * rounds (rounds 2, 4 or 8).  First-order 1-D and 2-D members
+ * take a block per pair, `grid` persistent blocks the others.  J (batch arrays) must be zero on entry.  out must not alias in. */
 int pic_batch_fused_push_esirkepov(const PicBatchSim* sims, const int32_t* work, int32_t n_work, int32_t rounds,
                                    int32_t grid, const PicParticles* in, const float* const E[3],
                                    const float* const B[3], PicParticles* out, float* const J[3], void* stream);
-/* Grid phase of every member, one block per member: J fold + refresh
- * (particle codes), B_half = B - dt/2 curl E_in, E_out = E_in + dt (C^2 curl
+/* Grid phase of every member, four launches: J fold + refresh (particle codes), B_half = B - dt/2 curl E_in, E_out = E_in + dt (C^2 curl
  * B_half - J/eps), B = B_half - dt/2 curl E_out, each refreshed. */
 int pic_batch_field_step(const PicBatchSim* sims, int32_t n_sims, const float* const E_in[3], float* const B[3],
                          float* const B_half[3], float* const J[3], float* const E_out[3], void* stream);

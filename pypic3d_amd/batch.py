@@ -1,20 +1,21 @@
 """Batched ensembles of independent simulations (uneven grids and particle counts).
 
 ``EnsembleRunner`` advances every member with the semantics of
-``time_loop_electrodynamic``'s Esirkepov branch (evolve.py:16-103), using one
-persistent launch per phase for the whole ensemble:
+``time_loop_electrodynamic``'s Esirkepov branch (evolve.py:16-103), seven
+launches a step for the whole ensemble:
 
 1. ``pic_fill_f32`` zeroes the batch J arrays;
-2. ``pic_batch_fused_push_esirkepov`` walks a work list of (member, block)
-   items with a fixed grid of persistent blocks (gather + push + Esirkepov +
-   position update + boundaries, the single-simulation block function);
-3. ``pic_batch_field_step`` runs one block per member for the J fold/refresh
-   and the three Yee passes.
+2. ``pic_batch_fused_push_esirkepov`` (gather + push + Esirkepov + position
+   update + boundaries, the single-simulation block functions) over a work list
+   of (member, block) items: a block per item for first-order 1-D and 2-D
+   members, then a fixed grid of persistent blocks for the others;
+3. ``pic_batch_field_step`` folds J and makes the three Yee passes, a launch
+   each over all members' points.
 
-``capture`` records one step into a HIP graph (torch.cuda.CUDAGraph) that
-``replay`` launches; the ops allocate nothing and use no memset, so the graph
-replays the same three kernels.  ``autotune`` picks the particles per block
-(256 x rounds) and the persistent grid size from timed steps.
+``capture`` records two steps into a HIP graph (torch.cuda.CUDAGraph) that
+``replay`` launches; the ops allocate nothing and use no memset.  ``autotune``
+picks the particles per item (256 x rounds) and the persistent grid size from
+timed steps.
 
 Members must have periodic field and particle boundaries, alpha = 1 and no
 external fields (the two-stream ensembles this targets).

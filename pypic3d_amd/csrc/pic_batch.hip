@@ -1,5 +1,6 @@
 // Batched ensembles: many independent simulations of uneven grid size and
-// particle count advance together, one persistent launch per phase.
+// particle count advance together, two launches for the particles and four for
+// the fields.
 //
 // Storage: every simulation's particle planes are a slice of one set of batch
 // planes (PicBatchSim::particle_offset) and every field component a slice of
@@ -7,9 +8,9 @@
 // layout.  The descriptor table lives in device memory.
 //
 // Particle phase: a work list of (simulation, block) items covers every
-// simulation's slots in blocks of kThreads * rounds; a fixed grid of
-// persistent blocks walks the list, and each item runs the same block
-// function as the single-simulation kernel (fast paths chosen per item).
+// simulation's slots in blocks of kThreads * rounds.  Items of first-order 1-D and
+// 2-D members take a block each (planar_chunk, as the single simulation does); a
+// fixed grid of persistent blocks walks the list for the others (fused_block_boxed).
 //
 // Field phase: the grid part of time_loop_electrodynamic's Esirkepov branch
 // (evolve.py:70-97) as four launches over all members: J fold, B half step with

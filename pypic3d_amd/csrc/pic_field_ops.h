@@ -1,8 +1,8 @@
-// Per-element field operations shared by the one-launch-per-op kernels
-// (pic_fields.hip) and the batched one-block-per-simulation field step
-// (pic_batch.hip).  Each function handles one element id `t` of its index
-// space; callers map threads to ids.  The scalar type T is float for the
-// FP32 path and double for the FP64 path.
+// Per-element field operations shared by the single-simulation kernels
+// (pic_fields.hip) and the ensembles' field passes (pic_batch.hip).  Each
+// function handles one element id `t` or one point (i, j, k); callers map
+// threads to them.  The scalar type T is float for the FP32 path and double for
+// the FP64 path.
 #pragma once
 #include "pic_common.h"
 

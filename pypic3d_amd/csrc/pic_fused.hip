@@ -270,8 +270,8 @@ __device__ inline bool tile_slots(const int32_t* __restrict__ starts, const Tile
 // full is put on the rare list (rare[0] = count, slots from rare[1]) and run
 // whole by fused_tile_rare_kernel, which overwrites what is stored here.
 //
-// Bound by VALU instructions (about 600 per 64 particles; the LDS and memory
-// traffic overlap them).  Summing cell moments in registers, FP64 box adds in
+// Bound by VALU instructions (577 per 64 particles, 81 % of the fastest launch at
+// 256^3 with 32; the LDS and memory traffic overlap them).  Summing cell moments in registers, FP64 box adds in
 // place of ds_add_f32 and a queue of (slot, velocity) took 128^3 with 2 x 16
 // particles per cell from 1963 to 1548 us (43 G particles/s, 2.2 TB/s) and
 // 256^3 with 32 from 12.1 to 9.7 ms; FP64 anchors in the same kernel take

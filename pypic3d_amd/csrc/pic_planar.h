@@ -14,9 +14,12 @@
 // queued and deposited in the 3-slot frame by lanes that all do so.
 //
 // Bound by the latency of a chunk's stages, so blocks are kept at sixteen waves
-// a CU.  64 members of up to 256 x 32 cells, 8.7M slots in order: 270 to 330 us,
+// a CU.  64 members of up to 256 x 32 cells, 8.7M slots in order: 329 to 343 us,
 // 852 us where each 256 slots were scanned by lane shuffles into an FP32 box; 262k
-// slots on 64 x 64: 22 us, 52 us before.  As slots lose their order ranges widen:
+// slots on 64 x 64: 25 us, 52 us before.  (A node's value is a difference of FP32
+// moments, so one of small weight carries the rounding of the cell's current; J
+// is as far from its FP64 value as sums of single node values, 4.2e-7 against
+// 4.9e-7 in the norm for two beams on 64 x 64.)  As slots lose their order ranges widen:
 // 80 KB of boxes (2 x 512 threads a CU) hold them longer than 40 KB (4 x 256, 10 %
 // faster in order, 25 % slower after 400 steps).
 #pragma once

@@ -3,8 +3,8 @@
 ``ElectrodynamicRunner`` performs exactly the call sequence of
 ``evolve.time_loop_electrodynamic`` (Esirkepov or direct branch) on
 preallocated ping-pong buffers: particle SoA planes alternate between two
-sets, E alternates between two buffers and B returns to its own buffer after
-the two half steps.  Optional cell re-sorting every ``sort_every`` steps keeps
+sets, E alternates between two buffers, J keeps its own and B returns to its
+own after the two half steps.  Optional cell re-sorting every ``sort_every`` steps keeps
 particles cache-local; with the tile-ordered fused kernels (exact grids) the
 re-bin stops at its permutation and the next step's fused kernel reads
 the particles through it (the permutation is applied on its own only when
@@ -36,8 +36,9 @@ class ElectrodynamicRunner:
         """tile (4 or 8): keep particles in tile-major cell order (sorted once
         here, then every ``sort_every`` steps) and use the tile-ordered kernels:
         the fused push + Esirkepov kernel (3-D first order); in the
-        J_from_rhov branch the fused push + direct-deposit kernel on exact 3-D
-        first-order grids, else the tiled direct deposit."""
+        J_from_rhov branch the fused push + direct-deposit kernel on 3-D
+        first-order grids, else the tiled direct deposit.  rounds and min_blocks
+        shape the strided comparison kernel (desc.variant 1) alone."""
         E, B, J, rho, phi, external_fields, pml_state, overflow = fields
         _check_pml(pml_state)
         if static_parameters.particle_pusher not in ("boris", "higuera_cary"):
@@ -91,8 +92,7 @@ class ElectrodynamicRunner:
         self.keys = None
         self.sorts_done = 0
         self.tile, self.rounds, self.min_blocks, self.starts = None, int(rounds), int(min_blocks), None
-        # launch shape of the fused direct kernel: 4 resident blocks per CU
-        # (two slots per thread) at tile 4, one at tile 8
+        # argument of the fused direct launch, which has one shape
         self.direct_min_blocks = 1
         self.sort_lookahead = None      # tile re-sort keys at x + t u; None: t = sort_every * dt / 2
         self.tile_ws, self.direct_fused, self._deposit_ws = None, False, None

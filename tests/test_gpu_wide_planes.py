@@ -1,6 +1,6 @@
-"""Guard refresh and conducting walls of a 2-D grid whose plane has more than
-2^28 rows of one cell: a launch of 64 threads a row in one grid axis would pass
-2^32 threads."""
+"""Guard refresh and conducting walls of 2-D grids whose planes have more than
+2^28 rows of one cell (a launch of 64 threads a row in one grid axis would pass
+2^32 threads), and with more than 2^31 guard cells (numbered in 64 bits)."""
 
 import pytest
 import torch
@@ -19,14 +19,16 @@ def _field(desc, seed):
     return torch.rand(tuple(desc.dims), generator=gen, device="cuda") + 1.0
 
 
-def test_refresh_of_a_wide_plane():
-    static, dyn = workloads.make_parameters((SIDE, SIDE, 1), dt=0.05, g=1)
+@pytest.mark.parametrize("side,g", [(SIDE, 1), (23200, 2)])
+def test_refresh_of_a_wide_plane(side, g):
+    static, dyn = workloads.make_parameters((side, side, 1), dt=0.05, g=g)
     desc = make_desc(static, dyn)
     f = _field(desc, 1)
-    inner = f[1:-1, 1:-1, 1].clone()
+    inner = f[g:-g, g:-g, g].clone()
     N.call("pic_halo_refresh", desc, N.ptr(f), 0, N.stream_handle())
-    want = torch.nn.functional.pad(inner[None, None], (1, 1, 1, 1), mode="circular")[0, 0]
-    for k in range(3):
+    rows = torch.cat([inner[-g:], inner, inner[:g]])
+    want = torch.cat([rows[:, -g:], rows, rows[:, :g]], dim=1)
+    for k in range(2 * g + 1):
         assert torch.equal(f[:, :, k], want)
 
 
