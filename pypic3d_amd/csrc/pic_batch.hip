@@ -86,7 +86,7 @@ __device__ inline bool any_item(const PicBatchSim* __restrict__ sims, const int3
 // The items of first-order 1-D and 2-D members, a block each: the chunks of planar_kernel.
 template <int kRounds>
 __global__ __launch_bounds__(kPlanarBlock, 2) void batch_planar_kernel(const PicBatchSim* __restrict__ sims,
-                                                                   const int32_t* __restrict__ work, int32_t n_work,
+                                                                   const int32_t* __restrict__ work,
                                                                    BatchParticleArgs args) {
     constexpr int kP = kRounds == 2 ? 1 : 2, kChunk = kPlanarBlock * kP;
     __shared__ PlanarShared<kP, kPlanarBlock> sh;
@@ -265,16 +265,20 @@ int pic_batch_fused_push_esirkepov(const PicBatchSim* sims, const int32_t* work,
     }
     hipStream_t st = as_stream(stream);
     const int g = grid < n_work ? grid : n_work;
-    if (rounds == 2) {
-        hipLaunchKernelGGL(batch_planar_kernel<2>, dim3(n_work), dim3(kPlanarBlock), 0, st, sims, work, n_work, args);
-        hipLaunchKernelGGL(batch_fused_kernel<2>, dim3(g), dim3(kThreads), 0, st, sims, work, n_work, args);
-    } else if (rounds == 4) {
-        hipLaunchKernelGGL(batch_planar_kernel<4>, dim3(n_work), dim3(kPlanarBlock), 0, st, sims, work, n_work, args);
-        hipLaunchKernelGGL(batch_fused_kernel<4>, dim3(g), dim3(kThreads), 0, st, sims, work, n_work, args);
-    } else {
-        hipLaunchKernelGGL(batch_planar_kernel<8>, dim3(n_work), dim3(kPlanarBlock), 0, st, sims, work, n_work, args);
-        hipLaunchKernelGGL(batch_fused_kernel<8>, dim3(g), dim3(kThreads), 0, st, sims, work, n_work, args);
-    }
+    // items of a launch with a block each: a launch of 2^32 threads would run the remainder only, without an error
+    constexpr int32_t kItems = 1 << 22;
+    static_assert((int64_t)kItems * kPlanarBlock < ((int64_t)1 << 32), "threads of a launch");
+#define PIC_BATCH_FUSED(R)                                                                                       \
+    do {                                                                                                         \
+        for (int32_t at = 0; at < n_work; at += std::min(kItems, n_work - at))                                   \
+            hipLaunchKernelGGL(batch_planar_kernel<R>, dim3((unsigned)std::min(kItems, n_work - at)),            \
+                               dim3(kPlanarBlock), 0, st, sims, work + 2 * (int64_t)at, args);                   \
+        hipLaunchKernelGGL(batch_fused_kernel<R>, dim3(g), dim3(kThreads), 0, st, sims, work, n_work, args);     \
+    } while (0)
+    if (rounds == 2) PIC_BATCH_FUSED(2);
+    else if (rounds == 4) PIC_BATCH_FUSED(4);
+    else PIC_BATCH_FUSED(8);
+#undef PIC_BATCH_FUSED
     PIC_CHECK_LAUNCH();
     return 0;
 }

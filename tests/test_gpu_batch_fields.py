@@ -56,3 +56,43 @@ def test_field_step_matches_the_single_simulation_kernels(members, g):
             for c in range(3):
                 a = got[c, at[m]:at[m] + n].view(shape)
                 assert float((a - want[c]).abs().max()) <= 4e-6 * float(want[c].abs().max())
+
+
+def test_more_work_items_than_one_launch_holds():
+    """A block per item would pass 2^32 threads at 2^23 items.  Member 1's only
+    item stands last, behind that many of member 0's (which repeat its step)."""
+    members, slots = 2, 300
+    static, dyn = workloads.make_parameters((8, 1, 1), dt=0.05)
+    d = make_desc(static, dyn)
+    table = (PicBatchSim * members)()
+    cells = d.dims[0] * d.dims[1] * d.dims[2]
+    for m in range(members):
+        ctypes.memmove(ctypes.addressof(table[m].desc), ctypes.addressof(d), ctypes.sizeof(N.PicDesc))
+        sp = table[m].species
+        sp.count, sp.slots = 1, slots
+        sp.charge[0], sp.mass[0], sp.weight[0] = -1.0, 1.0, 0.01
+        for a in range(3):
+            sp.update_x[0][a] = sp.update_u[0][a] = 1
+        table[m].particle_offset, table[m].field_offset = m * slots, m * cells
+    N.check(N.lib().pic_batch_check(ctypes.addressof(table), members, 2 * slots, 2 * cells), "pic_batch_check")
+    tab = torch.frombuffer(bytearray(bytes(table)), dtype=torch.uint8).cuda()
+    work = torch.zeros(((1 << 23) + 2, 2), dtype=torch.int32, device="cuda")
+    work[-1, 0] = 1
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = (torch.rand((3, 2 * slots), generator=gen, device="cuda") - 0.5) * 0.5
+    u = (torch.rand((3, 2 * slots), generator=gen, device="cuda") - 0.5) * 0.2
+    act = torch.ones(2 * slots, dtype=torch.uint8, device="cuda")
+    E, B, J = (torch.zeros((3, 2 * cells), device="cuda") for _ in range(3))
+    xo, uo, ao = torch.full_like(x, 9.0), torch.full_like(u, 9.0), torch.zeros_like(act)
+
+    def planes(xs, us, a):
+        p = N.PicParticles()
+        for c in range(3):
+            p.x[c], p.u[c] = xs[c].data_ptr(), us[c].data_ptr()
+        p.active = a.data_ptr()
+        return p
+
+    N.call("pic_batch_fused_push_esirkepov", tab.data_ptr(), work.data_ptr(), work.shape[0], 2, 64, planes(x, u, act),
+           N.p3(E), N.p3(B), planes(xo, uo, ao), N.p3(J), N.stream_handle())
+    assert bool((ao == 1).all())
+    assert float((uo - u).abs().max()) <= 1e-6 and float((xo - x - 0.05 * u).abs().max()) <= 1e-6
